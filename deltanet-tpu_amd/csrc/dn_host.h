@@ -28,22 +28,18 @@ struct PF {
   // workspace arrays (one unit = one (batch, exec head, chunk))
   int32_t* flags;            // [B][NCb][2] : is_new_doc, all_same_doc
   float* dvec;               // [unit][K]    : e^{Lambda_end}
-  int nct;                   // 16-column tiles of the value width (Vp / 16)
+  float* rows;               // [unit][3][64]: b e^Lambda, e^Lambda, e^{Lend - Lambda} per token (scalar gates)
   // Workspace, per unit = (batch, exec head, chunk).  Every operand array is
-  // fragment-native for its consumer (F = [tile][slab][lane][8] elements of a
-  // 16 x 32 MFMA operand slab, C = [row tile][col tile][lane][4] accumulator
-  // tiles).  Split operands have a high and a low array (bf16 mode; in fp32
-  // mode the low pointer aliases the high one).  "ST" = bf16 in bf16 mode,
-  // fp32 in fp32 mode.
-  void* PnA;                 // F  [8][4]      ST : Pn = -ke^T W, rows = state row (chain A)
-  float* QC;                 // C  [8][nct]    f32: Q = ke^T U (chain accumulator init)
-  void *XAh, *XAl;           // F  [8][4]      ST : X = qe - M W, rows = token (chain output B)
-  float* OiT;                // C  [8][nct]    f32: (M U)^T tiles (chain output accumulator init)
-  void* BeB;                 // F  [8][4]      ST : (b k e^Lambda)^T, first document
-  void *KeBh, *KeBl;         // F  [8][4]      ST : (k e^{Lend - Lambda})^T, last document
-  void *MAh, *MAl;           // F  [8][4]      ST : M, rows = token
-  float* QeA;                // F  [8][4]      f32: q e^Lambda, first document
-  void* sink;                // 1 KB the chain's output lanes past the last token store into
+  // fragment-native for its consumer ([tile][slab][lane][8] elements of a
+  // 16 x 32 MFMA operand slab).  Split operands have a high and a low array
+  // (bf16 mode; in fp32 mode the low pointer aliases the high one).  "ST" =
+  // bf16 in bf16 mode, fp32 in fp32 mode.  With scalar gates BeA, QeAh and
+  // KeTh hold the normalised k, q and k^T, one unit per key head.
+  void* BeA;                 // [4][4] ST : b k e^Lambda, rows = token, first document
+  void *QeAh, *QeAl;         // [4][4] ST : q e^Lambda, rows = token, first document
+  void *KeTh, *KeTl;         // [8][2] ST : (k e^{Lend - Lambda})^T, rows = key channel, last document
+  void *TAh, *TAl;           // [6] ST : T, rows = token (the six slabs that are not all zero)
+  void *MAh, *MAl;           // [6] ST : M, rows = token, slabs as T
 };
 
 // Records the message for dn_last_error() and returns `code`.

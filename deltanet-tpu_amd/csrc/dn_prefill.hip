@@ -8,24 +8,26 @@
 //   wrapper   gdn2.py:1970-2125 (clamps, scale, L2-norm, gate broadcast,
 //                                segment canonicalisation, padding)
 //
-// The MI355X design splits the work into two launches per token block so
-// that only a 128x128-by-128x16 product sits on the sequential critical path.
-// With Vnew = U - W S the reference's per-chunk update and output become
-//     S_next = [same doc] diag(e^Lend) S + Pn S + Q,  Pn = -ke^T W,  Q = ke^T U
-//     O      = X S + Oi,                              X = qe - M W,  Oi = M U
-// so:
-//   k_prepass (grid: one workgroup of 8 waves per (batch, exec head, chunk)
-//       unit) fused prologue, Lambda, A and M on MFMA, T by blocked
-//       substitution on fp32 MFMA, W, the chunk operators Pn and X, and
-//       then, from the T, ke^T and M it still holds in LDS, U = T (w*v),
-//       Q = ke^T U and Oi = M U (value_cols).
-//   k_chain   (grid: 16-column tile x exec-head x batch, 8 waves)
-//       the sequential scan over chunks with the fp32 state in VGPRs, and
-//       each chunk's output O = X S_c + Oi from the same S_c fragments.
+// The MI355X design runs 64-token chunks in two launches per token block.  Per
+// chunk, with be = b k e^Lambda, qe = q e^Lambda, ke = k e^{Lend - Lambda}
+// (tokens of the chunk's first / first / last document) and T = (I + A)^-1:
+//     Vn = T (w v - be S),   O = qe S + M Vn,
+//     S <- [same doc] diag(e^Lend) S + ke^T Vn
+//   k_prepass (one workgroup of 4 waves per (batch, exec head, chunk) unit)
+//       everything that depends neither on the values nor on the state:
+//       prologue, Lambda, be, qe, ke^T, A and M on MFMA, T by blocked
+//       substitution on fp32 MFMA.
+//   k_chain   (grid: 16-column tiles x exec head x batch, 8 waves)
+//       the sequential scan over chunks with the fp32 state in VGPRs, three
+//       dependent products per chunk, and each chunk's output beside it.
+// T is applied inside the scan: folding it into per-chunk operators of the
+// state (W = T be, U = T (w v), an affine map of S) made every unit read v and
+// w, run five more products and write operators as wide as the values; the
+// scan now reads v and w itself and the operators do not grow with the number
+// of value heads.
 //
 // Intermediates live in a caller-provided workspace sized for one token
-// block, small enough to stay resident in the 256 MB Infinity Cache; every
-// array is stored in the MFMA lane order of its consumer.
+// block; every array is stored in the MFMA lane order of its consumer.
 #include <mutex>
 
 #include "dn_common.h"
@@ -33,11 +35,12 @@
 
 namespace dn {
 
-constexpr int CH = 128;   // chunk size (gdn2.py:1869)
+constexpr int CH = 64;    // chunk size (the reference's 128 is a TPU tile size; the recurrence is the same)
+constexpr int NB = CH / 16;   // 16-token blocks of a chunk
 constexpr int KD = 128;   // key / value head dim (gdn2.py:1897)
-constexpr int XP = 132;
+constexpr int XP = 132;   // fp32 LDS pitch (floats) of the Lambda rows: conflict-free 16-lane column groups
+constexpr int AP = 68;    // fp32 LDS pitch of A and T
 constexpr int kMaxBlockChunks = 1024;   // chunks per token block (chain's LDS flag table)
-   // fp32 LDS pitch (floats): conflict-free 16-lane column groups
 
 // diag blocks whose in-block log2-decay span exceeds this use the
 // overflow-free hierarchical path (e^{69} stays far inside the fp32 range)
@@ -77,110 +80,6 @@ __device__ __forceinline__ SegId seg_raw(const PF& p, int b, int t) {
   const bool w64 = p.seg_dt == DT_I64;
   const int32_t* s32 = (const int32_t*)p.seg + (w64 ? 2 * i : i);
   return SegId{s32[0], s32[w64 ? 1 : 0]};
-}
-
-// v rows of one 32-column slab of execution head h, chunk c (row 16a + r16 of
-// block a, fragment order, as loaded) and the write gate of those rows when it
-// has one channel.  Issued apart from their use so a caller can put them in
-// flight ahead of other work: vmcnt counts loads and stores in issue order, so
-// the wait for these rows covers only what was issued before them.
-template <class TV> struct VRows {
-  Raw8<TV> v[8];
-  float ws[8];
-};
-
-template <class TV>
-__device__ __forceinline__ void v_rows_issue(const PF& p, int b, int h, int c, int col0, int l, VRows<TV>& r) {
-  const int r16 = l & 15, q = l >> 4;
-  const int tb = p.t0 + c * CH;
-  const int t_end = min(p.t0 + p.nt, p.L);
-  const int hv = p.gates_at_hv ? h : h * p.G + col0 / KD;
-  const int hw = vgate_head(p, p.w_h, hv);
-  const int cs = (col0 & ~31) % KD;
-  auto row_bt = [&](int a) { return (int64_t)b * p.L + min(tb + 16 * a + r16, t_end - 1); };
-  // (the w layout test sits outside the row loops: a branch between the
-  // loads would make each row wait for the one before)
-  if (p.w_c == 1) {
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const int64_t bt = row_bt(a);
-      r.v[a].load((const TV*)p.v + (bt * p.Hv + hv) * KD + cs, q);
-      r.ws[a] = ((const float*)p.w)[bt * p.w_h + hw];
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      r.v[a].load((const TV*)p.v + (row_bt(a) * p.Hv + hv) * KD + cs, q);
-      r.ws[a] = 0.f;
-    }
-  }
-}
-
-// (w*v)^T fragments of 16 NT value columns of execution head h, chunk c, from
-// column col0 (rows = value column, k = token): Bwv[nt][s] covers columns
-// col0 + 16nt .. + 15 and token slab s, from the rows r (v_rows_issue of the
-// same columns).  Each 16-token block is transposed by an identity product
-// into half of a slab (exact).
-template <bool BF, class TV, int NT>
-__device__ __forceinline__ void wv_frags(const PF& p, int b, int h, int c, int col0, int l, const VRows<TV>& r,
-                                         typename Pol<BF>::F3 (&Bwv)[NT][4]) {
-  using P = Pol<BF>;
-  using F1 = typename P::F1;
-  using F3 = typename P::F3;
-  const int r16 = l & 15, q = l >> 4;
-  const int tb = p.t0 + c * CH;
-  const int t_end = min(p.t0 + p.nt, p.L);
-  const int hv = p.gates_at_hv ? h : h * p.G + col0 / KD;
-  const int hw = vgate_head(p, p.w_h, hv);
-  const int h0 = NT == 2 ? 0 : (col0 >> 4) & 1;   // first 16-column half of the slab
-  const int cs = (col0 & ~31) % KD;
-  float ww[8][8];
-  if (p.w_c == 1) {
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ww[a][e] = r.ws[a];
-  } else {
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-      const int64_t bt = (int64_t)b * p.L + min(tb + 16 * a + r16, t_end - 1);
-      row8<float>((const float*)p.w + (bt * p.w_h + hw) * p.w_c + cs, q, ww[a]);
-    }
-  }
-  const F1 id0 = ident_frag<BF>(0, r16, q), id1 = ident_frag<BF>(1, r16, q);
-#pragma unroll
-  for (int a = 0; a < 8; ++a) {
-    const bool valid = tb + 16 * a + r16 < t_end;
-    float vv[8], x[8];
-    r.v[a].to(vv);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float wg = p.fuse ? sigmoid_fast(ww[a][e]) : ww[a][e];
-      x[e] = valid ? wg * vv[e] : 0.f;
-    }
-    const F3 fx = P::f3(x);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const bool second = nt + h0 == 1;
-      f32x4 chi = zero4();
-      mma(chi, P::hi(fx), second ? id1 : id0);
-      // lane (c, q): column 16nt + c, tokens 16a + 4q + ii -> slab a/2, half a&1
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        if constexpr (BF) {
-          Bwv[nt][a >> 1].hi.v[4 * (a & 1) + ii] = (bf16)chi[ii];
-        } else {
-          Bwv[nt][a >> 1].v[4 * (a & 1) + ii] = chi[ii];
-        }
-      }
-      if constexpr (BF) {
-        f32x4 clo = zero4();
-        mma(clo, fx.lo, second ? id1 : id0);
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) Bwv[nt][a >> 1].lo.v[4 * (a & 1) + ii] = (bf16)clo[ii];
-      }
-    }
-  }
 }
 
 // q, k and b * k of one token row in fragment order (slab s: elements
@@ -236,182 +135,169 @@ __device__ __forceinline__ void row_inputs(const PF& p, const Raw8<TIn> (&rq)[4]
   }
 }
 
-// ===========================================================================
-// Phases 1-3 of k_prepass for one decay and one b per (token, head) (the
-// Gated DeltaNet form, chunk_gdn: gdn.py:66-110 broadcasts them over the key
-// channels), precision "bf16" with bf16 q and k.  The per-channel machinery of
-// the general phases collapses:
-//   * Lambda is one cumulative sum per token (double-float, log2 units);
-//   * with the normalised q and k exactly bf16 (they are rounded back to the
-//     input type), the Gram matrices k k^T and q k^T are single bf16 MFMAs
-//     with fp32 accumulation, and
-//       A[i][j] = b_i e^{Lambda_i - Lambda_j} (k k^T)[i][j]   (i > j),
-//       M[i][j] =     e^{Lambda_i - Lambda_j} (q k^T)[i][j]   (i >= j),
-//     one exponential per pair, whose exponent is <= 0 for every unmasked
-//     pair (no factorisation, no overflow path);
-//   * (b k e^Lambda)^T, ke^T, qe and e^{Lambda_end} are per-row scalars times
-//     the row.
-// Results land where the general phases put them: A (fp32, row-major) in X,
-// M (split, fragment-native) and the transposed row operands in the
-// workspace; Y holds the q and k fragments until phase 4 takes it over.
-// Barriers inside wait for LDS only, so the per-row stores drain behind the
-// Gram products; the last one (a full __syncthreads) drains them before any
-// wave reads another's rows back.
-// ===========================================================================
-template <class TIn>
-__device__ __forceinline__ void prepass_scalar_gates(const PF& p, int b, int tb, int t_end, float g_tok,
-                                                     const Raw8<TIn> (&rq)[4], const Raw8<TIn> (&rk)[4],
-                                                     const Raw8<float> (&rb)[4], float b_scalar, const int* doc,
-                                                     float* X, float* Y, bf16* g_Mh, bf16* g_Ml, bf16* g_be,
-                                                     bf16* g_keh, bf16* g_kel, float* g_qe, float* g_dv) {
-  using P = Pol<true>;
-  using F1 = P::F1;
-  using F3 = P::F3;
-  using SS = Store<true>;
-  __shared__ float lam_h[CH], lam_l[CH];   // Lambda (log2 units), double-float
-  __shared__ float bet_s[CH];              // b per token (0 past the end)
-  const int tid = threadIdx.x;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, r16 = l & 15, q = l >> 4;
+// a 16 x 32 slab of an operand with two slabs per tile (reduction over the
+// chunk's 64 tokens)
+__device__ __forceinline__ int fofs2(int tile, int slab, int lane) { return ((tile * 2 + slab) * 64 + lane) * 8; }
 
-  // ---- Lambda: inclusive scan of g over the chunk (waves 0 and 1) ----------
-  float hi = 0.f, lo = 0.f;
-  if (tid < CH) {
-    float gv = fminf(g_tok, 0.f);   // _nonpositive (NaN -> 0)
-    gv = fminf(gv, p.guard ? -1e-6f : 0.f);
-    hi = (tb + tid < t_end) ? gv : 0.f;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float h2 = __shfl_up(hi, off), l2 = __shfl_up(lo, off);
-      if (l >= off) {
-        // error-free hi + h2 (TwoSum), the rounding error joins the low words
-        const float sum = hi + h2;
-        const float bb = sum - hi;
-        lo += l2 + ((hi - (sum - bb)) + (h2 - bb));
-        hi = sum;
+// T and M (64 x 64, lower triangular): the six slabs that are not all zero
+__device__ __forceinline__ int tofs(int tile, int slab, int lane) { return ((tile + tile / 3 + slab) * 64 + lane) * 8; }
+constexpr int TM = 6 * 64 * 8;   // elements of T or M
+
+// One unit of a prepass launch: (batch, execution head, chunk) with the
+// XCD-aware remap (the hardware deals linear block ids to the 8 XCDs
+// round-robin; consecutive chunks of a head share one XCD's L2).
+struct Unit {
+  int b, h, c, hk;
+  int tb, t_end;   // first token, end of the valid tokens
+  int64_t u;
+};
+__device__ __forceinline__ Unit unit_of(const PF& p) {
+  Unit x;
+  const int units = p.B * p.Hx * p.NCb;
+  int id = blockIdx.x;
+  if ((units & 7) == 0) id = (id & 7) * (units >> 3) + (id >> 3);
+  x.c = id % p.NCb;
+  id /= p.NCb;
+  x.h = id % p.Hx;
+  x.b = id / p.Hx;
+  x.hk = p.gates_at_hv ? x.h / p.G : x.h;
+  x.tb = p.t0 + x.c * CH;
+  x.t_end = min(p.t0 + p.nt, p.L);
+  x.u = ((int64_t)x.b * p.Hx + x.h) * p.NCb + x.c;
+  return x;
+}
+
+// Segment ids of a chunk: wave 0 loads token l's id and its predecessor's,
+// and the ids at the chunk's edge and at token 0 (every lane loads, so nothing
+// is consumed inside a divergent branch before it is needed).
+struct ChunkSeg {
+  SegId t{0, 0}, tp{0, 0}, s0{0, 0}, a{0, 0}, b{0, 0};
+  int32_t iseg = 0;
+  __device__ __forceinline__ void load(const PF& p, const Unit& x, int l) {
+    if (p.seg != nullptr) {
+      t = seg_raw(p, x.b, min(x.tb + l, x.t_end - 1));
+      tp = seg_raw(p, x.b, max(min(x.tb + l - 1, x.t_end - 1), 0));
+      s0 = seg_raw(p, x.b, 0);
+      a = seg_raw(p, x.b, x.tb);
+      b = seg_raw(p, x.b, max(x.tb - 1, 0));
+    }
+    if (p.init_seg != nullptr) iseg = p.init_seg[x.b];
+  }
+  // The in-chunk document index (segment canonicalisation: doc[i] = number of
+  // segment starts among tokens 1..i, one wave ballot) into LDS, and the
+  // chunk's flags (gdn2.py:1291-1302) from the lane of its last token.
+  __device__ __forceinline__ void finish(const PF& p, const Unit& x, int l, int* doc) {
+    const uint64_t bal = __ballot(l > 0 && p.seg != nullptr && (t != tp));
+    const int d = __popcll(bal & ((2ull << l) - 1ull));   // lanes 0..l (l = 63: all)
+    doc[l] = d;
+    if (l != 63 || x.h != 0) return;
+    int is_new;
+    if (x.tb == 0) {
+      if (p.has_init) {
+        is_new = 0;
+        // initial_state_segment_id is int32; a wider first id differs from it
+        // when its high word is not the sign extension of its low word
+        if (p.init_seg != nullptr) is_new = (s0.lo != iseg) || (p.seg_dt == DT_I64 && s0.hi != (iseg < 0 ? -1 : 0));
+      } else {
+        is_new = 1;
       }
+    } else if (x.c == 0 && !p.has_init) {
+      is_new = 1;
+    } else {
+      is_new = p.seg ? (a != b) : 0;
     }
-    if (w == 0 && l == 63) { lam_h[63] = hi; lam_l[63] = lo; }
+    p.flags[((int64_t)x.b * p.NCb + x.c) * 2 + 0] = is_new;
+    p.flags[((int64_t)x.b * p.NCb + x.c) * 2 + 1] = (d == 0);
   }
-  lds_barrier();
-  if (tid < CH) {
-    if (w == 1) {
-      const float h2 = lam_h[63], l2 = lam_l[63];
-      const float sum = hi + h2;
-      const float bb = sum - hi;
-      lo += l2 + ((hi - (sum - bb)) + (h2 - bb));
-      hi = sum;
-    }
-  }
-  lds_barrier();
-  if (tid < CH) {
-    const float ph = hi * kLog2e;
-    lam_h[tid] = ph;
-    lam_l[tid] = fmaf(hi, kLog2e, -ph) + lo * kLog2e;
-  }
-  lds_barrier();
-  const float le_h = lam_h[CH - 1], le_l = lam_l[CH - 1];
-  if (tid < KD) g_dv[tid] = fast_exp2(le_h + le_l);   // e^{Lambda_end}
+};
 
-  // ---- per-row operands of token block a = w --------------------------------
-  bf16* Kf = reinterpret_cast<bf16*>(Y);   // k fragments [block][slab][lane][8]
-  bf16* Qf = Kf + CH * KD;                 // q fragments
+// T = (I + A)^-1 of one chunk (A strictly lower, fp32 in X with pitch AP, the
+// tiles right of even diagonal blocks zeroed), by blocked forward
+// substitution; Tt is 64 x AP floats of scratch that nobody reads any more.
+// Wave w inverts diagonal block w, then per block row a wave bt < a forms
+// T[a][bt] = -D_a sum_{cc = bt}^{a-1} A[a][cc] T[cc][bt].  Each 16x16x16
+// product runs as 4 steps of the 16x16x4 fp32 MFMA with lane (r, q) holding
+// reduction index 4q + kk at step kk, so a lane's A operand (row of A) and B
+// operand (row of T^T, kept in Tt) are one 16-byte LDS read each.  T goes to
+// the workspace as fragments (wave w: row tile w), split in bf16 mode.
+template <bool BF>
+__device__ __forceinline__ void invert_and_store(float* X, float* Tt, typename Store<BF>::ST* g_Th,
+                                                 typename Store<BF>::ST* g_Tl, int w, int l) {
+  using SS = Store<BF>;
+  const int r16 = l & 15, q = l >> 4;
   {
+    // every lane group q works on the same columns (LDS reads broadcast); the
+    // group w stores, so the four waves write four different diagonal blocks
     const int a = w;
-    const int i = 16 * a + r16;
-    const bool valid = tb + i < t_end;
-    float qv[32], kv[32], bet[32];
-    row_inputs<TIn>(p, rq, rk, rb, b_scalar, valid, qv, kv, bet);
-    // b alone: b * k / k is not recoverable where k = 0, so take it again
-    float bsc = p.b_c == 1 ? b_scalar : 0.f;
-    if (p.guard) bsc = fmaxf(bsc, 0.f);
-    if (q == 0) bet_s[i] = valid ? bsc : 0.f;
-    const bool first = doc[i] == 0;
-    const bool last = doc[i] == doc[CH - 1];
-    const float li_h = lam_h[i], li_l = lam_l[i];
-    const float eL = fast_exp2(li_h + li_l);                    // e^{Lambda_i} <= 1
-    const float eK = fast_exp2((le_h - li_h) + (le_l - li_l));  // e^{Lambda_end - Lambda_i} <= 1
+    float tc[16];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      float bt[8], kt[8], qe[8];
+    for (int m = 0; m < 16; ++m) tc[m] = (m == r16) ? 1.f : 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        bt[e] = first ? bet[8 * s + e] * eL : 0.f;
-        kt[e] = last ? kv[8 * s + e] * eK : 0.f;
-        qe[e] = first ? qv[8 * s + e] * eL : 0.f;
-      }
-      Store<false>::st8(g_qe + fofs(a, s, l), qe);
-      // (b k e^Lambda)^T and ke^T in fragment layout (row = key, k = token)
-      const F1 fbt = P::f1(bt);
-      const F3 fkt = P::f3(kt);
+    for (int ii = 1; ii < 16; ++ii) {
+      float acc = 0.f;
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        const F1 id = ident_frag<true>(hf, r16, q);
-        f32x4 cb = zero4(), chi = zero4(), clo = zero4();
-        mma(cb, fbt, id);
-        mma(chi, fkt.hi, id);
-        mma(clo, fkt.lo, id);
-        const int o = fofs(2 * s + hf, a >> 1, l) + 4 * (a & 1);
-        const float xb[4] = {cb[0], cb[1], cb[2], cb[3]};
-        const float xh[4] = {chi[0], chi[1], chi[2], chi[3]};
-        const float xl[4] = {clo[0], clo[1], clo[2], clo[3]};
-        SS::st4(g_be + o, xb);
-        SS::st4(g_keh + o, xh);
-        SS::st4(g_kel + o, xl);
-      }
-      // the normalised rows are bf16 values: their fragments are exact
-      SS::st8(Kf + fofs(a, s, l), kv + 8 * s);
-      SS::st8(Qf + fofs(a, s, l), qv + 8 * s);
+      for (int m = 0; m < ii; ++m) acc += X[(16 * a + ii) * AP + 16 * a + m] * tc[m];
+      if (ii > r16) tc[ii] = -acc;
+    }
+    if (q == 0) {
+#pragma unroll
+      for (int ii = 0; ii < 16; ++ii) X[(16 * a + ii) * AP + 16 * a + r16] = tc[ii];
+    } else if (q == 1) {
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        *reinterpret_cast<f32x4*>(&Tt[(16 * a + r16) * AP + 16 * a + 4 * i4]) =
+            f32x4{tc[4 * i4], tc[4 * i4 + 1], tc[4 * i4 + 2], tc[4 * i4 + 3]};
     }
   }
   lds_barrier();
-
-  // ---- A and M tiles (a, bb), bb <= a: 36 tiles dealt round-robin ------------
-  for (int t = w; t < 36; t += 8) {
-    int a = 0;
-    while ((a + 1) * (a + 2) / 2 <= t) ++a;
-    const int bb = t - a * (a + 1) / 2;
-    f32x4 gk = zero4(), gq = zero4();
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const F1 ka = SS::fa(Kf + fofs(a, s, l));
-      const F1 kb = SS::fa(Kf + fofs(bb, s, l));
-      const F1 qa = SS::fa(Qf + fofs(a, s, l));
-      mma(gk, ka, kb);   // (k k^T)[16a + 4q + ii][16bb + r16]
-      mma(gq, kb, qa);   // (q k^T)[16a + r16][16bb + 4q + ii]
-    }
-    float mv[4];
+  for (int a = 1; a < NB; ++a) {
+    const int bt = w;
+    f32x4 res = zero4();
+    if (bt < a) {
+      f32x4 acc0 = zero4(), acc1 = zero4();
 #pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      {
-        const int i = 16 * a + 4 * q + ii, j = 16 * bb + r16;
-        const float d = (lam_h[i] - lam_h[j]) + (lam_l[i] - lam_l[j]);
-        const bool on = i > j && doc[i] == doc[j];
-        X[i * XP + j] = on ? bet_s[i] * fast_exp2(fminf(d, 0.f)) * gk[ii] : 0.f;
-        if (bb == a && (a & 1) == 0) X[i * XP + j + 16] = 0.f;
+      for (int cc = 0; cc < a; ++cc) {
+        if (cc >= bt) {
+          const f32x4 Ar = *reinterpret_cast<const f32x4*>(&X[(16 * a + r16) * AP + 16 * cc + 4 * q]);
+          const f32x4 Br = *reinterpret_cast<const f32x4*>(&Tt[(16 * bt + r16) * AP + 16 * cc + 4 * q]);
+#pragma unroll
+          for (int kk = 0; kk < 4; ++kk) {
+            if (cc & 1) acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Ar[kk], Br[kk], acc1, 0, 0, 0);
+            else acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(Ar[kk], Br[kk], acc0, 0, 0, 0);
+          }
+        }
       }
-      {
-        const int i = 16 * a + r16, j = 16 * bb + 4 * q + ii;
-        const float d = (lam_h[i] - lam_h[j]) + (lam_l[i] - lam_l[j]);
-        const bool on = i >= j && doc[i] == doc[j];
-        mv[ii] = on ? fast_exp2(fminf(d, 0.f)) * gq[ii] : 0.f;
-      }
+      const f32x4 Dr = *reinterpret_cast<const f32x4*>(&X[(16 * a + r16) * AP + 16 * a + 4 * q]);
+      // lane (j, q) holds P[4q + ii][j]: the B operand of step kk is acc[kk]
+      f32x4 r = zero4();
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        r = __builtin_amdgcn_mfma_f32_16x16x4f32(Dr[kk], acc0[kk] + acc1[kk], r, 0, 0, 0);
+      res = -r;
     }
-    const int mo = fofs(a, bb >> 1, l) + 4 * (bb & 1);
-    SS::st4s(g_Mh + mo, g_Ml + mo, mv);
-    if (bb == a && (a & 1) == 0) {
-      const float z[4] = {0.f, 0.f, 0.f, 0.f};
-      SS::st4s(g_Mh + mo + 4, g_Ml + mo + 4, z);
+    lds_barrier();   // row a of A is read
+    if (bt < a) {
+      // lane (j, q) holds T[16a + 4q + ii][16bt + j]
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) X[(16 * a + 4 * q + ii) * AP + 16 * bt + r16] = res[ii];
+      *reinterpret_cast<f32x4*>(&Tt[(16 * bt + r16) * AP + 16 * a + 4 * q]) = res;
+    }
+    lds_barrier();
+  }
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    if (s <= (w >> 1)) {
+      float x[8];
+      row8<float>(&X[(16 * w + r16) * AP + 32 * s], q, x);
+      SS::st8s(g_Th + tofs(w, s, l), g_Tl + tofs(w, s, l), x);
     }
   }
-  __syncthreads();
 }
 
 // ===========================================================================
-// k_prepass: everything per chunk that does not depend on the values (one
-// workgroup of 8 waves per (chunk, execution head, batch); wave w owns token
-// block w in the per-row phases and key tile w in phase 5): chunk flags,
-// Lambda, A and M, T = (I + A)^-1, W = T (b k e^Lambda), Pn = -ke^T W and
-// X = qe - M W; then U, Q and (M U)^T of every value column (value_cols).
+// k_prepass: the operands of one chunk that depend neither on the values nor
+// on the state (wave w owns token block w).
 //
 // Lambda is kept block-local: X[i] = sum of g over the 16-token block of i up
 // to and including i (log2 units, double-float hi in X / lo in Y), so a
@@ -420,116 +306,79 @@ __device__ __forceinline__ void prepass_scalar_gates(const PF& p, int b, int tb,
 // factors come from the per-block totals (sums of the totals before / after
 // block a, kept as the exponentials Ea / Sa).
 //
-// Products whose result feeds another kernel are computed transposed where
-// that puts the result directly in its consumer's fragment layout (M^T, Pn^T,
-// X^T); (b k e^Lambda)^T and ke^T are transposed by an identity product.
+// Bound by the latency of its dependent phases, so two independent workgroups
+// share a CU (80 KB of LDS, 256 VGPRs each).
 // ===========================================================================
-template <bool BF, class TV, int NT>
-__device__ __forceinline__ void value_cols(const PF& p, int b, int h, int c, int col0, int l, const VRows<TV>& vr,
-                                           const typename Store<BF>::ST* g_T, const typename Store<BF>::ST* g_keh,
-                                           const typename Store<BF>::ST* g_kel, const typename Store<BF>::ST* g_Mh,
-                                           const typename Store<BF>::ST* g_Ml);
-
-template <bool BF, class TIn, class TV, bool SC>
-__global__ __launch_bounds__(512) void k_prepass(const PF p) {
+template <bool BF, class TIn>
+__global__ __launch_bounds__(256, 2) void k_prepass(const PF p) {
   using P = Pol<BF>;
-  using F1 = typename P::F1;
   using F3 = typename P::F3;
   using SS = Store<BF>;
   using ST = typename SS::ST;
-  constexpr int YP = 132;
-  __shared__ float X[CH * XP];        // Lambda hi -> A -> T (fp32)
-  __shared__ float Y[CH * YP];        // Lambda lo -> Kc -> T fragment-native (ST)
-  __shared__ float Ftab[8 * KD];      // e^{total of block b}
-  __shared__ float Mid0[8 * KD];      // e^{g at the first token of block a}
-  __shared__ float Ea[8 * KD];        // e^{Lambda at the first token of block a} (chunk-global)
-  __shared__ float Sa[8 * KD];        // e^{sum of the totals of blocks > a}
-  __shared__ float Fa[8 * KD];        // e^{Lambda(last) - Lambda(first token) of block a}
-  __shared__ float Gt[8 * KD];        // e^{Lambda(first token of block a) - Lambda(row 64)}
+  __shared__ __align__(16) float X[CH * XP];   // Lambda hi -> A -> T (fp32)
+  __shared__ __align__(16) float Y[CH * XP];   // Lambda lo -> column factors -> T^T
+  __shared__ float Ftab[NB * KD];     // e^{total of block b}
+  __shared__ float Mid0[NB * KD];     // e^{g at the first token of block a}
+  __shared__ float Ea[NB * KD];       // e^{Lambda at the first token of block a} (chunk-global)
+  __shared__ float Sa[NB * KD];       // e^{sum of the totals of blocks > a}
+  __shared__ float Fa[NB * KD];       // e^{Lambda(last) - Lambda(first token) of block a}
+  __shared__ float Gt[NB * KD];       // e^{Lambda(first token of block a) - Lambda(row 32)}
   __shared__ int doc[CH];
-  __shared__ int unsafe_part[2][8];   // per 64-channel half: block needs the hierarchical path
+  __shared__ int unsafe_part[2][NB];  // per 64-channel half: block needs the hierarchical path
   __shared__ int wide_part[2];        // per 64-channel half: the chunk-reference path is unsafe
 
   const int tid = threadIdx.x;
-  // (the wave index as a scalar: loops and tile indices over waves stay in
-  // scalar registers, with no per-lane masks)
+  // (the wave index as a scalar: tile indices over waves stay in scalar registers)
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, r16 = l & 15, q = l >> 4;
-  const int units = p.B * p.Hx * p.NCb;
-  // chunk unit: XCD-aware remap (the hardware deals linear block ids to the 8
-  // XCDs round-robin; consecutive chunks of a head share one XCD's L2)
-  int c, h, b;
-  {
-    int id = blockIdx.x;
-    if ((units & 7) == 0) id = (id & 7) * (units >> 3) + (id >> 3);
-    c = id % p.NCb;
-    id /= p.NCb;
-    h = id % p.Hx;
-    b = id / p.Hx;
-  }
-  const int tb = p.t0 + c * CH;
-  const int t_end = min(p.t0 + p.nt, p.L);
-  const int64_t u = ((int64_t)b * p.Hx + h) * p.NCb + c;
-  const int64_t uf = u * (CH * KD);   // one 128 x 128 fragment-native array per unit
-  const int hk = p.gates_at_hv ? h / p.G : h;
-
-  ST* g_Pn = (ST*)p.PnA + uf;
-  ST* g_Xh = (ST*)p.XAh + uf;
-  ST* g_Xl = (ST*)p.XAl + uf;
-  ST* g_be = (ST*)p.BeB + uf;
-  ST* g_keh = (ST*)p.KeBh + uf;
-  ST* g_kel = (ST*)p.KeBl + uf;
-  ST* g_Mh = (ST*)p.MAh + uf;
-  ST* g_Ml = (ST*)p.MAl + uf;
-  float* g_qe = p.QeA + uf;
+  const Unit x0 = unit_of(p);
+  const int tb = x0.tb, t_end = x0.t_end, b = x0.b, h = x0.h;
+  const int64_t u = x0.u;
+  ST* g_be = (ST*)p.BeA + u * (CH * KD);
+  ST* g_qh = (ST*)p.QeAh + u * (CH * KD);
+  ST* g_ql = (ST*)p.QeAl + u * (CH * KD);
+  ST* g_keh = (ST*)p.KeTh + u * (CH * KD);
+  ST* g_kel = (ST*)p.KeTl + u * (CH * KD);
+  ST* g_Th = (ST*)p.TAh + u * TM;
+  ST* g_Tl = (ST*)p.TAl + u * TM;
+  ST* g_Mh = (ST*)p.MAh + u * TM;
+  ST* g_Ml = (ST*)p.MAl + u * TM;
   float* g_dv = p.dvec + u * KD;
 
   // Global loads are issued up front, in the order their values are needed
   // (the vector-memory counter drains in order, so a load is only ever waited
-  // for together with the loads issued before it): segment ids (phase 0),
-  // gates g (phase 1), then the q, k, b rows of this wave's token block
-  // (phase 2), whose latency then overlaps phases 0 and 1.
-  // (every lane loads, under wave-uniform conditions only, so no value is
-  // consumed inside a divergent branch before it is needed)
-  SegId sg_t{0, 0}, sg_tp{0, 0}, sg_0{0, 0}, sg_a{0, 0}, sg_b{0, 0};
-  int32_t iseg = 0;
-  if (p.seg != nullptr) {
-    const int ti = tid & (CH - 1);
-    sg_t = seg_raw(p, b, min(tb + ti, t_end - 1));
-    sg_tp = seg_raw(p, b, max(min(tb + ti - 1, t_end - 1), 0));
-    sg_0 = seg_raw(p, b, 0);
-    sg_a = seg_raw(p, b, tb);
-    sg_b = seg_raw(p, b, max(tb - 1, 0));
-  }
-  if (p.init_seg != nullptr) iseg = p.init_seg[b];
-  const int g_part = tid >> 7;   // phase 1: 4 parts of 32 tokens, channel tid & 127
-  float gl[SC ? 1 : 32];
-  if constexpr (SC) {
-    // one decay per token: thread t < 128 loads token t's (clamped to the last valid)
-    gl[0] = 0.f;
-    if (tid < CH) {
-      const int hg = kgate_head(p, p.g_h, h);
-      gl[0] = ((const float*)p.g)[((int64_t)b * p.L + min(tb + tid, t_end - 1)) * p.g_h + hg];
-    }
-  } else {
-    const int kap = tid & 127;
+  // for together with the loads issued before it).
+  ChunkSeg sg;
+  if (w == 0) sg.load(p, x0, l);
+  // gates g: lane (half, cg) holds tokens 16w + 8 half .. + 7 of channels
+  // 4cg..4cg+3 (a gate with one channel repeats it; out-of-range tokens read
+  // the last valid token and are zeroed below)
+  const int half = l >> 5, cg = l & 31;
+  f32x4 gl[8];
+  {
     const int hg = kgate_head(p, p.g_h, h);
-    const int tload = min(tb + 32 * g_part, t_end - 1);
-    const int nload = t_end - tload;   // >= 1
-    const int gstride = p.g_h * p.g_c;
-    const float* gp = (const float*)p.g + (((int64_t)b * p.L + tload) * p.g_h + hg) * p.g_c + (p.g_c == 1 ? 0 : kap);
-    // out-of-range tokens read the last valid token and are zeroed in phase 1
+    const int t8 = tb + 16 * w + 8 * half;
+    const float* gp = (const float*)p.g + ((int64_t)b * p.L * p.g_h + hg) * p.g_c;
+    const int64_t gs = (int64_t)p.g_h * p.g_c;
+    if (p.g_c == 1) {
 #pragma unroll
-    for (int i = 0; i < 32; ++i) gl[i] = gp[min(i, nload - 1) * gstride];
+      for (int i = 0; i < 8; ++i) {
+        const float* r = gp + min(t8 + i, t_end - 1) * gs;
+        gl[i] = f32x4{r[0], r[0], r[0], r[0]};
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) gl[i] = *reinterpret_cast<const f32x4*>(gp + min(t8 + i, t_end - 1) * gs + 4 * cg);
+    }
   }
-  const int hbg = kgate_head(p, p.b_h, h);
   Raw8<TIn> rq[4], rk[4];
   Raw8<float> rb[4];
   float b_scalar = 0.f;
   {
+    const int hbg = kgate_head(p, p.b_h, h);
     const int t = tb + 16 * w + r16;
     const int tt = t < t_end ? t : tb;
-    const TIn* qp = (const TIn*)p.q + (((int64_t)b * p.L + tt) * p.Hk + hk) * KD;
-    const TIn* kp = (const TIn*)p.k + (((int64_t)b * p.L + tt) * p.Hk + hk) * KD;
+    const TIn* qp = (const TIn*)p.q + (((int64_t)b * p.L + tt) * p.Hk + x0.hk) * KD;
+    const TIn* kp = (const TIn*)p.k + (((int64_t)b * p.L + tt) * p.Hk + x0.hk) * KD;
     const float* bp = (const float*)p.b + (((int64_t)b * p.L + tt) * p.b_h + hbg) * p.b_c;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -543,111 +392,83 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
       for (int s = 0; s < 4; ++s) rb[s].load(bp + 32 * s, q);
     }
   }
-  // first use of the segment ids: only now, after every entry load is issued
-  // (an empty asm that "updates" them keeps the compiler from comparing them
-  // earlier, which would wait before the later loads are even issued)
-  asm volatile("" : "+v"(sg_t.lo), "+v"(sg_t.hi), "+v"(sg_tp.lo), "+v"(sg_tp.hi));
-  asm volatile("" : "+v"(sg_0.lo), "+v"(sg_0.hi), "+v"(sg_a.lo), "+v"(sg_a.hi), "+v"(sg_b.lo), "+v"(sg_b.hi));
 
-  // ---- phase 0: in-chunk document index (segment canonicalisation) -------
-  // doc[i] = number of segment starts among tokens 1..i: a wave ballot and a
-  // popcount per token (waves 0 and 1 hold tokens 0..127), wave 1 adding
-  // wave 0's total
+  // ---- phase 1: block-local Lambda (double-float: X = hi, Y = lo) ----------
   {
-    __shared__ int starts0;
-    const bool st = tid < CH && tid > 0 && p.seg != nullptr && (sg_t != sg_tp);
-    const uint64_t bal = __ballot(st);
-    const int upto = __popcll(bal & ((2ull << l) - 1ull));   // lanes 0..l (l = 63: all)
-    if (tid == 0) starts0 = __popcll(bal);
-    __syncthreads();
-    if (tid < CH) doc[tid] = upto + (w == 1 ? starts0 : 0);
-    __syncthreads();
-  }
-  if (tid == 0 && h == 0) {
-    int is_new;
-    if (tb == 0) {
-      if (p.has_init) {
-        is_new = 0;
-        // initial_state_segment_id is int32; a wider first id differs from it
-        // when its high word is not the sign extension of its low word
-        if (p.init_seg != nullptr)
-          is_new = (sg_0.lo != iseg) || (p.seg_dt == DT_I64 && sg_0.hi != (iseg < 0 ? -1 : 0));
-      } else {
-        is_new = 1;
-      }
-    } else if (c == 0 && !p.has_init) {
-      is_new = 1;
-    } else {
-      is_new = p.seg ? (sg_a != sg_b) : 0;
-    }
-    p.flags[((int64_t)b * p.NCb + c) * 2 + 0] = is_new;
-    p.flags[((int64_t)b * p.NCb + c) * 2 + 1] = (doc[CH - 1] == 0);
-  }
-
-  if constexpr (SC) {
-    prepass_scalar_gates<TIn>(p, b, tb, t_end, gl[0], rq, rk, rb, b_scalar, doc, X, Y, g_Mh, g_Ml, g_be, g_keh,
-                              g_kel, g_qe, g_dv);
-  } else {
-  // ---- phase 1: block-local Lambda (double-float: X = hi, Y = lo), totals --
-  {
-    const int kap = tid & 127, part = g_part;
-    const int nvalid = t_end - (tb + 32 * part);   // tokens of this part in range (may be <= 0)
-    if (p.fuse) {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) gl[i] = -__expf(fminf(gl[i], 5.f));
-    } else {
-#pragma unroll
-      for (int i = 0; i < 32; ++i) gl[i] = fminf(gl[i], 0.f);  // _nonpositive (NaN -> 0)
-    }
     const float gmax = p.guard ? -1e-6f : 0.f;
+    const int nvalid = t_end - (tb + 16 * w + 8 * half);   // of this lane's tokens (may be <= 0)
+    f32x4 hi[8], lo[8];
+    f32x4 h = zero4(), lw = zero4();
 #pragma unroll
-    for (int i = 0; i < 32; ++i) gl[i] = (i < nvalid) ? fminf(gl[i], gmax) : 0.f;
+    for (int i = 0; i < 8; ++i) {
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      float hi = 0.f, lo = 0.f;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        // error-free accumulation (TwoSum), then an exact split of hi * log2(e)
-        const float gv = gl[16 * blk + j];
-        const float sum = hi + gv;
-        const float bb = sum - hi;
-        lo += (hi - (sum - bb)) + (gv - bb);
-        hi = sum;
-        const float ph = hi * kLog2e;
-        const float pe = fmaf(hi, kLog2e, -ph);
-        const int row = 32 * part + 16 * blk + j;
-        X[row * XP + kap] = ph;
-        Y[row * XP + kap] = pe + lo * kLog2e;
+      for (int e = 0; e < 4; ++e) {
+        float gv = gl[i][e];
+        gv = p.fuse ? -__expf(fminf(gv, 5.f)) : fminf(gv, 0.f);   // _nonpositive (NaN -> 0)
+        gv = i < nvalid ? fminf(gv, gmax) : 0.f;
+        // error-free accumulation (TwoSum)
+        const float sum = h[e] + gv;
+        const float bb = sum - h[e];
+        lw[e] += (h[e] - (sum - bb)) + (gv - bb);
+        h[e] = sum;
       }
+      hi[i] = h;
+      lo[i] = lw;
+    }
+    // the second half of the block continues the first (held by lane - 32)
+    f32x4 h1, l1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float hp = __shfl_xor(h[e], 32), lp = __shfl_xor(lw[e], 32);
+      h1[e] = half ? hp : 0.f;
+      l1[e] = half ? lp : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f32x4 xo, yo;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float sum = h1[e] + hi[i][e];
+        const float bb = sum - h1[e];
+        const float lt = l1[e] + lo[i][e] + ((h1[e] - (sum - bb)) + (hi[i][e] - bb));
+        // an exact split of hi * log2(e)
+        const float ph = sum * kLog2e;
+        xo[e] = ph;
+        yo[e] = fmaf(sum, kLog2e, -ph) + lt * kLog2e;
+      }
+      const int row = 16 * w + 8 * half + i;
+      *reinterpret_cast<f32x4*>(&X[row * XP + 4 * cg]) = xo;
+      *reinterpret_cast<f32x4*>(&Y[row * XP + 4 * cg]) = yo;
     }
   }
-  __syncthreads();
+  if (w == 0) sg.finish(p, x0, l, doc);
+  lds_barrier();
   if (tid < KD) {
-    float tot[8];
+    float tot[NB];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) tot[a] = X[(16 * a + 15) * XP + tid] + Y[(16 * a + 15) * XP + tid];
-    float acc = 0.f, lg[8];
+    for (int a = 0; a < NB; ++a) tot[a] = X[(16 * a + 15) * XP + tid] + Y[(16 * a + 15) * XP + tid];
+    float acc = 0.f, lg[NB];
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
+    for (int a = 0; a < NB; ++a) {
       const float lsa = X[(16 * a) * XP + tid] + Y[(16 * a) * XP + tid];
       lg[a] = acc + lsa;   // chunk-global Lambda at the first token of block a
       Ea[a * KD + tid] = fast_exp2(lg[a]);
+      Mid0[a * KD + tid] = fast_exp2(lsa);
       acc += tot[a];
     }
     g_dv[tid] = fast_exp2(acc);   // e^{Lambda_end}
-    // chunk reference row 64: every off-diagonal A / M entry factors as
-    // (row i: e^{Lambda_i - Lambda_64}) (column j: e^{Lambda_64 - Lambda_j}),
-    // both within 2^{+-100} when the spans on either side of row 64 are
-    bool wide = (lg[0] - lg[4] > kDiagSafeLog2) || (lg[4] - acc > kDiagSafeLog2);
+    // chunk reference row 32: every off-diagonal A / M entry factors as
+    // (row i: e^{Lambda_i - Lambda_32}) (column j: e^{Lambda_32 - Lambda_j}),
+    // both within 2^{+-100} when the spans on either side of row 32 are
+    bool wide = (lg[0] - lg[NB / 2] > kDiagSafeLog2) || (lg[NB / 2] - acc > kDiagSafeLog2);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) Gt[a * KD + tid] = fast_exp2(lg[a] - lg[4]);
+    for (int a = 0; a < NB; ++a) Gt[a * KD + tid] = fast_exp2(lg[a] - lg[NB / 2]);
     acc = 0.f;
 #pragma unroll
-    for (int a = 7; a >= 0; --a) { Sa[a * KD + tid] = fast_exp2(acc); acc += tot[a]; }
+    for (int a = NB - 1; a >= 0; --a) { Sa[a * KD + tid] = fast_exp2(acc); acc += tot[a]; }
 #pragma unroll
-    for (int a = 0; a < 8; ++a) {
+    for (int a = 0; a < NB; ++a) {
       Ftab[a * KD + tid] = fast_exp2(tot[a]);
-      Mid0[a * KD + tid] = fast_exp2(X[(16 * a) * XP + tid] + Y[(16 * a) * XP + tid]);
       // span of the block after its first token: Lambda(sa) - Lambda(ea) >= 0
       const int sa = 16 * a, ea = sa + 15;
       const float span = (X[sa * XP + tid] - X[ea * XP + tid]) + (Y[sa * XP + tid] - Y[ea * XP + tid]);
@@ -659,21 +480,19 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
     wide = __any(wide);
     if (l == 0) wide_part[w] = wide;
   }
-  __syncthreads();
+  lds_barrier();
   // no block needs the hierarchical path and the chunk reference is safe:
   // phase 2 leaves the column factors of every block as split fragments in
   // Y, and phase 3 is MFMA products of stored fragments only
   const bool chunk_ref = __builtin_amdgcn_readfirstlane(!(wide_part[0] | wide_part[1]));
 
-  // ---- phase 2: per-row quantities, diagonal A/M blocks --------------------
-  F3 Rf[1][4], Qf[1][4];
-  f32x4 Adiag[1];
-#pragma unroll
-  for (int bi = 0; bi < 1; ++bi) {
+  // ---- phase 2: per-row operands, diagonal A/M blocks ----------------------
+  F3 Rf[4], Qf[4];
+  f32x4 Adiag;
+  {
     const int a = w;
     const int i = 16 * a + r16;
-    const int t = tb + i;
-    const bool valid = t < t_end;
+    const bool valid = tb + i < t_end;
     float qv[32], kv[32], bet[32];
     row_inputs<TIn>(p, rq, rk, rb, b_scalar, valid, qv, kv, bet);
     const bool first = doc[i] == 0;
@@ -681,14 +500,14 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
     const bool blk_unsafe = unsafe_part[0][a] | unsafe_part[1][a];
     // accA: A tile (lane = column token); accM: M^T tile (lane = row token)
     f32x4 accA = zero4(), accM = zero4();
-    float dq = 0.f;
-#pragma unroll
-    for (int e = 0; e < 32; ++e) dq += qv[e] * kv[e];
-    dq += __shfl_xor(dq, 16);
-    dq += __shfl_xor(dq, 32);
     // Blocks with a large in-block decay span take the hierarchical path
     // first, while the slab loop's fragments are not yet live.
     if (blk_unsafe) {
+      float dq = 0.f;
+#pragma unroll
+      for (int e = 0; e < 32; ++e) dq += qv[e] * kv[e];
+      dq += __shfl_xor(dq, 16);
+      dq += __shfl_xor(dq, 32);
       // Overflow-free hierarchical factorisation: the pair (i, j) is split at
       // the highest bit where the in-block indices differ; rows above and
       // columns below the split point are scaled toward it, so every
@@ -783,21 +602,18 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
           qe[e] = first ? qh * eL : 0.f;
         }
       }
-      Store<false>::st8(g_qe + fofs(a, s, l), qe);
+      SS::st8(g_be + fofs(a, s, l), bt);
+      SS::st8s(g_qh + fofs(a, s, l), g_ql + fofs(a, s, l), qe);
       {
-        // (b k e^Lambda)^T and ke^T in fragment layout (row = key, k = token)
-        const F1 fbt = P::f1(bt);
+        // ke^T in fragment layout (row = key, k = token)
         const F3 fkt = P::f3(kt);
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
-          const F1 id = ident_frag<BF>(hf, r16, q);
-          f32x4 cb = zero4(), chi = zero4();
-          mma(cb, fbt, id);
+          const auto id = ident_frag<BF>(hf, r16, q);
+          f32x4 chi = zero4();
           mma(chi, P::hi(fkt), id);
-          const int o = fofs(2 * s + hf, a >> 1, l) + 4 * (a & 1);
-          const float xb[4] = {cb[0], cb[1], cb[2], cb[3]};
+          const int o = fofs2(2 * s + hf, a >> 1, l) + 4 * (a & 1);
           const float xh[4] = {chi[0], chi[1], chi[2], chi[3]};
-          SS::st4(g_be + o, xb);
           SS::st4(g_keh + o, xh);
           if constexpr (BF) {
             f32x4 clo = zero4();
@@ -808,7 +624,7 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
         }
       }
       if (chunk_ref) {
-        // rows relative to row 64 instead of the block's first token
+        // rows relative to row 32 instead of the block's first token
         float gt[8];
         row8<float>(&Gt[a * KD + 32 * s], q, gt);
 #pragma unroll
@@ -818,20 +634,20 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
           bd[e] *= __builtin_amdgcn_rcpf(gt[e]);
         }
       }
-      Rf[bi][s] = P::f3(rA);
-      Qf[bi][s] = P::f3(rM);
+      Rf[s] = P::f3(rA);
+      Qf[s] = P::f3(rM);
       if (!blk_unsafe) {
         // A_aa, M_aa = (R, Qr) (k e^{Lambda_ref - Lambda})^T: every factor stays
         // within 2^{+-100} of 1, so the factorisation cannot overflow.
         const F3 fb = P::f3(bd);
-        P::m33(accA, Rf[bi][s], fb);
-        P::m33(accM, fb, Qf[bi][s]);
+        P::m33(accA, Rf[s], fb);
+        P::m33(accM, fb, Qf[s]);
         if (chunk_ref) {
           // the column factors replace this slab's 16 rows x 32 columns of
           // Lambda low words (2 KB, once all lanes of the wave have read
           // them) as the split fragment of lane l: row l / 4, 32 bytes at
           // (l % 4) * 32 of the slab's 128 bytes in that row
-          ST* fp = reinterpret_cast<ST*>(&Y[(16 * a + (l >> 2)) * YP + 32 * s]) + (l & 3) * (32 / sizeof(ST));
+          ST* fp = reinterpret_cast<ST*>(&Y[(16 * a + (l >> 2)) * XP + 32 * s]) + (l & 3) * (32 / sizeof(ST));
           SS::stf(fp, P::hi(fb));
           if constexpr (BF) SS::stf(fp + 8, fb.lo);
         }
@@ -839,8 +655,8 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
       if (!chunk_ref) {
         // Kc replaces this slab of the row's Lambda low words once all lanes
         // of the wave have read it (the other slabs' columns are untouched)
-        st4<float>(&Y[i * YP + 32 * s + 4 * q], kc);
-        st4<float>(&Y[i * YP + 32 * s + 16 + 4 * q], kc + 4);
+        st4<float>(&Y[i * XP + 32 * s + 4 * q], kc);
+        st4<float>(&Y[i * XP + 32 * s + 16 + 4 * q], kc + 4);
       }
     }
     // diagonal blocks: A (row-major, LDS) and M (fragment-native, rows = token)
@@ -849,591 +665,363 @@ __global__ __launch_bounds__(512) void k_prepass(const PF p) {
     for (int ii = 0; ii < 4; ++ii) {
       const int il = 4 * q + ii, ia = 16 * a + il, ja = 16 * a + r16;
       const bool same = doc[ia] == doc[ja];
-      Adiag[bi][ii] = (il > r16 && same) ? accA[ii] : 0.f;   // A[ia][ja]
+      Adiag[ii] = (il > r16 && same) ? accA[ii] : 0.f;        // A[ia][ja]
       mv[ii] = (r16 >= il && same) ? accM[ii] : 0.f;          // M[ja][ia]
     }
-    const int mo = fofs(a, a >> 1, l) + 4 * (a & 1);
+    const int mo = tofs(a, a >> 1, l) + 4 * (a & 1);
     SS::st4s(g_Mh + mo, g_Ml + mo, mv);
     if ((a & 1) == 0) {
       const float z[4] = {0.f, 0.f, 0.f, 0.f};
       SS::st4s(g_Mh + mo + 4, g_Ml + mo + 4, z);
     }
   }
-  __syncthreads();
+  lds_barrier();
 
   // ---- phase 3: off-diagonal A/M blocks (X becomes A) -----------------------
-  // Block a has a pairs (a, bb < a).  Blocks 4..7 keep the pairs with
-  // bb >= lo(a) = 1, 2, 3, 3 and hand the others to wave 7 - a, whose own
-  // block has 7 - a pairs, so no wave computes more than 4.  The R / Q
-  // fragments of blocks 4..7 reach those waves through X, which holds nothing
-  // live between phases 2 and 4: every wave keeps its A tiles in registers
-  // until all pairs are done and writes them to X afterwards.
+  // Wave a forms the pairs (a, bb < a).
   {
-    constexpr int RQA = 2048;                       // elements per fragment array
-    constexpr int RQB = (BF ? 4 : 2) * RQA;         // per block: R hi, (R lo,) Q hi, (Q lo)
-    ST* rq_s = reinterpret_cast<ST*>(X);
-    auto rq_ptr = [&](int a, int which, bool lo) -> ST* {   // which: 0 = R, 1 = Q
-      return rq_s + (a - 4) * RQB + (BF ? (2 * which + (lo ? 1 : 0)) : which) * RQA;
-    };
-    if (w >= 4) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int o = (s * 64 + l) * 8;
-        SS::stf(rq_ptr(w, 0, false) + o, P::hi(Rf[0][s]));
-        SS::stf(rq_ptr(w, 1, false) + o, P::hi(Qf[0][s]));
-        if constexpr (BF) {
-          SS::stf(rq_ptr(w, 0, true) + o, Rf[0][s].lo);
-          SS::stf(rq_ptr(w, 1, true) + o, Qf[0][s].lo);
-        }
-      }
-    }
-    __syncthreads();
-    auto lo_of = [](int a) { return a < 4 ? 0 : (a == 4 ? 1 : (a == 5 ? 2 : 3)); };
-    f32x4 Ap[4];
-    int pa[4], pb[4];
-    int np = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { Ap[k] = zero4(); pa[k] = 0; pb[k] = 0; }
+    const int a = w;
     // one pair's A tile (rows of block a) and M^T tile, masked by document
-    auto pair_out = [&](int a, int bb, f32x4 accA, const f32x4& accM) {
+    auto pair_out = [&](int bb, const f32x4& accA, const f32x4& accM) {
       float mv[4];
 #pragma unroll
       for (int ii = 0; ii < 4; ++ii) {
         const int ia = 16 * a + 4 * q + ii, jb = 16 * bb + r16;
-        accA[ii] = (doc[ia] == doc[jb]) ? accA[ii] : 0.f;
+        X[ia * AP + jb] = (doc[ia] == doc[jb]) ? accA[ii] : 0.f;
         mv[ii] = (doc[16 * a + r16] == doc[16 * bb + 4 * q + ii]) ? accM[ii] : 0.f;
       }
-      const int mo = fofs(a, bb >> 1, l) + 4 * (bb & 1);
+      const int mo = tofs(a, bb >> 1, l) + 4 * (bb & 1);
       SS::st4s(g_Mh + mo, g_Ml + mo, mv);
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (np == k) { Ap[k] = accA; pa[k] = a; pb[k] = bb; }
-      ++np;
     };
-    auto pairs_ref = [&](int a, const F3 (&RF)[4], const F3 (&QF)[4], int bb_hi, int bb_lo) {
-      auto ld_fb = [&](int bb, F3 (&fb)[4]) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const ST* fp = reinterpret_cast<const ST*>(&Y[(16 * bb + (l >> 2)) * YP + 32 * s]) + (l & 3) * (32 / sizeof(ST));
-          if constexpr (BF) {
-            fb[s].hi = SS::fa(fp);
-            fb[s].lo = SS::fa(fp + 8);
-          } else {
-            fb[s] = SS::fa(fp);
-          }
-        }
-      };
-      F3 fb[4];
-      ld_fb(bb_hi, fb);
-      for (int bb = bb_hi; bb >= bb_lo; --bb) {
+    if (chunk_ref) {
+      for (int bb = a - 1; bb >= 0; --bb) {
         // two accumulators per tile (leading and correction products) halve
         // the dependent MFMA chains
         f32x4 accA = zero4(), accM = zero4(), accA2 = zero4(), accM2 = zero4();
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
+          const ST* fp = reinterpret_cast<const ST*>(&Y[(16 * bb + (l >> 2)) * XP + 32 * s]) + (l & 3) * (32 / sizeof(ST));
           if constexpr (BF) {
-            mma(accA, RF[s].hi, fb[s].hi);   // A[16a + 4q + ii][16bb + r16]
-            mma(accM, fb[s].hi, QF[s].hi);   // M[16a + r16][16bb + 4q + ii]
-            mma(accA2, RF[s].hi, fb[s].lo);
-            mma(accM2, fb[s].hi, QF[s].lo);
-            mma(accA2, RF[s].lo, fb[s].hi);
-            mma(accM2, fb[s].lo, QF[s].hi);
+            const F3 fb = SS::fa3(fp, fp + 8);
+            mma(accA, Rf[s].hi, fb.hi);   // A[16a + 4q + ii][16bb + r16]
+            mma(accM, fb.hi, Qf[s].hi);   // M[16a + r16][16bb + 4q + ii]
+            mma(accA2, Rf[s].hi, fb.lo);
+            mma(accM2, fb.hi, Qf[s].lo);
+            mma(accA2, Rf[s].lo, fb.hi);
+            mma(accM2, fb.lo, Qf[s].hi);
           } else {
-            P::m33(s & 1 ? accA2 : accA, RF[s], fb[s]);
-            P::m33(s & 1 ? accM2 : accM, fb[s], QF[s]);
+            const F3 fb = SS::fa(fp);
+            P::m33(s & 1 ? accA2 : accA, Rf[s], fb);
+            P::m33(s & 1 ? accM2 : accM, fb, Qf[s]);
           }
         }
-        if (bb > bb_lo) ld_fb(bb - 1, fb);
 #pragma unroll
         for (int ii = 0; ii < 4; ++ii) { accA[ii] += accA2[ii]; accM[ii] += accM2[ii]; }
-        pair_out(a, bb, accA, accM);
+        pair_out(bb, accA, accM);
       }
-    };
-    auto pairs = [&](int a, const F3 (&RF)[4], const F3 (&QF)[4], int bb_hi, int bb_lo) {
-      if (chunk_ref) {
-        pairs_ref(a, RF, QF, bb_hi, bb_lo);
-        return;
-      }
+    } else {
       float mloc[32];
 #pragma unroll
       for (int s = 0; s < 4; ++s) row8<float>(&Mid0[a * KD + 32 * s], q, mloc + 8 * s);
-      for (int b2 = a - 1; b2 > bb_hi; --b2) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          float f[8];
-          row8<float>(&Ftab[b2 * KD + 32 * s], q, f);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) mloc[8 * s + e] *= f[e];
-        }
-      }
-      for (int bb = bb_hi; bb >= bb_lo; --bb) {
+      for (int bb = a - 1; bb >= 0; --bb) {
         f32x4 accA = zero4(), accM = zero4();
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
-          float x[8];
-          row8<float>(&Y[(16 * bb + r16) * YP + 32 * s], q, x);
+          float x[8], f[8];
+          row8<float>(&Y[(16 * bb + r16) * XP + 32 * s], q, x);
+          row8<float>(&Ftab[bb * KD + 32 * s], q, f);
 #pragma unroll
           for (int e = 0; e < 8; ++e) x[e] *= mloc[8 * s + e];
           const F3 fb = P::f3(x);
-          P::m33(accA, RF[s], fb);   // A[16a + 4q + ii][16bb + r16]
-          P::m33(accM, fb, QF[s]);   // M[16a + r16][16bb + 4q + ii]
-        }
-        pair_out(a, bb, accA, accM);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          float f[8];
-          row8<float>(&Ftab[bb * KD + 32 * s], q, f);
+          P::m33(accA, Rf[s], fb);   // A[16a + 4q + ii][16bb + r16]
+          P::m33(accM, fb, Qf[s]);   // M[16a + r16][16bb + 4q + ii]
 #pragma unroll
           for (int e = 0; e < 8; ++e) mloc[8 * s + e] *= f[e];
         }
-      }
-    };
-    pairs(w, Rf[0], Qf[0], w - 1, lo_of(w));
-    if (w < 4) {
-      const int a1 = 7 - w;
-      F3 RF[4], QF[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const int o = (s * 64 + l) * 8;
-        RF[s] = SS::fa3(rq_ptr(a1, 0, false) + o, rq_ptr(a1, 0, true) + o);
-        QF[s] = SS::fa3(rq_ptr(a1, 1, false) + o, rq_ptr(a1, 1, true) + o);
-      }
-      pairs(a1, RF, QF, lo_of(a1) - 1, 0);
-    }
-    __syncthreads();
-    // A tiles of this wave's pairs and of its own diagonal block
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (k < np) {
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) X[(16 * pa[k] + 4 * q + ii) * XP + 16 * pb[k] + r16] = Ap[k][ii];
+        pair_out(bb, accA, accM);
       }
     }
-    {
-      const int a = w;
+    // this wave's diagonal block
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        const int ia = 16 * a + 4 * q + ii;
-        X[ia * XP + 16 * a + r16] = Adiag[0][ii];
-        if ((a & 1) == 0) X[ia * XP + 16 * a + 16 + r16] = 0.f;
-      }
+    for (int ii = 0; ii < 4; ++ii) {
+      const int ia = 16 * a + 4 * q + ii;
+      X[ia * AP + 16 * a + r16] = Adiag[ii];
+      if ((a & 1) == 0) X[ia * AP + 16 * a + 16 + r16] = 0.f;
     }
   }
-  __syncthreads();
-
-  }
-
-  // M (and, in bf16 mode, the high words of ke^T) are staged into LDS for
-  // phase 5 once T no longer needs it; their loads are issued here so they
-  // overlap the substitution.  16 bytes per load, 4 per array and thread.
-  constexpr bool kStageKe = BF;
-  using V16 = f32x4;
-  V16 st_mh[4], st_ml[4], st_ke[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int o = (tid + 512 * j) * (16 / (int)sizeof(ST));   // element offset of chunk
-    st_mh[j] = *reinterpret_cast<const V16*>(g_Mh + o);
-    if constexpr (BF) st_ml[j] = *reinterpret_cast<const V16*>(g_Ml + o);
-    if constexpr (kStageKe) st_ke[j] = *reinterpret_cast<const V16*>(g_keh + o);
-  }
-
-  // ---- phase 4: T = (I + A)^-1 (blocked forward substitution, fp32) -------
-  if (w < 2) {
-    const int a = 4 * w + q;
-    float tc[16];
-#pragma unroll
-    for (int m = 0; m < 16; ++m) tc[m] = (m == r16) ? 1.f : 0.f;
-#pragma unroll
-    for (int ii = 1; ii < 16; ++ii) {
-      float acc = 0.f;
-#pragma unroll
-      for (int m = 0; m < ii; ++m) acc += X[(16 * a + ii) * XP + 16 * a + m] * tc[m];
-      if (ii > r16) tc[ii] = -acc;
-    }
-#pragma unroll
-    for (int ii = 0; ii < 16; ++ii) X[(16 * a + ii) * XP + 16 * a + r16] = tc[ii];
-    // and transposed (Tt = Y, free during this phase: row 16a + r16 holds
-    // column r16 of the block), the B operand layout of the steps below
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4)
-      *reinterpret_cast<f32x4*>(&Y[(16 * a + r16) * YP + 16 * a + 4 * i4]) =
-          f32x4{tc[4 * i4], tc[4 * i4 + 1], tc[4 * i4 + 2], tc[4 * i4 + 3]};
-  }
-  __syncthreads();
-  // Block row a: T[a][bt] = -D_a sum_{cc = bt}^{a-1} A[a][cc] T[cc][bt], by
-  // wave bt.  Each 16x16x16 product runs as 4 steps of the 16x16x4 fp32
-  // MFMA with lane (r, q) holding reduction index 4q + kk at step kk, so a
-  // lane's A operand (row of A) and B operand (row of T^T, kept in Y) are
-  // one 16-byte LDS read each; all of a step's reads are issued before its
-  // MFMAs, and the sum runs in two accumulation chains.
-  float* Tt = Y;
-  for (int a = 1; a < 8; ++a) {
-    const int bt = w;
-    f32x4 res = zero4();
-    if (bt < a) {
-      f32x4 Ar[7], Br[7];
-#pragma unroll
-      for (int cc = 0; cc < 7; ++cc) {
-        if (cc >= bt && cc < a) {
-          Ar[cc] = *reinterpret_cast<const f32x4*>(&X[(16 * a + r16) * XP + 16 * cc + 4 * q]);
-          Br[cc] = *reinterpret_cast<const f32x4*>(&Tt[(16 * bt + r16) * YP + 16 * cc + 4 * q]);
-        }
-      }
-      const f32x4 Dr = *reinterpret_cast<const f32x4*>(&X[(16 * a + r16) * XP + 16 * a + 4 * q]);
-      f32x4 acc0 = zero4(), acc1 = zero4();
-#pragma unroll
-      for (int cc = 0; cc < 7; ++cc) {
-        if (cc >= bt && cc < a) {
-#pragma unroll
-          for (int kk = 0; kk < 4; ++kk) {
-            if (cc & 1) acc1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Ar[cc][kk], Br[cc][kk], acc1, 0, 0, 0);
-            else acc0 = __builtin_amdgcn_mfma_f32_16x16x4f32(Ar[cc][kk], Br[cc][kk], acc0, 0, 0, 0);
-          }
-        }
-      }
-      f32x4 acc;
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) acc[ii] = acc0[ii] + acc1[ii];
-      // lane (j, q) holds P[4q + ii][j]: the B operand of step kk is acc[kk]
-      f32x4 r = zero4();
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) r = __builtin_amdgcn_mfma_f32_16x16x4f32(Dr[kk], acc[kk], r, 0, 0, 0);
-      res = -r;
-    }
-    __syncthreads();
-    if (bt < a) {
-      // lane (j, q) holds T[16a + 4q + ii][16bt + j]
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) X[(16 * a + 4 * q + ii) * XP + 16 * bt + r16] = res[ii];
-      *reinterpret_cast<f32x4*>(&Tt[(16 * bt + r16) * YP + 16 * a + 4 * q]) = res;
-    }
-    __syncthreads();
-  }
-  // T in fragment-native layout in Y (LDS), for W and the value columns.  In
-  // bf16 mode its low words go after it, where ke^T is staged once W is formed.
-  ST* Ts = reinterpret_cast<ST*>(Y);
-  ST* Tl = Ts + CH * KD;
-  F1 Bbe[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) Bbe[s] = SS::fa(g_be + fofs(w, s, l));
-  for (int idx = w; idx < 32; idx += 8) {
-    const int rt = idx >> 2, s = idx & 3;
-    if (s > (rt >> 1)) continue;
-    float x[8];
-    row8<float>(&X[(16 * rt + r16) * XP + 32 * s], q, x);
-    if constexpr (BF) SS::st8s(Ts + fofs(rt, s, l), Tl + fofs(rt, s, l), x);
-    else SS::st8(Ts + fofs(rt, s, l), x);
-  }
-  __syncthreads();
-  // ---- W = T be (key tile w) -------------------------------------------------
-  // In bf16 mode T enters as high and low words: with nearly repeated keys
-  // and b near 1, T is close to I minus a unit subdiagonal and W = T be
-  // cancels to a small remainder, which a bf16-rounded T would leave with
-  // 2^-9 / (1 - b) relative error (identical keys, b = 0.993: 7e-2 of the
-  // output against 9e-3 with T split).
-  f32x4 Wc[8];
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt) Wc[rt] = zero4();
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      if (s <= rt / 2) {
-        P::m11(Wc[rt], SS::fa(Ts + fofs(rt, s, l)), Bbe[s]);
-        if constexpr (BF) P::m11(Wc[rt], SS::fa(Tl + fofs(rt, s, l)), Bbe[s]);
-      }
-    }
-  }
-  if constexpr (BF) __syncthreads();   // T's low words are read: ke^T takes their place
-  // X (T in fp32) is free now: M high / low words there, ke^T high words
-  // after T in Y (bf16 mode)
-  ST* Mh_s = reinterpret_cast<ST*>(X);
-  ST* Ml_s = BF ? Mh_s + CH * CH : Mh_s;
-  ST* ke_s = Ts + CH * KD;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int o = (tid + 512 * j) * (16 / (int)sizeof(ST));
-    *reinterpret_cast<V16*>(Mh_s + o) = st_mh[j];
-    if constexpr (BF) *reinterpret_cast<V16*>(Ml_s + o) = st_ml[j];
-    if constexpr (kStageKe) *reinterpret_cast<V16*>(ke_s + o) = st_ke[j];
-  }
-  const ST* keA = kStageKe ? ke_s : g_keh;
-  if constexpr (!BF) {
-    // fp32 mode: M is 64 KB (the 4 loads above covered 32 KB); finish it
-#pragma unroll
-    for (int j = 4; j < 8; ++j) {
-      const int o = (tid + 512 * j) * 4;
-      *reinterpret_cast<V16*>(Mh_s + o) = *reinterpret_cast<const V16*>(g_Mh + o);
-    }
-  }
-  __syncthreads();
-
-  // The v rows of this wave's first value tile (16-column tiles, bf16 v) are
-  // issued now, ahead of phase 5's loads and stores: they arrive while W, Pn
-  // and X are formed.
-  constexpr bool kPreV = std::is_same<TV, bf16>::value;
-  VRows<TV> vpre;
-  if (kPreV && p.Vp < 256 && w < p.Vp / 16) v_rows_issue<TV>(p, b, h, c, 16 * w, l, vpre);
-
-  // ---- phase 5: Pn = -ke^T W ; X = qe - M W  (key tile w; W formed above) ----
-  // W^T fragments (rows = key j, k = token), and their negation
-  F3 W3[4], W3n[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    float x[8] = {Wc[2 * s][0], Wc[2 * s][1], Wc[2 * s][2], Wc[2 * s][3],
-                  Wc[2 * s + 1][0], Wc[2 * s + 1][1], Wc[2 * s + 1][2], Wc[2 * s + 1][3]};
-    W3[s] = P::f3(x);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = -x[e];
-    W3n[s] = P::f3(x);
-  }
-  // Pn^T tile (keys 16w.., state rows 16m..): lane (c, q) holds
-  // Pn[16m + c][16w + 4q + ii] = element 4(w & 1) + ii of slab w / 2 of Pn's fragment
-  const int hofs = 4 * (w & 1);
-  auto pn_tile = [&](int m, const F1 (&kb)[4]) {
-    f32x4 P0 = zero4();
-#pragma unroll
-    for (int s = 0; s < 4; ++s) P::m11(P0, P::hi(W3[s]), kb[s]);
-    const float x[4] = {-P0[0], -P0[1], -P0[2], -P0[3]};
-    SS::st4(g_Pn + fofs(m, w >> 1, l) + hofs, x);
-  };
-  {
-    F1 kb0[4], kb1[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) kb0[s] = SS::fa(keA + fofs(0, s, l));
-#pragma unroll 1
-    for (int m = 0; m < 8; m += 2) {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) kb1[s] = SS::fa(keA + fofs(m + 1, s, l));
-      pn_tile(m, kb0);
-      if (m + 2 < 8) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) kb0[s] = SS::fa(keA + fofs(m + 2, s, l));
-      }
-      pn_tile(m + 1, kb1);
-    }
-  }
-  // X^T tile (keys 16w.., tokens 16rt..): lane (c, q) holds
-  // X[16rt + c][16w + 4q + ii] = element 4(w & 1) + ii of slab w / 2 of X's fragment.
-  // Operands of tile rt + 1 load while tile rt computes.
-  struct XOps {
-    f32x4 q0;
-    F3 m[4];
-  };
-  auto ld_x = [&](int rt, XOps& o) {
-    o.q0 = *reinterpret_cast<const f32x4*>(g_qe + fofs(rt, w >> 1, l) + hofs);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (s <= rt / 2) o.m[s] = SS::fa3(Mh_s + fofs(rt, s, l), Ml_s + fofs(rt, s, l));
-  };
-  auto x_tile = [&](int rt, const XOps& o) {
-    f32x4 X0 = o.q0;
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (s <= rt / 2) P::m33(X0, W3n[s], o.m[s]);
-    const float x[4] = {X0[0], X0[1], X0[2], X0[3]};
-    const int xo = fofs(rt, w >> 1, l) + hofs;
-    SS::st4s(g_Xh + xo, g_Xl + xo, x);
-  };
-  {
-    XOps xa, xb;
-    ld_x(0, xa);
-#pragma unroll 1
-    for (int rt = 0; rt < 8; rt += 2) {
-      ld_x(rt + 1, xb);
-      x_tile(rt, xa);
-      if (rt + 2 < 8) ld_x(rt + 2, xa);
-      x_tile(rt + 1, xb);
-    }
-  }
-  // ---- phase 6: U, Q and (M U)^T of value columns 32g.. (wave w: g = w, w + 8, ..)
-  // from the copies of T, M (and in bf16 mode ke^T's high words) phase 5
-  // read from LDS; ke^T's low words from the workspace (written in phase 2).
-  // One workgroup holding T, ke and M on chip replaces a separate launch
-  // that reloaded them once per 32 columns (config 2: 91 vs 94 µs per step,
-  // config 5: 3.7 vs 4.2 ms).
-  // 32 columns per wave when every wave gets some, else 16 (value heads of 128
-  // columns: all 8 waves instead of 4)
-  if (p.Vp >= 256) {
-    for (int g = w; g < p.Vp / 32; g += 8) {
-      VRows<TV> vr;
-      v_rows_issue<TV>(p, b, h, c, 32 * g, l, vr);
-      value_cols<BF, TV, 2>(p, b, h, c, 32 * g, l, vr, Ts, keA, g_kel, Mh_s, Ml_s);
-    }
-  } else {
-    for (int g = w; g < p.Vp / 16; g += 8) {
-      if (!(kPreV && g == w)) v_rows_issue<TV>(p, b, h, c, 16 * g, l, vpre);
-      value_cols<BF, TV, 1>(p, b, h, c, 16 * g, l, vpre, Ts, keA, g_kel, Mh_s, Ml_s);
-    }
-  }
+  lds_barrier();
+  invert_and_store<BF>(X, Y, g_Th, g_Tl, w, l);
 }
 
 // ===========================================================================
-// value_cols: U = T (w*v), Q = ke^T U and (M U)^T for value columns
-// [col0, col0 + 16 NT) of one chunk unit -- one wave's share, the last phase of
-// k_prepass.  The (w*v)^T fragments are formed here from v and w; T, ke^T
-// (high / low words) and M (high / low words) are the unit's fragment-native
-// arrays (LDS or workspace pointers).
+// k_prepass_sc: the prepass for one decay, one b and one w per (token, head)
+// (the Gated DeltaNet form, chunk_gdn: gdn.py:66-110 broadcasts them over the
+// channels), precision "bf16" with bf16 q and k.  The per-channel machinery
+// collapses:
+//   * Lambda is one cumulative sum per token (double-float, log2 units);
+//   * the normalised q and k are exactly bf16 (they are rounded back to the
+//     input type), so the Gram matrices k k^T and q k^T are single bf16 MFMAs
+//     with fp32 accumulation, and
+//       A[i][j] = b_i e^{Lambda_i - Lambda_j} (k k^T)[i][j]   (i > j),
+//       M[i][j] =     e^{Lambda_i - Lambda_j} (q k^T)[i][j]   (i >= j),
+//     one exponential per pair, whose exponent is <= 0 for every unmasked
+//     pair (no factorisation, no overflow path);
+//   * be, qe and ke are row scalars times k, q and k: the scan takes the
+//     normalised rows once per key head (k, q and k^T fragments, single bf16
+//     words, exact) and the row scalars per execution head.
 // ===========================================================================
-template <bool BF, class TV, int NT>
-__device__ __forceinline__ void value_cols(const PF& p, int b, int h, int c, int col0, int l, const VRows<TV>& vr,
-                                           const typename Store<BF>::ST* g_T, const typename Store<BF>::ST* g_keh,
-                                           const typename Store<BF>::ST* g_kel, const typename Store<BF>::ST* g_Mh,
-                                           const typename Store<BF>::ST* g_Ml) {
-  using P = Pol<BF>;
-  using F1 = typename P::F1;
-  using F3 = typename P::F3;
-  using SS = Store<BF>;
-  using ST = typename SS::ST;
-  const int64_t u = ((int64_t)b * p.Hx + h) * p.NCb + c;
-  float* g_Q = p.QC + u * (int64_t)(KD * p.Vp);
-  float* g_Oi = p.OiT + u * (int64_t)(CH * p.Vp);
+template <class TIn>
+__global__ __launch_bounds__(256, 3) void k_prepass_sc(const PF p) {
+  using P = Pol<true>;
+  using F1 = P::F1;
+  using SS = Store<true>;
+  __shared__ __align__(16) float X[CH * AP];           // A -> T (fp32)
+  __shared__ __align__(16) bf16 Kf[2 * CH * KD];       // k, then q fragments [block][slab][lane][8]; -> T^T
+  __shared__ float lam_h[CH], lam_l[CH];               // Lambda (log2 units), double-float
+  __shared__ float bet_s[CH];                          // b per token (0 past the end)
+  __shared__ int doc[CH];
+  bf16* Qf = Kf + CH * KD;
 
-  // (w*v)^T fragments of this wave's value columns (rows = column, k = token)
-  F3 Bwv[NT][4];
-  wv_frags<BF, TV, NT>(p, b, h, c, col0, l, vr, Bwv);
-  f32x4 Uc[NT][8];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int rt = 0; rt < 8; ++rt) Uc[nt][rt] = zero4();
-#pragma unroll
-  for (int rt = 0; rt < 8; ++rt) {
-#pragma unroll
-    for (int s = 0; s <= rt / 2; ++s) {
-      const F1 t = SS::fa(g_T + fofs(rt, s, l));
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) P::m13(Uc[nt][rt], t, Bwv[nt][s]);
-    }
-    // T read where it is used: keep the scheduler from hoisting every row's
-    // fragment reads ahead (that would need them all live at once)
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // U^T fragments (rows = value column, k = token)
-  F3 U3[NT][4];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float x[8] = {Uc[nt][2 * s][0], Uc[nt][2 * s][1], Uc[nt][2 * s][2], Uc[nt][2 * s][3],
-                          Uc[nt][2 * s + 1][0], Uc[nt][2 * s + 1][1], Uc[nt][2 * s + 1][2], Uc[nt][2 * s + 1][3]};
-      U3[nt][s] = P::f3(x);
-    }
-  const int ct0 = col0 / 16;   // value tile of nt = 0 within the execution head
-  // Q tiles (rows = key, columns = value), the chain's accumulator layout
-  auto q_tile = [&](int m, const F3 (&ka)[4]) {
-    f32x4 Qa[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) Qa[nt] = zero4();
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) P::m33(Qa[nt], ka[s], U3[nt][s]);
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) *reinterpret_cast<f32x4*>(g_Q + cofs(m, ct0 + nt, p.nct, l)) = Qa[nt];
-  };
-  auto ld_ke = [&](int m, F3 (&ka)[4]) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) ka[s] = SS::fa3(g_keh + fofs(m, s, l), g_kel + fofs(m, s, l));
-  };
+  const int tid = threadIdx.x;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63, r16 = l & 15, q = l >> 4;
+  const Unit x0 = unit_of(p);
+  const int tb = x0.tb, t_end = x0.t_end, b = x0.b, h = x0.h;
+  const int64_t u = x0.u;
+  const int64_t ku = ((int64_t)b * p.Hk + x0.hk) * p.NCb + x0.c;   // key-head unit of the k, q operands
+  const bool rows_out = !p.gates_at_hv || h % p.G == 0;           // one unit per key head stores them
+
+  ChunkSeg sg;
+  if (w == 0) sg.load(p, x0, l);
+  float g_tok = 0.f;
+  if (w == 0)
+    g_tok = ((const float*)p.g)[((int64_t)b * p.L + min(tb + l, t_end - 1)) * p.g_h + kgate_head(p, p.g_h, h)];
+  Raw8<TIn> rq[4], rk[4];
+  float b_scalar;
   {
-    F3 kb0[4], kb1[4];
-    ld_ke(0, kb0);
-#pragma unroll 1
-    for (int m = 0; m < 8; m += 2) {
-      ld_ke(m + 1, kb1);
-      q_tile(m, kb0);
-      if (m + 2 < 8) ld_ke(m + 2, kb0);
-      q_tile(m + 1, kb1);
-    }
-  }
-  // (M U)^T tiles (rows = value, columns = token), the output kernel's layout
-  struct MOps {
-    F3 m[4];
-  };
-  auto ld_m = [&](int rt, MOps& o) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      if (s <= rt / 2) o.m[s] = SS::fa3(g_Mh + fofs(rt, s, l), g_Ml + fofs(rt, s, l));
-  };
-  auto oi_tile = [&](int rt, const MOps& o) {
-    f32x4 Oa[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) Oa[nt] = zero4();
+    const int t = tb + 16 * w + r16;
+    const int tt = t < t_end ? t : tb;
+    const TIn* qp = (const TIn*)p.q + (((int64_t)b * p.L + tt) * p.Hk + x0.hk) * KD;
+    const TIn* kp = (const TIn*)p.k + (((int64_t)b * p.L + tt) * p.Hk + x0.hk) * KD;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      if (s <= rt / 2) {
+      rq[s].load(qp + 32 * s, q);
+      rk[s].load(kp + 32 * s, q);
+    }
+    b_scalar = ((const float*)p.b)[((int64_t)b * p.L + tt) * p.b_h + kgate_head(p, p.b_h, h)];
+  }
+
+  // ---- Lambda: inclusive scan of g over the chunk (wave 0) -----------------
+  if (w == 0) {
+    sg.finish(p, x0, l, doc);
+    float gv = fminf(g_tok, 0.f);   // _nonpositive (NaN -> 0)
+    gv = fminf(gv, p.guard ? -1e-6f : 0.f);
+    float hi = (tb + l < t_end) ? gv : 0.f, lo = 0.f;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) P::m33(Oa[nt], U3[nt][s], o.m[s]);
+    for (int off = 1; off < 64; off <<= 1) {
+      const float h2 = __shfl_up(hi, off), l2 = __shfl_up(lo, off);
+      if (l >= off) {
+        // error-free hi + h2 (TwoSum), the rounding error joins the low words
+        const float sum = hi + h2;
+        const float bb = sum - hi;
+        lo += l2 + ((hi - (sum - bb)) + (h2 - bb));
+        hi = sum;
       }
     }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) *reinterpret_cast<f32x4*>(g_Oi + cofs(rt, ct0 + nt, p.nct, l)) = Oa[nt];
-  };
+    const float ph = hi * kLog2e;
+    lam_h[l] = ph;
+    lam_l[l] = fmaf(hi, kLog2e, -ph) + lo * kLog2e;
+  }
+  // ---- rows of token block w ------------------------------------------------
   {
-    MOps ma, mb;
-    ld_m(0, ma);
-#pragma unroll 1
-    for (int rt = 0; rt < 8; rt += 2) {
-      ld_m(rt + 1, mb);
-      oi_tile(rt, ma);
-      if (rt + 2 < 8) ld_m(rt + 2, ma);
-      oi_tile(rt + 1, mb);
+    const int i = 16 * w + r16;
+    const bool valid = tb + i < t_end;
+    float qv[32], kv[32], bet[32];
+    const Raw8<float> none[4] = {};
+    row_inputs<TIn>(p, rq, rk, none, b_scalar, valid, qv, kv, bet);
+    float bsc = b_scalar;
+    if (p.guard) bsc = fmaxf(bsc, 0.f);
+    if (q == 0) bet_s[i] = valid ? bsc : 0.f;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      // the normalised rows are bf16 values: their fragments are exact
+      const F1 fk = P::f1(kv + 8 * s), fq = P::f1(qv + 8 * s);
+      SS::stf(Kf + fofs(w, s, l), fk);
+      SS::stf(Qf + fofs(w, s, l), fq);
+      if (rows_out) {
+        SS::stf((bf16*)p.BeA + ku * (CH * KD) + fofs(w, s, l), fk);
+        SS::stf((bf16*)p.QeAh + ku * (CH * KD) + fofs(w, s, l), fq);
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+          f32x4 c = zero4();
+          mma(c, fk, ident_frag<true>(hf, r16, q));
+          const float x[4] = {c[0], c[1], c[2], c[3]};
+          SS::st4((bf16*)p.KeTh + ku * (CH * KD) + fofs2(2 * s + hf, w >> 1, l) + 4 * (w & 1), x);
+        }
+      }
     }
   }
+  lds_barrier();
+  // ---- row scalars: b e^Lambda, e^Lambda (first document), e^{Lend - Lambda} (last)
+  const float le_h = lam_h[CH - 1], le_l = lam_l[CH - 1];
+  if (w == 0) {
+    const bool first = doc[l] == 0, last = doc[l] == doc[CH - 1];
+    const float eL = first ? fast_exp2(lam_h[l] + lam_l[l]) : 0.f;                      // e^{Lambda_i} <= 1
+    const float eK = last ? fast_exp2((le_h - lam_h[l]) + (le_l - lam_l[l])) : 0.f;     // e^{Lambda_end - Lambda_i} <= 1
+    float* rs = p.rows + u * (3 * CH);
+    rs[l] = bet_s[l] * eL;
+    rs[CH + l] = eL;
+    rs[2 * CH + l] = eK;
+    if (l == 0) p.dvec[u * KD] = fast_exp2(le_h + le_l);   // e^{Lambda_end}
+  }
+  // ---- A and M tiles (a, bb), bb <= a: 10 tiles dealt round-robin ------------
+  bf16* g_Mh = (bf16*)p.MAh + u * TM;
+  bf16* g_Ml = (bf16*)p.MAl + u * TM;
+  for (int t = w; t < 10; t += 4) {
+    const int a = t >= 6 ? 3 : (t >= 3 ? 2 : (t >= 1 ? 1 : 0));
+    const int bb = t - a * (a + 1) / 2;
+    f32x4 gk = zero4(), gq = zero4();
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const F1 ka = SS::fa(Kf + fofs(a, s, l));
+      const F1 kb = SS::fa(Kf + fofs(bb, s, l));
+      const F1 qa = SS::fa(Qf + fofs(a, s, l));
+      mma(gk, ka, kb);   // (k k^T)[16a + 4q + ii][16bb + r16]
+      mma(gq, kb, qa);   // (q k^T)[16a + r16][16bb + 4q + ii]
+    }
+    float mv[4];
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) {
+      {
+        const int i = 16 * a + 4 * q + ii, j = 16 * bb + r16;
+        const float d = (lam_h[i] - lam_h[j]) + (lam_l[i] - lam_l[j]);
+        const bool on = i > j && doc[i] == doc[j];
+        X[i * AP + j] = on ? bet_s[i] * fast_exp2(fminf(d, 0.f)) * gk[ii] : 0.f;
+        if (bb == a && (a & 1) == 0) X[i * AP + j + 16] = 0.f;
+      }
+      {
+        const int i = 16 * a + r16, j = 16 * bb + 4 * q + ii;
+        const float d = (lam_h[i] - lam_h[j]) + (lam_l[i] - lam_l[j]);
+        const bool on = i >= j && doc[i] == doc[j];
+        mv[ii] = on ? fast_exp2(fminf(d, 0.f)) * gq[ii] : 0.f;
+      }
+    }
+    const int mo = tofs(a, bb >> 1, l) + 4 * (bb & 1);
+    SS::st4s(g_Mh + mo, g_Ml + mo, mv);
+    if (bb == a && (a & 1) == 0) {
+      const float z[4] = {0.f, 0.f, 0.f, 0.f};
+      SS::st4s(g_Mh + mo + 4, g_Ml + mo + 4, z);
+    }
+  }
+  lds_barrier();
+  invert_and_store<true>(X, reinterpret_cast<float*>(Kf), (bf16*)p.TAh + u * TM, (bf16*)p.TAl + u * TM, w, l);
 }
 
+// Output rows of one value head, written through a buffer resource that ends
+// with the last valid token's row: lanes past it are dropped by the hardware,
+// without a branch (a branch would leave the compiler unsure how many
+// vector-memory operations are pending, and the waits for prefetched operands
+// would then cover the stores too).
+template <class TV> struct OutRows {
+  TV* base;
+  int rowb, ofs;
+  __amdgpu_buffer_rsrc_t rs;
+  __device__ __forceinline__ OutRows(const PF& p, int b, int hv, int row, int col) {
+    base = (TV*)p.out + (((int64_t)b * p.L + p.t0) * p.Hv + hv) * KD;
+    rowb = p.Hv * KD * (int)sizeof(TV);
+    ofs = row * rowb + col * (int)sizeof(TV);
+  }
+  __device__ __forceinline__ void chunk(const PF& p, int c) {
+    const int rows = min(CH, min(p.nt, p.L - p.t0) - c * CH);   // >= 1
+    rs = __builtin_amdgcn_make_buffer_rsrc(base + (int64_t)c * CH * p.Hv * KD, (short)0,
+                                           (rows - 1) * rowb + KD * (int)sizeof(TV), 0x00020000);
+  }
+  // columns col + dc .. + 3
+  __device__ __forceinline__ void st(const f32x4& v, int dc) const {
+    if constexpr (sizeof(TV) == 4) {
+      typedef unsigned u4 __attribute__((ext_vector_type(4)));
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, ofs + dc * 4, 0, 0);
+    } else {
+      typedef unsigned u2 __attribute__((ext_vector_type(2)));
+      bf16x4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = (bf16)v[e];
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), rs, ofs + dc * 2, 0, 0);
+    }
+  }
+};
 
 // ===========================================================================
-// k_chain: S_{c+1} = [same doc] D_c S_c + Pn_c S_c + Q_c, and the output
-// O_c = X_c S_c + Oi_c of every chunk, for one 16-column value tile of one
-// exec head.  One workgroup of 8 waves in two roles that meet at one LDS
-// barrier per chunk:
+// k_chain: the scan over chunks for NTL 16-column value tiles of one exec
+// head, and each chunk's output.  One workgroup of 8 waves in two roles that
+// meet at three LDS barriers per chunk:
 //   waves 0-3 (recurrence): wave w owns state rows 32w..32w+31 (fp32, in
-//     VGPRs) and publishes them to LDS as slab w of the S_c^T fragment
-//     (split high / low bf16 in bf16 mode); after the barrier it reads the
-//     whole fragment and forms S_{c+1}: two independent chains of 4 MFMAs
-//     on the sequential path.
-//   waves 4-7 (output): wave 4 + t computes token tiles 2t and 2t + 1 of the
-//     chunk as O^T = S^T X^T + (M U)^T from the same fragments, beside the
-//     recurrence on the other wave slot of each SIMD.
-// A chunk step is short next to the latency of its operand loads, so each
-// role keeps several chunks of operands in flight in VGPRs (ChainSets: the
-// number of operand sets; a chunk's loads are issued that many steps minus
-// one ahead).  Two waves per SIMD leave each wave 256 VGPRs for them.
-// The role is a scalar (wave-uniform) branch, and both roles execute exactly
-// one barrier per chunk.  Loop trips run whole groups of chunks and the
-// remainder runs after the loop: an exit in the middle of a trip would make
-// the loop head wait for every outstanding load, the prefetches included.
+//     VGPRs) and publishes them to LDS as slab w of the S_c^T fragment (split
+//     high / low bf16 in bf16 mode); after barrier 1 it forms token tile w of
+//     be S and of R = w v - be S; after barrier 2 token tile w of Vn = T R;
+//     after barrier 3 its state rows' ke^T Vn.
+//   waves 4-7 (output): wave 4 + t computes token tile t of the chunk as
+//     O^T = S^T qe^T + Vn^T M^T, beside the recurrence on the other wave slot
+//     of each SIMD.
+// With SC (k_prepass_sc) be, qe and ke are row scalars times k, q and k:
+// be S = diag(b e^Lambda) (k S), and Vn is scaled before its product with k^T.
+// The scalars are applied in fp32, so only S and Vn enter as split words.
+// An operand's registers are loaded again for the next chunk as soon as their
+// product is issued, in the shadow of the LDS reads that follow a barrier, so
+// a load has most of a step to arrive and the loads are spread over the step
+// (the output role, which has registers to spare, keeps whole sets).
+// LDS fragments are read in bursts ahead of the products that use them.
+// The role is a scalar (wave-uniform) branch.
 // ===========================================================================
-// (one tile: 2 and 3 sets, config 2 chain 28.4-28.8 to 27.8 us and config 5
-// 1325-1336 to 1300-1304 us against 4 and 3; several tiles per workgroup: one
-// recurrence set, the registers two would hold spilled, config 3 chain
-// 492-502 to 434-438 us)
-template <bool BF, int NTL> struct ChainSets {
-  static constexpr int rec = NTL == 1 ? 2 : 1, out = NTL == 1 ? 3 : 2;
-};
-template <int NTL> struct ChainSets<false, NTL> {   // fp32 fragments are twice as wide
-  static constexpr int rec = 2, out = 3;
-};
 
 // NTL: 16-column tiles per workgroup.  One tile per workgroup spreads a
-// head's columns over the most CUs (config 2: 192 workgroups); when the tiles
-// outnumber the CUs, a workgroup takes NTL tiles of one value head, so each
-// chunk's Pn and X fragments are loaded once for all of them (the CU's load
-// rate bounds a step: one tile loads 112 KB per chunk, NTL tiles 48 + 64 NTL).
-template <bool BF, class TO, int NTL>
+// head's columns over the most CUs; when the tiles outnumber the CUs, a
+// workgroup takes NTL tiles of one value head, so each chunk's operands are
+// loaded once for all of them.  Index n of tile j is column NTL n + j of the
+// workgroup's 16 NTL: a lane's NTL values of one row are neighbours in memory.
+template <class T, int N> struct RowVec { typedef T V __attribute__((ext_vector_type(N))); };
+template <class T> struct RowVec<T, 1> { typedef T V; };
+template <class T, int N> __device__ __forceinline__ T row_el(const typename RowVec<T, N>::V& v, int j) {
+  if constexpr (N == 1) return v; else return v[j];
+}
+
+// products of a split operand pair over two accumulators: the leading one
+// and the corrections (independent chains; fp32: alternating by slab)
+template <bool BF, class A, class B>
+__device__ __forceinline__ void mma2(f32x4& c0, f32x4& c1, int s, const A& a, const B& b) {
+  using P = Pol<BF>;
+  if constexpr (!BF) {
+    P::m33(s & 1 ? c1 : c0, a, b);
+  } else if constexpr (std::is_same<A, typename P::F1>::value) {
+    mma(c0, a, b.hi);
+    mma(c1, a, b.lo);
+  } else if constexpr (std::is_same<B, typename P::F1>::value) {
+    mma(c0, a.hi, b);
+    mma(c1, a.lo, b);
+  } else {
+    mma(c0, a.hi, b.hi);
+    mma(c1, a.hi, b.lo);
+    mma(c1, a.lo, b.hi);
+  }
+}
+
+// (WCH: one write gate per value channel, not one per token -- a template
+// argument so that no branch stands between the loads of the loop)
+template <bool BF, bool SC, bool WCH, class TV, int NTL>
 __global__ __launch_bounds__(512) void k_chain(const PF p) {
   using P = Pol<BF>;
   using F1 = typename P::F1;
   using F3 = typename P::F3;
   using SS = Store<BF>;
   using ST = typename SS::ST;
+  using WV = typename RowVec<float, NTL>::V;
   constexpr int NT = 512;
-  constexpr int FR = 4 * 64 * 8;   // elements of one tile's S^T fragment
-  // S_c^T fragments of the NTL tiles, high and low words, double-buffered
-  __shared__ __align__(16) ST Sh_s[2][NTL][FR];
-  __shared__ __align__(16) ST Sl_s[2][NTL][BF ? FR : 1];
+  constexpr int FS = 4 * 64 * 8;   // elements of one tile's S^T fragment
+  constexpr int FV = 2 * 64 * 8;   // elements of one tile's R / Vn fragment
+  __shared__ __align__(16) ST Sh_s[NTL][FS], Sl_s[NTL][BF ? FS : 8];
+  __shared__ __align__(16) ST Rh_s[NTL][FV], Rl_s[NTL][BF ? FV : 8];
+  __shared__ __align__(16) ST Vh_s[NTL][FV], Vl_s[NTL][BF ? FV : 8];
+  __shared__ __align__(16) ST Kh_s[SC ? NTL : 1][SC ? FV : 8], Kl_s[SC ? NTL : 1][SC ? FV : 8];   // Vn e^{Lend - Lambda}
+  __shared__ __align__(16) float wv_s[4][NTL][64 * 4];   // w v: token tile, column tile, lane (index r16, tokens 4q..)
   __shared__ int flg[2 * kMaxBlockChunks];   // is_new_doc, all_same_doc per chunk
   const int tid = threadIdx.x;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1442,172 +1030,311 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
   xcd_block(ctg, h, b);
   const int ct0 = NTL * ctg;       // first tile; the NTL tiles lie in one value head
   const int hv = p.gates_at_hv ? h : h * p.G + (16 * ct0) / KD;
+  const int hk = p.gates_at_hv ? h / p.G : h;
   const int vc0 = (16 * ct0) % KD;   // first column of the tiles inside head hv
-  auto frag_lo = [&](int buf, int j) -> ST* { return BF ? &Sl_s[buf][j][0] : &Sh_s[buf][j][0]; };
+  const int t_end = min(p.t0 + p.nt, p.L);
   // chunk flags into LDS once, so testing them never waits on vector loads
   for (int i = tid; i < 2 * p.NCb; i += NT) flg[i] = p.flags[(int64_t)b * p.NCb * 2 + i];
-  __syncthreads();
+  // unit of chunk c (clamped to the last) for the per-head operands, and for
+  // the k / q operands that SC keeps once per key head
+  auto unit = [&](int c) { return ((int64_t)b * p.Hx + h) * p.NCb + min(c, p.NCb - 1); };
+  auto kunit = [&](int c) { return SC ? ((int64_t)b * p.Hk + hk) * p.NCb + min(c, p.NCb - 1) : unit(c); };
+  auto lo_p = [](ST* hi, ST* lo) { return BF ? lo : hi; };
+  auto ld_s = [&](int j, F3 (&f)[4]) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int o = (s * 64 + l) * 8;
+      f[s] = SS::fa3(&Sh_s[j][o], lo_p(&Sh_s[j][0], &Sl_s[j][0]) + o);
+    }
+  };
 
   if (wid < 4) {
     // ---------------- recurrence: state rows 32w.. ----------------
-    constexpr int RS = ChainSets<BF, NTL>::rec;
+    // (its dependent products set the step: first in line for the LDS and for
+    // load issue, config 2 chain 54.5 to 53.6 us)
+    __builtin_amdgcn_s_setprio(3);
     const int w = wid;
-    const int64_t sbase = ((int64_t)b * p.Hv + hv) * KD * KD + vc0 + r16;
+    const int64_t sbase = ((int64_t)b * p.Hv + hv) * KD * KD + vc0 + NTL * r16;
     f32x4 S[NTL][2];
 #pragma unroll
-    for (int j = 0; j < NTL; ++j)
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) {
+        WV x;
+        if (p.has_init) x = *reinterpret_cast<const WV*>(p.init + sbase + (int64_t)(32 * w + 16 * r + 4 * q + ii) * KD);
+        else x = WV{};
+#pragma unroll
+        for (int j = 0; j < NTL; ++j) S[j][r][ii] = row_el<float, NTL>(x, j);
+      }
+    using FK = std::conditional_t<SC, F1, F3>;
+    F1 be[4];            // be (SC: k) rows of token tile w
+    F3 tr[2];            // T rows of token tile w
+    FK kt[2][2];         // ke^T (SC: k^T) state row tiles 2w, 2w + 1
+    f32x4 dv[2];         // e^{Lend} of the state rows (SC: one value)
+    f32x4 bl, eK;        // SC: row scalars of tokens 16w + 4q + ii
+    // operands of chunk c's first product
+    auto load_a = [&](int c) {
+      const ST* bp = (const ST*)p.BeA + kunit(c) * (CH * KD);
+      if constexpr (SC) bl = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (3 * CH) + 16 * w + 4 * q);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) be[s] = SS::fa(bp + fofs(w, s, l));
+    };
+    auto load_t = [&](int c) {
+      const ST* th = (const ST*)p.TAh + unit(c) * TM;
+      const ST* tl = (const ST*)p.TAl + unit(c) * TM;
+      // (slab 1 of T's upper row tiles is all zero and not stored)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) tr[s] = SS::fa3(th + tofs(w, min(s, w >> 1), l), tl + tofs(w, min(s, w >> 1), l));
+      if constexpr (SC) eK = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (3 * CH) + 2 * CH + 16 * w + 4 * q);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        if constexpr (SC) dv[r] = f32x4{p.dvec[unit(c) * KD], 0.f, 0.f, 0.f};
+        else dv[r] = *reinterpret_cast<const f32x4*>(p.dvec + unit(c) * KD + 32 * w + 16 * r + 4 * q);
+      }
+    };
+    auto load_k = [&](int c) {
+      const ST* kh = (const ST*)p.KeTh + kunit(c) * (CH * KD);
+      const ST* kl = (const ST*)p.KeTl + kunit(c) * (CH * KD);
 #pragma unroll
       for (int r = 0; r < 2; ++r)
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii)
-          S[j][r][ii] = p.has_init ? p.init[sbase + 16 * j + (int64_t)(32 * w + 16 * r + 4 * q + ii) * KD] : 0.f;
-    struct Ops {
-      F1 pf[2][4];
-      f32x4 qc[NTL][2], dv[2];
+        for (int s = 0; s < 2; ++s) {
+          if constexpr (SC) kt[r][s] = SS::fa(kh + fofs2(2 * w + r, s, l));
+          else kt[r][s] = SS::fa3(kh + fofs2(2 * w + r, s, l), kl + fofs2(2 * w + r, s, l));
+        }
     };
-    auto load_ops = [&](int c, Ops& o) {
-      const int cc = min(c, p.NCb - 1);
-      const int64_t u = ((int64_t)b * p.Hx + h) * p.NCb + cc;
-      const ST* Pn = (const ST*)p.PnA + u * (KD * KD);
-      const float* Qc = p.QC + u * (int64_t)(KD * p.Vp);
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) o.pf[r][s] = SS::fa(Pn + fofs(2 * w + r, s, l));
-#pragma unroll
-        for (int j = 0; j < NTL; ++j) o.qc[j][r] = *reinterpret_cast<const f32x4*>(Qc + cofs(2 * w + r, ct0 + j, p.nct, l));
-        o.dv[r] = *reinterpret_cast<const f32x4*>(p.dvec + u * KD + 32 * w + 16 * r + 4 * q);
-      }
-    };
-    auto step = [&](int c, const Ops& o) {
-      const int is_new = flg[2 * c], same = flg[2 * c + 1];
-      const int fo = (w * 64 + l) * 8;
+    // a tile of R or Vn (lane: index r16, tokens 16w + 4q + ii) as half w & 1
+    // of slab w >> 1 of the fragment
+    const int vo = ((w >> 1) * 64 + l) * 8 + 4 * (w & 1);
+    const int fo = (w * 64 + l) * 8;
+    load_a(0);
+    load_t(0);
+    load_k(0);
+    lds_barrier();   // the flags and chunk 0's w v
+    int is_new = flg[0], same = flg[1];
+#pragma unroll 1
+    for (int c = 0; c < p.NCb; ++c) {
 #pragma unroll
       for (int j = 0; j < NTL; ++j) {
         if (is_new) { S[j][0] = zero4(); S[j][1] = zero4(); }
         // lane (n, q) holds rows 32w + 16r + 4q + ii = element 4r + ii of slab w
         const float x[8] = {S[j][0][0], S[j][0][1], S[j][0][2], S[j][0][3],
                             S[j][1][0], S[j][1][1], S[j][1][2], S[j][1][3]};
-        SS::st8s(&Sh_s[c & 1][j][fo], frag_lo(c & 1, j) + fo, x);
+        SS::st8s(&Sh_s[j][fo], lo_p(&Sh_s[j][0], &Sl_s[j][0]) + fo, x);
       }
-      lds_barrier();
+      lds_barrier();   // 1
+      F3 sf[2][4];
+      ld_s(0, sf[0]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int j = 0; j < NTL; ++j) {
-        F1 Sf[4];
+        if (j + 1 < NTL) {
+          ld_s(j + 1, sf[(j + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const f32x4 wv = *reinterpret_cast<const f32x4*>(&wv_s[w][j][4 * l]);
+        f32x4 acc = zero4(), acc2 = zero4();
 #pragma unroll
-        for (int s = 0; s < 4; ++s) Sf[s] = SS::fa(&Sh_s[c & 1][j][(s * 64 + l) * 8]);
+        for (int s = 0; s < 4; ++s) mma2<BF>(acc, acc2, s, be[s], sf[j & 1][s]);
+        float x[4];
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) {
+          const float ks = acc[ii] + acc2[ii];
+          x[ii] = SC ? fmaf(-bl[ii], ks, wv[ii]) : wv[ii] - ks;
+        }
+        SS::st4s(&Rh_s[j][vo], lo_p(&Rh_s[j][0], &Rl_s[j][0]) + vo, x);
+      }
+      lds_barrier();   // 2
+      F3 rf[NTL][2];
+      auto ld_rv = [&](ST* hi, ST* lo, F3 (&f)[2]) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) f[s] = SS::fa3(hi + (s * 64 + l) * 8, lo_p(hi, lo) + (s * 64 + l) * 8);
+      };
+#pragma unroll
+      for (int j = 0; j < NTL; ++j) ld_rv(Rh_s[j], Rl_s[j], rf[j]);
+      __builtin_amdgcn_sched_barrier(0);
+      load_a(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NTL; ++j) {
+        f32x4 acc = zero4(), acc2 = zero4();
+        mma2<BF>(acc, acc2, 0, tr[0], rf[j][0]);
+        if (w >= 2) mma2<BF>(acc, acc2, 1, tr[1], rf[j][1]);
+        float x[4];
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) x[ii] = acc[ii] + acc2[ii];
+        SS::st4s(&Vh_s[j][vo], lo_p(&Vh_s[j][0], &Vl_s[j][0]) + vo, x);
+        if constexpr (SC) {
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) x[ii] *= eK[ii];
+          SS::st4s(&Kh_s[j][vo], &Kl_s[j][vo], x);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) S[j][r][ii] = same ? dv[r][SC ? 0 : ii] * S[j][r][ii] : 0.f;
+      }
+      lds_barrier();   // 3
+#pragma unroll
+      for (int j = 0; j < NTL; ++j) {
+        if constexpr (SC) ld_rv(Kh_s[j], Kl_s[j], rf[j]);
+        else ld_rv(Vh_s[j], Vl_s[j], rf[j]);
+      }
+      const int cn = min(c + 1, p.NCb - 1);
+      is_new = flg[2 * cn];
+      same = flg[2 * cn + 1];
+      __builtin_amdgcn_sched_barrier(0);
+      load_t(c + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NTL; ++j)
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-          f32x4 acc = o.qc[j][r];
+          f32x4 acc2 = zero4();
 #pragma unroll
-          for (int s = 0; s < 4; ++s) P::m11(acc, o.pf[r][s], Sf[s]);
+          for (int s = 0; s < 2; ++s) mma2<BF>(S[j][r], acc2, s, kt[r][s], rf[j][s]);
 #pragma unroll
-          for (int ii = 0; ii < 4; ++ii) S[j][r][ii] = acc[ii] + (same ? o.dv[r][ii] * S[j][r][ii] : 0.f);
+          for (int ii = 0; ii < 4; ++ii) S[j][r][ii] += acc2[ii];
         }
-      }
-    };
-    Ops o[RS];
-#pragma unroll
-    for (int jj = 0; jj + 1 < RS; ++jj) load_ops(jj, o[jj]);
-    const int ntrip = p.NCb / RS;
-#pragma unroll 1
-    for (int k = 0; k < ntrip; ++k) {
-#pragma unroll
-      for (int jj = 0; jj < RS; ++jj) {
-        load_ops(RS * k + jj + RS - 1, o[(jj + RS - 1) % RS]);
-        step(RS * k + jj, o[jj]);
-      }
+      load_k(c + 1);
     }
-    const int rem = p.NCb - RS * ntrip;   // < RS; their operands are loaded
 #pragma unroll
-    for (int jj = 0; jj + 1 < RS; ++jj)
-      if (jj < rem) step(RS * ntrip + jj, o[jj]);
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-    for (int j = 0; j < NTL; ++j)
+      for (int ii = 0; ii < 4; ++ii) {
+        WV x;
 #pragma unroll
-      for (int r = 0; r < 2; ++r)
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) p.fin[sbase + 16 * j + (int64_t)(32 * w + 16 * r + 4 * q + ii) * KD] = S[j][r][ii];
+        for (int j = 0; j < NTL; ++j) {
+          if constexpr (NTL == 1) x = S[0][r][ii]; else x[j] = S[j][r][ii];
+        }
+        *reinterpret_cast<WV*>(p.fin + sbase + (int64_t)(32 * w + 16 * r + 4 * q + ii) * KD) = x;
+      }
   } else {
-    // ---------------- output: token tiles 2t, 2t + 1 ----------------
-    constexpr int OS = ChainSets<BF, NTL>::out;
-    const int t2 = 2 * (wid - 4);
-    struct Ops {
-      F3 xb[2][4];        // X fragments of the two token tiles (all NTL column tiles use them)
-      f32x4 oi[NTL][2];   // (M U)^T tiles of the two token tiles
-    };
-    auto load_ops = [&](int c, Ops& o) {
-      const int cc = min(c, p.NCb - 1);
-      const int64_t u = ((int64_t)b * p.Hx + h) * p.NCb + cc;
-      const ST* Xh = (const ST*)p.XAh + u * (CH * KD);
-      const ST* Xl = (const ST*)p.XAl + u * (CH * KD);
+    // ---------------- output: token tile t2, and w v for the recurrence ----------------
+    const int t2 = wid - 4;
+    // v and w of the chunk whose w v is formed next: lane = token 16 t2 + l / 4,
+    // columns 4 NTL (l % 4) .. + 4 NTL - 1 (index n of tile j is column NTL n + j)
+    const int hw = vgate_head(p, p.w_h, hv);
+    const int vt = 16 * t2 + (l >> 2), vcol = 4 * NTL * (l & 3);
+    const TV* vp = (const TV*)p.v + ((int64_t)b * p.L * p.Hv + hv) * KD + vc0;
+    const float* wp = (const float*)p.w + ((int64_t)b * p.L * p.w_h + hw) * p.w_c + (WCH ? vc0 : 0);
+    const uint32_t vs = (uint32_t)p.Hv * KD, ws = (uint32_t)p.w_h * p.w_c;
+    typedef TV V4 __attribute__((ext_vector_type(4)));
+    V4 v[NTL];
+    f32x4 wg[WCH ? NTL : 1];
+    auto load_v = [&](int c) {
+      const int t0 = p.t0 + min(c, p.NCb - 1) * CH;
+      const uint32_t row = min(vt, t_end - 1 - t0);   // rows past the last token read the last one
 #pragma unroll
-      for (int r = 0; r < 2; ++r) {
+      for (int j = 0; j < NTL; ++j) v[j] = *reinterpret_cast<const V4*>(vp + t0 * (int64_t)vs + (row * vs + vcol + 4 * j));
+      if constexpr (WCH) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) o.xb[r][s] = SS::fa3(Xh + fofs(t2 + r, s, l), Xl + fofs(t2 + r, s, l));
-#pragma unroll
-        for (int j = 0; j < NTL; ++j)
-          o.oi[j][r] = *reinterpret_cast<const f32x4*>(p.OiT + u * (int64_t)(CH * p.Vp) + cofs(t2 + r, ct0 + j, p.nct, l));
+        for (int j = 0; j < NTL; ++j) wg[j] = *reinterpret_cast<const f32x4*>(wp + t0 * (int64_t)ws + (row * ws + vcol + 4 * j));
+      } else {
+        wg[0][0] = (wp + t0 * (int64_t)ws)[row * ws];
       }
     };
-    f32x4 res[NTL][2];
-    auto step = [&](int c, const Ops& o) {
-      lds_barrier();
+    auto put_wv = [&](int c) {
+      const bool valid = vt <= t_end - 1 - (p.t0 + min(c, p.NCb - 1) * CH);
+      float y[4 * NTL];
 #pragma unroll
-      for (int j = 0; j < NTL; ++j) {
-        res[j][0] = o.oi[j][0];
-        res[j][1] = o.oi[j][1];
+      for (int e = 0; e < 4 * NTL; ++e) y[e] = WCH ? wg[e / 4][e % 4] : wg[0][0];
+      if (!SC && p.fuse) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const int fs = (s * 64 + l) * 8;
-          const F3 sf = SS::fa3(&Sh_s[c & 1][j][fs], frag_lo(c & 1, j) + fs);
-          P::m33(res[j][0], sf, o.xb[0][s]);
-          P::m33(res[j][1], sf, o.xb[1][s]);
-        }
+        for (int e = 0; e < 4 * NTL; ++e) y[e] = sigmoid_fast(y[e]);
+      }
+      // element (token 16 t2 + 4 q' + ii, index n) of a tile at word (16 q' + n) * 4 + ii
+      const int o = (l >> 4) * 64 + 16 * (l & 3) + ((l >> 2) & 3);
+#pragma unroll
+      for (int e = 0; e < 4 * NTL; ++e) {
+        const float x = y[e] * (float)v[e / 4][e % 4];
+        wv_s[t2][e % NTL][o + 4 * (e / NTL)] = valid ? x : 0.f;
       }
     };
-    // lane (t, q) holds O[token 16 (t2 + r) + t][column 16 (ct0 + j) + 4q + ii].
-    // Every lane stores (tokens past the end into the workspace's sink): a
-    // store skipped under a branch would leave the compiler unsure how many
-    // vector-memory operations are pending at the loop head, and it would
-    // then wait for all of them (the prefetches included).
-    auto store = [&](int c) {
+    // qe (SC: q) and M rows of the token tile, and e^Lambda of its token r16
+    // (SC): loaded again for the next chunk as soon as they are used
+    std::conditional_t<SC, F1, F3> qe[4];
+    F3 m[2];
+    float eL = 0.f;
+    auto load_q = [&](int c) {
+      const ST* qh = (const ST*)p.QeAh + kunit(c) * (CH * KD);
+      const ST* ql = (const ST*)p.QeAl + kunit(c) * (CH * KD);
 #pragma unroll
-      for (int j = 0; j < NTL; ++j) {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          const int t = p.t0 + c * CH + 16 * (t2 + r) + r16;
-          const bool tv = t < min(p.t0 + p.nt, p.L);
-          const int64_t ob = (((int64_t)b * p.L + (tv ? t : 0)) * p.Hv + hv) * KD + vc0 + 16 * j + 4 * q;
-          TO* dst = tv ? (TO*)p.out + ob : (TO*)p.sink + 4 * l;
-          const float x[4] = {res[j][r][0], res[j][r][1], res[j][r][2], res[j][r][3]};
-          st4<TO>(dst, x);
-        }
+      for (int s = 0; s < 4; ++s) {
+        if constexpr (SC) qe[s] = SS::fa(qh + fofs(t2, s, l));
+        else qe[s] = SS::fa3(qh + fofs(t2, s, l), ql + fofs(t2, s, l));
       }
+      if constexpr (SC) eL = p.rows[unit(c) * (3 * CH) + CH + 16 * t2 + r16];
     };
-    // Each chunk's prefetch is issued before its output store: the wait for
-    // a prefetched operand then never covers a store (the vector-memory
-    // counter counts stores too and drains in order).
-    Ops o[OS];
+    auto load_m = [&](int c) {
+      const ST* mh = (const ST*)p.MAh + unit(c) * TM;
+      const ST* ml = (const ST*)p.MAl + unit(c) * TM;
 #pragma unroll
-    for (int jj = 0; jj + 1 < OS; ++jj) load_ops(jj, o[jj]);
-    const int ntrip = p.NCb / OS;
+      for (int s = 0; s < 2; ++s) m[s] = SS::fa3(mh + tofs(t2, min(s, t2 >> 1), l), ml + tofs(t2, min(s, t2 >> 1), l));
+    };
+    // lane (t, q) holds O[token 16 t2 + t][columns NTL (4q + ii) + j]: 4 NTL
+    // neighbouring columns
+    OutRows<TV> orow(p, b, hv, 16 * t2 + r16, vc0 + 4 * NTL * q);
+    load_v(0);
+    load_q(0);
+    load_m(0);
+    put_wv(0);
+    load_v(1);
+    lds_barrier();   // the flags and chunk 0's w v
 #pragma unroll 1
-    for (int k = 0; k < ntrip; ++k) {
+    for (int c = 0; c < p.NCb; ++c) {
+      f32x4 res[NTL];
+      lds_barrier();   // 1
+      F3 sf[2][4];
+      ld_s(0, sf[0]);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int jj = 0; jj < OS; ++jj) {
-        step(OS * k + jj, o[jj]);
-        load_ops(OS * k + jj + OS - 1, o[(jj + OS - 1) % OS]);
-        store(OS * k + jj);
+      for (int j = 0; j < NTL; ++j) {
+        if (j + 1 < NTL) {
+          ld_s(j + 1, sf[(j + 1) & 1]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        f32x4 acc2 = zero4();
+        res[j] = zero4();
+#pragma unroll
+        for (int s = 0; s < 4; ++s) mma2<BF>(res[j], acc2, s, sf[j & 1][s], qe[s]);
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) res[j][ii] = SC ? (res[j][ii] + acc2[ii]) * eL : res[j][ii] + acc2[ii];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      load_q(c + 1);
+      lds_barrier();   // 2
+      put_wv(c + 1);   // (the recurrence has read chunk c's)
+      load_v(c + 2);
+      lds_barrier();   // 3
+      F3 vf[NTL][2];
+#pragma unroll
+      for (int j = 0; j < NTL; ++j)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const int fs = (s * 64 + l) * 8;
+          vf[j][s] = SS::fa3(&Vh_s[j][fs], lo_p(&Vh_s[j][0], &Vl_s[j][0]) + fs);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NTL; ++j) {
+        f32x4 acc2 = zero4();
+        mma2<BF>(res[j], acc2, 0, vf[j][0], m[0]);
+        if (t2 >= 2) mma2<BF>(res[j], acc2, 1, vf[j][1], m[1]);
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) res[j][ii] += acc2[ii];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      load_m(c + 1);
+      orow.chunk(p, c);
+#pragma unroll
+      for (int j4 = 0; j4 < NTL; ++j4) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = res[(4 * j4 + e) % NTL][(4 * j4 + e) / NTL];
+        orow.st(x, 4 * j4);
       }
     }
-    const int rem = p.NCb - OS * ntrip;
-#pragma unroll
-    for (int jj = 0; jj + 1 < OS; ++jj)
-      if (jj < rem) {
-        step(OS * ntrip + jj, o[jj]);
-        store(OS * ntrip + jj);
-      }
   }
 }
 
@@ -1617,34 +1344,35 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
 namespace {
 
 struct WsLayout {
-  size_t flags, dvec, PnA, QC, XAh, XAl, OiT, BeB, KeBh, KeBl, MAh, MAl, QeA, sink, carry, total;
+  size_t flags, dvec, rows, BeA, QeAh, QeAl, KeTh, KeTl, TAh, TAl, MAh, MAl, carry, total;
 };
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
-// Split operands (X, St, ke^T, M) have a low-word array in bf16 mode only.
-WsLayout ws_layout(const dn_prefill_args* a, int Hx, int Vp, int NCb, bool bf) {
+// Split operands have a low-word array in bf16 mode only.  With scalar gates
+// (sc) the k, q and k^T operands are kept once per key head, as single words.
+WsLayout ws_layout(const dn_prefill_args* a, int Hx, int NCb, bool sc) {
   WsLayout L{};
+  const bool bf = a->precision == 0;
   const size_t es = bf ? 2 : 4;
   const size_t ls = bf ? 2 : 0;
   const size_t units = (size_t)a->B * Hx * NCb;
-  const size_t sq = (size_t)CH * KD;   // elements of one 128 x 128 operand
+  const size_t kunits = sc ? (size_t)a->B * a->Hk * NCb : units;
+  const size_t sq = (size_t)CH * KD;
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
   L.flags = take((size_t)a->B * NCb * 2 * 4);
   L.dvec = take(units * KD * 4);
-  L.PnA = take(units * sq * es);
-  L.QC = take(units * KD * Vp * 4);
-  L.XAh = take(units * sq * es);
-  L.XAl = take(units * sq * ls);
-  L.OiT = take(units * CH * Vp * 4);
-  L.BeB = take(units * sq * es);
-  L.KeBh = take(units * sq * es);
-  L.KeBl = take(units * sq * ls);
-  L.MAh = take(units * sq * es);
-  L.MAl = take(units * sq * ls);
-  L.QeA = take(units * sq * 4);
-  L.sink = take(64 * 16);
+  L.rows = take(sc ? units * 3 * CH * 4 : 0);
+  L.BeA = take(kunits * sq * es);
+  L.QeAh = take(kunits * sq * es);
+  L.QeAl = take(sc ? 0 : kunits * sq * ls);
+  L.KeTh = take(kunits * sq * es);
+  L.KeTl = take(sc ? 0 : kunits * sq * ls);
+  L.TAh = take(units * TM * es);
+  L.TAl = take(units * TM * ls);
+  L.MAh = take(units * TM * es);
+  L.MAl = take(units * TM * ls);
   L.carry = take((size_t)a->B * a->Hv * KD * KD * 4);
   L.total = off;
   return L;
@@ -1657,20 +1385,20 @@ WsLayout ws_layout(const dn_prefill_args* a, int Hx, int Vp, int NCb, bool bf) {
 // launch each (4.15 ms against 5.47 ms); config 2 (147 MB) is unaffected.
 constexpr size_t kAutoBudget = size_t(4096) << 20;
 
-// Chunks per token block: block_tokens when given, else the most that keep
-// the workspace within kAutoBudget.  A hard budget (the allocation-free entry
-// point's scratch) also caps a given block_tokens.
-int block_chunks(const dn_prefill_args* a, int Hx, int Vp, size_t budget = 0) {
-  const int nct = (a->nt + CH - 1) / CH;
-  int ncb = std::min(nct, kMaxBlockChunks);
+// Chunks per token block (a whole number of 128-token blocks): block_tokens
+// when given, else the most that keep the workspace within kAutoBudget.  A
+// hard budget (the allocation-free entry point's scratch) also caps a given
+// block_tokens.
+int block_chunks(const dn_prefill_args* a, int Hx, bool sc, size_t budget = 0) {
+  constexpr int R = 128 / CH;
+  int n = std::min((a->nt + 127) / 128, kMaxBlockChunks / R);
   if (a->block_tokens > 0) {
-    ncb = std::max(1, std::min(ncb, a->block_tokens / CH));
-    if (budget == 0) return ncb;
+    n = std::max(1, std::min(n, a->block_tokens / 128));
+    if (budget == 0) return n * R;
   }
   if (budget == 0) budget = kAutoBudget;
-  const bool bf = a->precision == 0;
-  while (ncb > 1 && ws_layout(a, Hx, Vp, ncb, bf).total > budget) ncb = (ncb + 1) / 2;
-  return std::max(1, ncb);
+  while (n > 1 && ws_layout(a, Hx, n * R, sc).total > budget) n = (n + 1) / 2;
+  return n * R;
 }
 
 int check_args(const dn_prefill_args* a) {
@@ -1679,7 +1407,7 @@ int check_args(const dn_prefill_args* a) {
   if (a->K != KD || a->V != KD) return set_error(DN_E_INVALID, "K and V must both be 128");
   if (a->B <= 0 || a->L <= 0 || a->Hk <= 0 || a->Hv <= 0) return set_error(DN_E_INVALID, "non-positive dimension");
   if (a->Hv % a->Hk != 0) return set_error(DN_E_INVALID, "Hv must be a multiple of Hk");
-  if (a->t0 < 0 || a->t0 % CH != 0 || a->nt <= 0 || a->t0 + a->nt > a->L)
+  if (a->t0 < 0 || a->t0 % 128 != 0 || a->nt <= 0 || a->t0 + a->nt > a->L)
     return set_error(DN_E_INVALID, "token range must satisfy 0 <= t0 < t0+nt <= L with t0 % 128 == 0");
   if (!a->q || !a->k || !a->v || !a->g || !a->b || !a->w || !a->out)
     return set_error(DN_E_INVALID, "missing tensor pointer");
@@ -1698,7 +1426,7 @@ int check_args(const dn_prefill_args* a) {
     return set_error(DN_E_INVALID, "g or b has Hv heads: gates_at_hv must be set");
   if (a->seg && a->seg_dtype != DN_I32 && a->seg_dtype != DN_I64) return set_error(DN_E_INVALID, "segment ids must be int32 or int64");
   if (a->precision != 0 && a->precision != 1) return set_error(DN_E_INVALID, "precision must be 0 (bf16) or 1 (fp32)");
-  if (a->block_tokens < 0 || a->block_tokens % CH != 0) return set_error(DN_E_INVALID, "block_tokens must be a multiple of 128");
+  if (a->block_tokens < 0 || a->block_tokens % 128 != 0) return set_error(DN_E_INVALID, "block_tokens must be a multiple of 128");
   return DN_OK;
 }
 
@@ -1714,60 +1442,70 @@ int chain_tiles() {
 
 int g_prepass_scalar = -1;   // -1: unread; 0: general path forced (DN_PREPASS_SCALAR=0, measurements)
 
-// One decay and one b per (token, head) with bf16 q / k in precision "bf16"
-// (the Gated DeltaNet form) runs the scalar-gate prepass.
-bool scalar_gates(const PF& p) {
+// One decay, one b and one w per (token, head) with bf16 q / k in precision
+// "bf16" (the Gated DeltaNet form) runs the scalar-gate kernels.
+bool scalar_gates(const dn_prefill_args* a) {
   if (g_prepass_scalar < 0) {
     const char* e = getenv("DN_PREPASS_SCALAR");
     g_prepass_scalar = (e && atoi(e) == 0) ? 0 : 1;
   }
-  return g_prepass_scalar == 1 && p.g_c == 1 && p.b_c == 1 && !p.fuse;
+  return g_prepass_scalar == 1 && a->precision == 0 && a->qk_dtype == DN_BF16 && a->g_chans == 1 && a->b_chans == 1 &&
+         a->w_chans == 1 && !a->fuse_prologue;
 }
 
-template <bool BF, class TIn, class TV>
-hipError_t launch_all(const PF& p, hipStream_t st) {
-  prof_mark(0, st, false);
-  bool sc = false;
-  if constexpr (BF && std::is_same<TIn, bf16>::value) {
-    sc = scalar_gates(p);
-    if (sc) hipLaunchKernelGGL((k_prepass<BF, TIn, TV, true>), dim3(p.B * p.Hx * p.NCb), dim3(512), 0, st, p);
-  }
-  if (!sc) hipLaunchKernelGGL((k_prepass<BF, TIn, TV, false>), dim3(p.B * p.Hx * p.NCb), dim3(512), 0, st, p);
-  prof_mark(0, st, true);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  prof_mark(2, st, false);
+template <bool BF, bool SC, class TV>
+void launch_chain(const PF& p, hipStream_t st) {
   // several column tiles per workgroup once the tiles outnumber the CUs
   // (bf16 mode; config 3: 1024 tiles)
   const int tiles = (p.Vp / 16) * p.Hx * p.B;
-  int ntl = 1;
-  if constexpr (BF) {
-    ntl = chain_tiles();
-    if (ntl == 0) ntl = tiles >= 4 * 256 ? 4 : (tiles >= 2 * 256 ? 2 : 1);
-    if (ntl == 4)
-      hipLaunchKernelGGL((k_chain<BF, TV, 4>), dim3(p.Vp / 64, p.Hx, p.B), dim3(512), 0, st, p);
-    else if (ntl == 2)
-      hipLaunchKernelGGL((k_chain<BF, TV, 2>), dim3(p.Vp / 32, p.Hx, p.B), dim3(512), 0, st, p);
+  int ntl = chain_tiles();
+  if (ntl == 0) ntl = tiles > 2 * 256 ? 4 : (tiles > 256 ? 2 : 1);
+  if (!BF) ntl = 1;
+  const dim3 grid(p.Vp / (16 * ntl), p.Hx, p.B), blk(512);
+  auto go = [&](auto wch) {
+    constexpr bool W = decltype(wch)::value;
+    if constexpr (BF) {
+      if (ntl == 4) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 4>), grid, blk, 0, st, p);
+      else if (ntl == 2) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 2>), grid, blk, 0, st, p);
+    }
+    if (ntl == 1) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 1>), grid, blk, 0, st, p);
+  };
+  if constexpr (!SC) {
+    if (p.w_c != 1) go(std::true_type{});
+    else go(std::false_type{});
+  } else {
+    go(std::false_type{});
   }
-  if (ntl == 1) hipLaunchKernelGGL((k_chain<BF, TV, 1>), dim3(p.Vp / 16, p.Hx, p.B), dim3(512), 0, st, p);
+}
+
+template <bool BF, class TIn>
+hipError_t launch_all(const PF& p, hipStream_t st, bool v_bf16, bool sc) {
+  prof_mark(0, st, false);
+  if constexpr (BF && std::is_same<TIn, bf16>::value) {
+    if (sc) hipLaunchKernelGGL((k_prepass_sc<TIn>), dim3(p.B * p.Hx * p.NCb), dim3(256), 0, st, p);
+  }
+  if (!sc) hipLaunchKernelGGL((k_prepass<BF, TIn>), dim3(p.B * p.Hx * p.NCb), dim3(256), 0, st, p);
+  prof_mark(0, st, true);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  prof_mark(2, st, false);
+  if constexpr (BF && std::is_same<TIn, bf16>::value) {
+    if (sc) v_bf16 ? launch_chain<BF, true, bf16>(p, st) : launch_chain<BF, true, float>(p, st);
+  }
+  if (!sc) v_bf16 ? launch_chain<BF, false, bf16>(p, st) : launch_chain<BF, false, float>(p, st);
   prof_mark(2, st, true);
   return hipGetLastError();
 }
 
-template <bool BF, class TIn>
-hipError_t dispatch_v(const PF& p, hipStream_t st, bool v_bf16) {
-  return v_bf16 ? launch_all<BF, TIn, bf16>(p, st) : launch_all<BF, TIn, float>(p, st);
-}
-
 template <bool BF>
-hipError_t dispatch_qk(const PF& p, hipStream_t st, int qk_dt, bool v_bf16) {
-  if (qk_dt == DN_BF16) return dispatch_v<BF, bf16>(p, st, v_bf16);
-  if (qk_dt == DN_F16) return dispatch_v<BF, f16>(p, st, v_bf16);
-  return dispatch_v<BF, float>(p, st, v_bf16);
+hipError_t dispatch_qk(const PF& p, hipStream_t st, int qk_dt, bool v_bf16, bool sc) {
+  if (qk_dt == DN_BF16) return launch_all<BF, bf16>(p, st, v_bf16, sc);
+  if (qk_dt == DN_F16) return launch_all<BF, f16>(p, st, v_bf16, sc);
+  return launch_all<BF, float>(p, st, v_bf16, sc);
 }
 
-hipError_t dispatch(const PF& p, hipStream_t st, bool bf, int qk_dt, bool v_bf16) {
-  return bf ? dispatch_qk<true>(p, st, qk_dt, v_bf16) : dispatch_qk<false>(p, st, qk_dt, v_bf16);
+hipError_t dispatch(const PF& p, hipStream_t st, bool bf, int qk_dt, bool v_bf16, bool sc) {
+  return bf ? dispatch_qk<true>(p, st, qk_dt, v_bf16, sc) : dispatch_qk<false>(p, st, qk_dt, v_bf16, sc);
 }
 
 }  // namespace
@@ -1778,10 +1516,9 @@ using namespace dn;
 
 extern "C" size_t dn_prefill_workspace_size(const dn_prefill_args* a) {
   if (check_args(a) != DN_OK) return 0;
-  const int G = a->Hv / a->Hk;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  const int Vp = a->gates_at_hv ? KD : G * KD;
-  return ws_layout(a, Hx, Vp, block_chunks(a, Hx, Vp), a->precision == 0).total;
+  const bool sc = scalar_gates(a);
+  return ws_layout(a, Hx, block_chunks(a, Hx, sc), sc).total;
 }
 
 namespace {
@@ -1792,7 +1529,8 @@ int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int 
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
   const int Vp = a->gates_at_hv ? KD : G * KD;
   const bool bf = a->precision == 0;
-  const WsLayout Lw = ws_layout(a, Hx, Vp, ncb, bf);
+  const bool sc = scalar_gates(a);
+  const WsLayout Lw = ws_layout(a, Hx, ncb, sc);
   if (ws == nullptr || workspace_bytes < Lw.total) return set_error(DN_E_WORKSPACE, "workspace too small");
 
   PF p{};
@@ -1808,19 +1546,16 @@ int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int 
   p.scale = a->scale; p.l2norm = a->qk_l2norm; p.fuse = a->fuse_prologue; p.guard = a->stability_guard;
   p.flags = (int32_t*)(ws + Lw.flags);
   p.dvec = (float*)(ws + Lw.dvec);
-  p.nct = Vp / 16;
-  p.PnA = ws + Lw.PnA;
-  p.QC = (float*)(ws + Lw.QC);
-  p.XAh = ws + Lw.XAh;
-  p.XAl = bf ? ws + Lw.XAl : p.XAh;
-  p.OiT = (float*)(ws + Lw.OiT);
-  p.BeB = ws + Lw.BeB;
-  p.KeBh = ws + Lw.KeBh;
-  p.KeBl = bf ? ws + Lw.KeBl : p.KeBh;
+  p.rows = (float*)(ws + Lw.rows);
+  p.BeA = ws + Lw.BeA;
+  p.QeAh = ws + Lw.QeAh;
+  p.QeAl = bf ? ws + Lw.QeAl : p.QeAh;
+  p.KeTh = ws + Lw.KeTh;
+  p.KeTl = bf ? ws + Lw.KeTl : p.KeTh;
+  p.TAh = ws + Lw.TAh;
+  p.TAl = bf ? ws + Lw.TAl : p.TAh;
   p.MAh = ws + Lw.MAh;
   p.MAl = bf ? ws + Lw.MAl : p.MAh;
-  p.QeA = (float*)(ws + Lw.QeA);
-  p.sink = ws + Lw.sink;
   float* carry = a->final_state ? a->final_state : (float*)(ws + Lw.carry);
 
   const int t_stop = a->t0 + a->nt;
@@ -1832,7 +1567,7 @@ int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int 
     p.has_init = first ? (a->init_state != nullptr) : 1;
     p.init = first ? a->init_state : carry;
     p.fin = carry;
-    const hipError_t e = dispatch(p, st, bf, a->qk_dtype, a->v_dtype == DN_BF16);
+    const hipError_t e = dispatch(p, st, bf, a->qk_dtype, a->v_dtype == DN_BF16, sc);
     if (e != hipSuccess) return set_error(DN_E_LAUNCH, hipGetErrorString(e));
   }
   return DN_OK;
@@ -1853,8 +1588,7 @@ extern "C" int dn_prefill_fwd(const dn_prefill_args* a, void* workspace, size_t 
   const int rc = prefill_shape_ok(a);
   if (rc != DN_OK) return rc;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  const int Vp = a->gates_at_hv ? KD : (a->Hv / a->Hk) * KD;
-  return prefill_run(a, (char*)workspace, workspace_bytes, block_chunks(a, Hx, Vp), (hipStream_t)stream);
+  return prefill_run(a, (char*)workspace, workspace_bytes, block_chunks(a, Hx, scalar_gates(a)), (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1900,11 +1634,11 @@ extern "C" int dn_prefill_fwd_noalloc(const dn_prefill_args* a, void* stream) {
   const int rc = prefill_shape_ok(a);
   if (rc != DN_OK) return rc;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  const int Vp = a->gates_at_hv ? KD : (a->Hv / a->Hk) * KD;
-  const int ncb = block_chunks(a, Hx, Vp, DN_NOALLOC_SCRATCH_BYTES);
-  if (ws_layout(a, Hx, Vp, ncb, a->precision == 0).total > DN_NOALLOC_SCRATCH_BYTES)
+  const bool sc = scalar_gates(a);
+  const int ncb = block_chunks(a, Hx, sc, DN_NOALLOC_SCRATCH_BYTES);
+  if (ws_layout(a, Hx, ncb, sc).total > DN_NOALLOC_SCRATCH_BYTES)
     return set_error(DN_E_WORKSPACE,
-                     "dn_prefill_fwd_noalloc: one 128-token chunk of every (batch, head) needs more than "
+                     "dn_prefill_fwd_noalloc: one 128-token block of every (batch, head) needs more than "
                      "DN_NOALLOC_SCRATCH_BYTES of scratch; use dn_prefill_fwd with a workspace");
   char* ws = scratch_address();
   if (ws == nullptr) return DN_E_LAUNCH;
