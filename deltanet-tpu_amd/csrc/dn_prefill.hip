@@ -32,108 +32,15 @@
 
 #include "dn_common.h"
 #include "dn_host.h"
+#include "dn_prefill.h"
 
 namespace dn {
 
 constexpr int CH = 64;    // chunk size (the reference's 128 is a TPU tile size; the recurrence is the same)
 constexpr int NB = CH / 16;   // 16-token blocks of a chunk
-constexpr int KD = 128;   // key / value head dim (gdn2.py:1897)
 constexpr int XP = 132;   // fp32 LDS pitch (floats) of the Lambda rows: conflict-free 16-lane column groups
 constexpr int AP = 68;    // fp32 LDS pitch of A and T
 constexpr int kMaxBlockChunks = 1024;   // chunks per token block (chain's LDS flag table)
-
-// diag blocks whose in-block log2-decay span exceeds this use the
-// overflow-free hierarchical path (e^{69} stays far inside the fp32 range)
-constexpr float kDiagSafeLog2 = 100.f;
-
-// ---------------------------------------------------------------------------
-// gate activations (gdn2.py:38-47, 133-142, 1970-1974): g = -exp(min(g, 5)),
-// b, w = sigmoid.  The sigmoid uses the hardware reciprocal (v_rcp_f32, 1 ulp):
-// 1 + e^{-x} >= 1, and an infinite denominator gives exactly 0.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ float sigmoid_fast(float x) { return __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
-
-// head of a K-side gate (g, b) used by execution head h
-__device__ __forceinline__ int kgate_head(const PF& p, int H, int h) {
-  if (H == 1) return 0;
-  if (p.gates_at_hv) return (H == p.Hv) ? h : h / p.G;
-  return h;
-}
-// head of a value-side gate (w) used by value head hv
-__device__ __forceinline__ int vgate_head(const PF& p, int H, int hv) {
-  if (H == 1) return 0;
-  return (H == p.Hv) ? hv : hv / p.G;
-}
-
-// A segment id as two 32-bit words loaded without a branch, so the loads can
-// be issued early (the value is only compared for equality).  int32 ids read
-// their word twice.
-// A segment id as its two 32-bit words; an int32 id repeats its one word in
-// hi (no select on the loaded value, so nothing waits for the load until the
-// ids are compared; equality is unchanged)
-struct SegId {
-  int32_t lo, hi;
-  __device__ __forceinline__ bool operator!=(const SegId& o) const { return lo != o.lo || hi != o.hi; }
-};
-__device__ __forceinline__ SegId seg_raw(const PF& p, int b, int t) {
-  const int64_t i = p.seg_batched ? (int64_t)b * p.L + t : (int64_t)t;
-  const bool w64 = p.seg_dt == DT_I64;
-  const int32_t* s32 = (const int32_t*)p.seg + (w64 ? 2 * i : i);
-  return SegId{s32[0], s32[w64 ? 1 : 0]};
-}
-
-// q, k and b * k of one token row in fragment order (slab s: elements
-// 8s..8s+7), after the prologue: L2 normalisation (gdn2.py:1990-1996, the
-// normalised q and k rounded back to the input type), the q scale, the b
-// activation or clamp, and zeros for tokens past the end.
-template <class TIn>
-__device__ __forceinline__ void row_inputs(const PF& p, const Raw8<TIn> (&rq)[4], const Raw8<TIn> (&rk)[4],
-                                           const Raw8<float> (&rb)[4], float b_scalar, bool valid, float (&qv)[32],
-                                           float (&kv)[32], float (&bet)[32]) {
-#pragma unroll
-  for (int s = 0; s < 4; ++s) {
-    rq[s].to(qv + 8 * s);
-    rk[s].to(kv + 8 * s);
-  }
-  if (p.b_c == 1) {
-#pragma unroll
-    for (int e = 0; e < 32; ++e) bet[e] = b_scalar;
-  } else {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) rb[s].to(bet + 8 * s);
-  }
-  float ssq = 0.f, ssk = 0.f;
-#pragma unroll
-  for (int e = 0; e < 32; ++e) { ssq += qv[e] * qv[e]; ssk += kv[e] * kv[e]; }
-  ssq += __shfl_xor(ssq, 16); ssq += __shfl_xor(ssq, 32);
-  ssk += __shfl_xor(ssk, 16); ssk += __shfl_xor(ssk, 32);
-  if (p.fuse) {
-    const float rq = rsqrtf(ssq + 1e-6f) , rk = rsqrtf(ssk + 1e-6f);
-#pragma unroll
-    for (int e = 0; e < 32; ++e) {
-      qv[e] = (qv[e] * rq) * p.scale;
-      kv[e] = kv[e] * rk;
-      bet[e] = sigmoid_fast(bet[e]);
-    }
-  } else if (p.l2norm) {
-    const float rq = rsqrtf(ssq + 1e-6f), rk = rsqrtf(ssk + 1e-6f);
-#pragma unroll
-    for (int e = 0; e < 32; ++e) { qv[e] = round_as<TIn>((qv[e] * rq) * p.scale); kv[e] = round_as<TIn>(kv[e] * rk); }
-  } else {
-#pragma unroll
-    for (int e = 0; e < 32; ++e) qv[e] = round_as<TIn>(qv[e] * p.scale);
-  }
-  if (p.guard && !p.fuse) {
-#pragma unroll
-    for (int e = 0; e < 32; ++e) bet[e] = fmaxf(bet[e], 0.f);
-  }
-#pragma unroll
-  for (int e = 0; e < 32; ++e) {
-    qv[e] = valid ? qv[e] : 0.f;
-    kv[e] = valid ? kv[e] : 0.f;
-    bet[e] = valid ? bet[e] * kv[e] : 0.f;
-  }
-}
 
 // a 16 x 32 slab of an operand with two slabs per tile (reduction over the
 // chunk's 64 tokens)
@@ -1344,16 +1251,22 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
 namespace {
 
 struct WsLayout {
-  size_t flags, dvec, rows, BeA, QeAh, QeAl, KeTh, KeTl, TAh, TAl, MAh, MAl, carry, total;
+  size_t flags, dvec, rows, BeA, QeAh, QeAl, KeTh, KeTl, TAh, TAl, MAh, MAl, lng, carry, total;
 };
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+// How a call is run: chunks of 64 tokens with their operands applied in the
+// scan (kScan, with scalar gates kScalar), or the 128-token affine form of
+// dn_prefill_long.hip.
+enum Form { kScan, kScalar, kLong };
+int chunk_of(Form f) { return f == kLong ? 128 : CH; }
+
 // Split operands have a low-word array in bf16 mode only.  With scalar gates
-// (sc) the k, q and k^T operands are kept once per key head, as single words.
-WsLayout ws_layout(const dn_prefill_args* a, int Hx, int NCb, bool sc) {
+// the k, q and k^T operands are kept once per key head, as single words.
+WsLayout ws_layout(const dn_prefill_args* a, int Hx, int Vp, int NCb, Form form) {
   WsLayout L{};
-  const bool bf = a->precision == 0;
+  const bool bf = a->precision == 0, sc = form == kScalar;
   const size_t es = bf ? 2 : 4;
   const size_t ls = bf ? 2 : 0;
   const size_t units = (size_t)a->B * Hx * NCb;
@@ -1363,16 +1276,20 @@ WsLayout ws_layout(const dn_prefill_args* a, int Hx, int NCb, bool sc) {
   auto take = [&](size_t bytes) { size_t o = off; off += align256(bytes); return o; };
   L.flags = take((size_t)a->B * NCb * 2 * 4);
   L.dvec = take(units * KD * 4);
-  L.rows = take(sc ? units * 3 * CH * 4 : 0);
-  L.BeA = take(kunits * sq * es);
-  L.QeAh = take(kunits * sq * es);
-  L.QeAl = take(sc ? 0 : kunits * sq * ls);
-  L.KeTh = take(kunits * sq * es);
-  L.KeTl = take(sc ? 0 : kunits * sq * ls);
-  L.TAh = take(units * TM * es);
-  L.TAl = take(units * TM * ls);
-  L.MAh = take(units * TM * es);
-  L.MAl = take(units * TM * ls);
+  if (form == kLong) {
+    L.lng = take(long_workspace(units, Vp, bf));
+  } else {
+    L.rows = take(sc ? units * 3 * CH * 4 : 0);
+    L.BeA = take(kunits * sq * es);
+    L.QeAh = take(kunits * sq * es);
+    L.QeAl = take(sc ? 0 : kunits * sq * ls);
+    L.KeTh = take(kunits * sq * es);
+    L.KeTl = take(sc ? 0 : kunits * sq * ls);
+    L.TAh = take(units * TM * es);
+    L.TAl = take(units * TM * ls);
+    L.MAh = take(units * TM * es);
+    L.MAl = take(units * TM * ls);
+  }
   L.carry = take((size_t)a->B * a->Hv * KD * KD * 4);
   L.total = off;
   return L;
@@ -1385,20 +1302,19 @@ WsLayout ws_layout(const dn_prefill_args* a, int Hx, int NCb, bool sc) {
 // launch each (4.15 ms against 5.47 ms); config 2 (147 MB) is unaffected.
 constexpr size_t kAutoBudget = size_t(4096) << 20;
 
-// Chunks per token block (a whole number of 128-token blocks): block_tokens
-// when given, else the most that keep the workspace within kAutoBudget.  A
-// hard budget (the allocation-free entry point's scratch) also caps a given
-// block_tokens.
-int block_chunks(const dn_prefill_args* a, int Hx, bool sc, size_t budget = 0) {
-  constexpr int R = 128 / CH;
+// 128-token blocks per token block: block_tokens when given, else the most
+// that keep the workspace within kAutoBudget.  A hard budget (the
+// allocation-free entry point's scratch) also caps a given block_tokens.
+int block_128s(const dn_prefill_args* a, int Hx, int Vp, Form form, size_t budget = 0) {
+  const int R = 128 / chunk_of(form);
   int n = std::min((a->nt + 127) / 128, kMaxBlockChunks / R);
   if (a->block_tokens > 0) {
     n = std::max(1, std::min(n, a->block_tokens / 128));
-    if (budget == 0) return n * R;
+    if (budget == 0) return n;
   }
   if (budget == 0) budget = kAutoBudget;
-  while (n > 1 && ws_layout(a, Hx, n * R, sc).total > budget) n = (n + 1) / 2;
-  return n * R;
+  while (n > 1 && ws_layout(a, Hx, Vp, n * R, form).total > budget) n = (n + 1) / 2;
+  return n;
 }
 
 int check_args(const dn_prefill_args* a) {
@@ -1451,6 +1367,26 @@ bool scalar_gates(const dn_prefill_args* a) {
   }
   return g_prepass_scalar == 1 && a->precision == 0 && a->qk_dtype == DN_BF16 && a->g_chans == 1 && a->b_chans == 1 &&
          a->w_chans == 1 && !a->fuse_prologue;
+}
+
+// The long form where its scan, half the steps at 1.4 us against 1.3 us each,
+// outweighs its prepass, whose cost grows with the heads H and, less, with the
+// value heads G of each: `width` = H (5 + 2 G).  Measured (64-token scan / long
+// form, us): width 9-36, 2048 tokens 65 / 77, 4096 104 / 97, 16384 350 / 230;
+// width 72, 4096 tokens 112 / 115, 16384 638 / 536; width 104-112, 4096 tokens
+// 120-149 / 180-190, 16384 650-755 / 637-733; width 224, 16384 tokens
+// 965 / 1191; fp32 width 9-36, 2048 tokens 123 / 163, 16384 800 / 525.  With
+// scalar gates the scan's prepass is the smaller by far: width 14, 4096 tokens
+// 92 / 97, 16384 316 / 290.
+Form form_of(const dn_prefill_args* a) {
+  const bool sc = scalar_gates(a);
+  const int64_t G = a->gates_at_hv ? 1 : a->Hv / a->Hk;
+  const int64_t width = (int64_t)a->B * (a->gates_at_hv ? a->Hv : a->Hk) * (5 + 2 * G);
+  int64_t least = INT64_MAX;   // tokens from which the long form is the faster
+  if (sc) least = width <= 28 ? 8192 : INT64_MAX;
+  else least = width <= 40 ? 3072 : (width <= 75 ? 8192 : (width <= 115 ? 16384 : INT64_MAX));
+  if (a->nt >= least) return kLong;
+  return sc ? kScalar : kScan;
 }
 
 template <bool BF, bool SC, class TV>
@@ -1517,20 +1453,21 @@ using namespace dn;
 extern "C" size_t dn_prefill_workspace_size(const dn_prefill_args* a) {
   if (check_args(a) != DN_OK) return 0;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  const bool sc = scalar_gates(a);
-  return ws_layout(a, Hx, block_chunks(a, Hx, sc), sc).total;
+  const int Vp = a->gates_at_hv ? KD : (a->Hv / a->Hk) * KD;
+  const Form form = form_of(a);
+  return ws_layout(a, Hx, Vp, block_128s(a, Hx, Vp, form) * (128 / chunk_of(form)), form).total;
 }
 
 namespace {
 
-// One dn_prefill_fwd call in token blocks of ncb chunks over the workspace ws.
-int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int ncb, hipStream_t st) {
+// One dn_prefill_fwd call in token blocks of n 128-token blocks over the workspace ws.
+int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int n, Form form, hipStream_t st) {
   const int G = a->Hv / a->Hk;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
   const int Vp = a->gates_at_hv ? KD : G * KD;
   const bool bf = a->precision == 0;
-  const bool sc = scalar_gates(a);
-  const WsLayout Lw = ws_layout(a, Hx, ncb, sc);
+  const int ch = chunk_of(form);
+  const WsLayout Lw = ws_layout(a, Hx, Vp, n * (128 / ch), form);
   if (ws == nullptr || workspace_bytes < Lw.total) return set_error(DN_E_WORKSPACE, "workspace too small");
 
   PF p{};
@@ -1559,15 +1496,17 @@ int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int 
   float* carry = a->final_state ? a->final_state : (float*)(ws + Lw.carry);
 
   const int t_stop = a->t0 + a->nt;
-  for (int tb = a->t0; tb < t_stop; tb += ncb * CH) {
+  for (int tb = a->t0; tb < t_stop; tb += n * 128) {
     p.t0 = tb;
-    p.nt = std::min(ncb * CH, t_stop - tb);
-    p.NCb = (p.nt + CH - 1) / CH;
+    p.nt = std::min(n * 128, t_stop - tb);
+    p.NCb = (p.nt + ch - 1) / ch;
     const bool first = tb == a->t0;
     p.has_init = first ? (a->init_state != nullptr) : 1;
     p.init = first ? a->init_state : carry;
     p.fin = carry;
-    const hipError_t e = dispatch(p, st, bf, a->qk_dtype, a->v_dtype == DN_BF16, sc);
+    const bool v_bf16 = a->v_dtype == DN_BF16;
+    const hipError_t e = form == kLong ? long_prefill(p, ws + Lw.lng, st, bf, a->qk_dtype, v_bf16)
+                                       : dispatch(p, st, bf, a->qk_dtype, v_bf16, form == kScalar);
     if (e != hipSuccess) return set_error(DN_E_LAUNCH, hipGetErrorString(e));
   }
   return DN_OK;
@@ -1588,7 +1527,9 @@ extern "C" int dn_prefill_fwd(const dn_prefill_args* a, void* workspace, size_t 
   const int rc = prefill_shape_ok(a);
   if (rc != DN_OK) return rc;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  return prefill_run(a, (char*)workspace, workspace_bytes, block_chunks(a, Hx, scalar_gates(a)), (hipStream_t)stream);
+  const int Vp = a->gates_at_hv ? KD : (a->Hv / a->Hk) * KD;
+  const Form form = form_of(a);
+  return prefill_run(a, (char*)workspace, workspace_bytes, block_128s(a, Hx, Vp, form), form, (hipStream_t)stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1634,13 +1575,14 @@ extern "C" int dn_prefill_fwd_noalloc(const dn_prefill_args* a, void* stream) {
   const int rc = prefill_shape_ok(a);
   if (rc != DN_OK) return rc;
   const int Hx = a->gates_at_hv ? a->Hv : a->Hk;
-  const bool sc = scalar_gates(a);
-  const int ncb = block_chunks(a, Hx, sc, DN_NOALLOC_SCRATCH_BYTES);
-  if (ws_layout(a, Hx, ncb, sc).total > DN_NOALLOC_SCRATCH_BYTES)
+  const int Vp = a->gates_at_hv ? KD : (a->Hv / a->Hk) * KD;
+  const Form form = form_of(a);
+  const int n = block_128s(a, Hx, Vp, form, DN_NOALLOC_SCRATCH_BYTES);
+  if (ws_layout(a, Hx, Vp, n * (128 / chunk_of(form)), form).total > DN_NOALLOC_SCRATCH_BYTES)
     return set_error(DN_E_WORKSPACE,
                      "dn_prefill_fwd_noalloc: one 128-token block of every (batch, head) needs more than "
                      "DN_NOALLOC_SCRATCH_BYTES of scratch; use dn_prefill_fwd with a workspace");
   char* ws = scratch_address();
   if (ws == nullptr) return DN_E_LAUNCH;
-  return prefill_run(a, ws, DN_NOALLOC_SCRATCH_BYTES, ncb, (hipStream_t)stream);
+  return prefill_run(a, ws, DN_NOALLOC_SCRATCH_BYTES, n, form, (hipStream_t)stream);
 }
