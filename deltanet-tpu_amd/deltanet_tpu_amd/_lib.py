@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 
 LIB_NAME = "libdeltanet_amd.so"
@@ -66,6 +67,12 @@ class DecodeArgs(ctypes.Structure):
     ]
 
 
+# ``DecodeArgs`` in one call: the same fields in the same order and native
+# alignment (one ctypes field assignment costs about as much as packing six
+# fields).
+DECODE_PACK = struct.Struct("@6i3P2iP3iP3iP3iPiPiPPf2if0P").pack
+
+
 class BackwardArgs(ctypes.Structure):
     """Mirror of ``dn_backward_args``."""
 
@@ -103,6 +110,21 @@ PROFILE_KINDS = ("prepass", "value", "chain", "decode", "backward")
 
 _lock = threading.Lock()
 _lib = None
+_packed = None
+
+
+def packed_decode():
+    """``dn_decode_step`` and ``dn_decode_steps`` of the loaded library, taking
+    the argument block as packed bytes."""
+    global _packed
+    if _packed is None:
+        load_library()
+        lib = ctypes.CDLL(LIB_PATH)   # the same library; function objects of its own
+        one, many = lib.dn_decode_step, lib.dn_decode_steps
+        one.argtypes, one.restype = [ctypes.c_char_p, _c_ptr], ctypes.c_int
+        many.argtypes, many.restype = [ctypes.c_char_p, _c_i32, _c_ptr], ctypes.c_int
+        _packed = one, many
+    return _packed
 
 
 def load_library(path: str | None = None) -> ctypes.CDLL:
