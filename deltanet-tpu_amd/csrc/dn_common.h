@@ -185,13 +185,22 @@ template <> struct Pol<true> {
   using F1 = Frag<true>;
   struct F3 { Frag<true> hi, lo; };
   static __device__ __forceinline__ F1 f1(const float* x) { return make_frag<true>(x); }
+  // (converted in pairs: one instruction rounds two values, and the high words
+  // widen again by a shift and a mask of the pair)
   static __device__ __forceinline__ F3 f3(const float* x) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef bf16 b2 __attribute__((ext_vector_type(2)));
     F3 r;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bf16 h = (bf16)x[e];
-      r.hi.v[e] = h;
-      r.lo.v[e] = (bf16)(x[e] - (float)h);
+    for (int e = 0; e < 8; e += 2) {
+      const b2 h = __builtin_convertvector((f2{x[e], x[e + 1]}), b2);
+      const uint32_t u = __builtin_bit_cast(uint32_t, h);
+      const b2 l = __builtin_convertvector((f2{x[e] - __builtin_bit_cast(float, u << 16),
+                                               x[e + 1] - __builtin_bit_cast(float, u & 0xffff0000u)}), b2);
+      r.hi.v[e] = h[0];
+      r.hi.v[e + 1] = h[1];
+      r.lo.v[e] = l[0];
+      r.lo.v[e + 1] = l[1];
     }
     return r;
   }

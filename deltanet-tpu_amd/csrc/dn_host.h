@@ -28,7 +28,7 @@ struct PF {
   // workspace arrays (one unit = one (batch, exec head, chunk))
   int32_t* flags;            // [B][NCb][2] : is_new_doc, all_same_doc
   float* dvec;               // [unit][K]    : e^{Lambda_end}
-  float* rows;               // [unit][3][64]: b e^Lambda, e^Lambda, e^{Lend - Lambda} per token (scalar gates)
+  float* rows;               // [unit][4][64]: b e^Lambda, e^Lambda, e^{Lend - Lambda}, e^{Lend} per token (scalar gates)
   // Workspace, per unit = (batch, exec head, chunk).  Every operand array is
   // fragment-native for its consumer ([tile][slab][lane][8] elements of a
   // 16 x 32 MFMA operand slab).  Split operands have a high and a low array

@@ -774,11 +774,11 @@ __global__ __launch_bounds__(256, 3) void k_prepass_sc(const PF p) {
     const bool first = doc[l] == 0, last = doc[l] == doc[CH - 1];
     const float eL = first ? fast_exp2(lam_h[l] + lam_l[l]) : 0.f;                      // e^{Lambda_i} <= 1
     const float eK = last ? fast_exp2((le_h - lam_h[l]) + (le_l - lam_l[l])) : 0.f;     // e^{Lambda_end - Lambda_i} <= 1
-    float* rs = p.rows + u * (3 * CH);
+    float* rs = p.rows + u * (4 * CH);
     rs[l] = bet_s[l] * eL;
     rs[CH + l] = eL;
     rs[2 * CH + l] = eK;
-    if (l == 0) p.dvec[u * KD] = fast_exp2(le_h + le_l);   // e^{Lambda_end}
+    rs[3 * CH + l] = fast_exp2(le_h + le_l);   // e^{Lambda_end}
   }
   // ---- A and M tiles (a, bb), bb <= a: 10 tiles dealt round-robin ------------
   bf16* g_Mh = (bf16*)p.MAh + u * TM;
@@ -842,17 +842,17 @@ template <class TV> struct OutRows {
     rs = __builtin_amdgcn_make_buffer_rsrc(base + (int64_t)c * CH * p.Hv * KD, (short)0,
                                            (rows - 1) * rowb + KD * (int)sizeof(TV), 0x00020000);
   }
-  // columns col + dc .. + 3
-  __device__ __forceinline__ void st(const f32x4& v, int dc) const {
+  // columns col + dc .. + 3 of row + dr
+  __device__ __forceinline__ void st(const f32x4& v, int dc, int dr = 0) const {
     if constexpr (sizeof(TV) == 4) {
       typedef unsigned u4 __attribute__((ext_vector_type(4)));
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, ofs + dc * 4, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, v), rs, ofs + dr * rowb + dc * 4, 0, 0);
     } else {
       typedef unsigned u2 __attribute__((ext_vector_type(2)));
       bf16x4 x;
 #pragma unroll
       for (int e = 0; e < 4; ++e) x[e] = (bf16)v[e];
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), rs, ofs + dc * 2, 0, 0);
+      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, x), rs, ofs + dr * rowb + dc * 2, 0, 0);
     }
   }
 };
@@ -958,7 +958,7 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
   if (wid < 4) {
     // ---------------- recurrence: state rows 32w.. ----------------
     // (its dependent products set the step: first in line for the LDS and for
-    // load issue, config 2 chain 54.5 to 53.6 us)
+    // load issue: 2048 tokens, 16 value heads 54.5 to 53.6 us)
     __builtin_amdgcn_s_setprio(3);
     const int w = wid;
     const int64_t sbase = ((int64_t)b * p.Hv + hv) * KD * KD + vc0 + NTL * r16;
@@ -982,7 +982,7 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
     // operands of chunk c's first product
     auto load_a = [&](int c) {
       const ST* bp = (const ST*)p.BeA + kunit(c) * (CH * KD);
-      if constexpr (SC) bl = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (3 * CH) + 16 * w + 4 * q);
+      if constexpr (SC) bl = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (4 * CH) + 16 * w + 4 * q);
 #pragma unroll
       for (int s = 0; s < 4; ++s) be[s] = SS::fa(bp + fofs(w, s, l));
     };
@@ -992,10 +992,10 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
       // (slab 1 of T's upper row tiles is all zero and not stored)
 #pragma unroll
       for (int s = 0; s < 2; ++s) tr[s] = SS::fa3(th + tofs(w, min(s, w >> 1), l), tl + tofs(w, min(s, w >> 1), l));
-      if constexpr (SC) eK = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (3 * CH) + 2 * CH + 16 * w + 4 * q);
+      if constexpr (SC) eK = *reinterpret_cast<const f32x4*>(p.rows + unit(c) * (4 * CH) + 2 * CH + 16 * w + 4 * q);
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
-        if constexpr (SC) dv[r] = f32x4{p.dvec[unit(c) * KD], 0.f, 0.f, 0.f};
+        if constexpr (SC) dv[r] = f32x4{p.rows[unit(c) * (4 * CH) + 3 * CH], 0.f, 0.f, 0.f};
         else dv[r] = *reinterpret_cast<const f32x4*>(p.dvec + unit(c) * KD + 32 * w + 16 * r + 4 * q);
       }
     };
@@ -1171,7 +1171,7 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
         if constexpr (SC) qe[s] = SS::fa(qh + fofs(t2, s, l));
         else qe[s] = SS::fa3(qh + fofs(t2, s, l), ql + fofs(t2, s, l));
       }
-      if constexpr (SC) eL = p.rows[unit(c) * (3 * CH) + CH + 16 * t2 + r16];
+      if constexpr (SC) eL = p.rows[unit(c) * (4 * CH) + CH + 16 * t2 + r16];
     };
     auto load_m = [&](int c) {
       const ST* mh = (const ST*)p.MAh + unit(c) * TM;
@@ -1246,6 +1246,272 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
 }
 
 // ===========================================================================
+// k_chain_cols: the scalar-gate scan for 64 columns of one exec head per
+// workgroup.  Wave j < 4 owns column tile j with the whole state (128 rows, 32
+// VGPRs): a tile's S, R and Vn never leave its registers (an accumulator tile
+// pair is the next product's fragment), so a step has no exchange between
+// waves and one barrier, where the split by state rows (k_chain) meets three
+// times and sends S, R and Vn of every tile through LDS to all eight waves.
+// Waves 4-7 copy the operands all four tiles share (k, T, k^T, q, M: 72 KB per
+// chunk, fragment-native, 1 KB per instruction and no registers) from the
+// workspace into the other half of a double buffer, one chunk ahead.
+// Bound by the LDS reads of those operands (84 KB per wave and chunk) beside
+// 132 MFMAs per wave.  chunk_gdn, 4 x 8192 tokens, 32 value heads, bf16: 434 us
+// with the rows split, 400 us here (3.1 us a chunk against 1 us of MFMA issue);
+// with every read waited for in turn, the compiler's order, 435 us.
+// ===========================================================================
+template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// 64 lanes x 16 bytes from src (each lane's own address) to 1 KB of LDS at dst
+__device__ __forceinline__ void copy_to_lds(const void* src, void* dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+
+__global__ __launch_bounds__(512) void k_chain_cols(const PF p) {
+  using P = Pol<true>;
+  using F1 = P::F1;
+  using F3 = P::F3;
+  using SS = Store<true>;
+  constexpr int OK = 0, OT = CH * KD, OKT = OT + 2 * TM, OQ = OKT + CH * KD, OM = OQ + CH * KD, ON = OM + 2 * TM;
+  __shared__ __align__(16) bf16 ops[2][ON];
+  __shared__ __align__(16) float row_s[2][4 * CH];   // b e^Lambda, e^Lambda, e^{Lend - Lambda}, e^{Lend}
+  __shared__ __align__(16) float w_s[2][CH];         // write gate per token
+  __shared__ uint8_t flg[kMaxBlockChunks];           // bit 0: is_new_doc, bit 1: all_same_doc
+  const int tid = threadIdx.x;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l = tid & 63, r16 = l & 15, q = l >> 4;
+  int ctg, h, b;
+  xcd_block(ctg, h, b);
+  const int hv = p.gates_at_hv ? h : h * p.G + (64 * ctg) / KD;
+  const int hk = p.gates_at_hv ? h / p.G : h;
+  const int NCb = p.NCb, t_end = min(p.t0 + p.nt, p.L);
+  auto unit = [&](int c) { return ((int64_t)b * p.Hx + h) * NCb + min(c, NCb - 1); };
+
+  if (wid >= 4) {
+    // ---------------- loaders: fragment 4 i + w of each operand by wave w ----------------
+    const int w = wid - 4;
+    const float* wp = (const float*)p.w + (int64_t)b * p.L * p.w_h + vgate_head(p, p.w_h, hv);
+    auto copy = [&](const bf16* src, bf16* dst, int n) {
+      for (int i = w; i < n; i += 4) copy_to_lds(src + i * 512 + l * 8, dst + i * 512);
+    };
+    auto load = [&](int c) {
+      const int64_t u = unit(c), ku = ((int64_t)b * p.Hk + hk) * NCb + min(c, NCb - 1);
+      bf16* o = ops[c & 1];
+      copy((const bf16*)p.BeA + ku * (CH * KD), o + OK, 16);
+      copy((const bf16*)p.TAh + u * TM, o + OT, 6);
+      copy((const bf16*)p.TAl + u * TM, o + OT + TM, 6);
+      copy((const bf16*)p.KeTh + ku * (CH * KD), o + OKT, 16);
+      copy((const bf16*)p.QeAh + ku * (CH * KD), o + OQ, 16);
+      copy((const bf16*)p.MAh + u * TM, o + OM, 6);
+      copy((const bf16*)p.MAl + u * TM, o + OM + TM, 6);
+      if (w == 3) copy_to_lds(p.rows + u * (4 * CH) + l * 4, row_s[c & 1]);
+      // (tokens past the last one read its gate)
+      const int t0 = p.t0 + min(c, NCb - 1) * CH;
+      if (w == 2)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp + min(t0 + l, t_end - 1) * (int64_t)p.w_h),
+                                         (__attribute__((address_space(3))) void*)w_s[c & 1], 4, 0, 0);
+    };
+    load(0);
+    if (NCb > 1) load(1);
+    for (int i = tid - 256; i < NCb; i += 256) {
+      const int32_t* f = p.flags + ((int64_t)b * NCb + i) * 2;
+      flg[i] = (f[0] ? 1 : 0) | (f[1] ? 2 : 0);
+    }
+    wait_vm<0>();
+    lds_barrier();   // chunks 0 and 1, the flags
+#pragma unroll 1
+    for (int c = 0; c < NCb; ++c) {
+      wait_vm<0>();   // chunk c + 1 is there
+      lds_barrier();  // chunk c is read
+      if (c + 2 < NCb) load(c + 2);
+    }
+  } else {
+    // ---------------- column tile j = wid ----------------
+    const int vc0 = (64 * ctg) % KD + 16 * wid;   // first column of the tile inside head hv
+    const int64_t sbase = ((int64_t)b * p.Hv + hv) * KD * KD + vc0 + r16;
+    f32x4 S[8];   // lane (n, q): column n, state rows 16m + 4q + ii
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) S[m][ii] = p.has_init ? p.init[sbase + (int64_t)(16 * m + 4 * q + ii) * KD] : 0.f;
+    OutRows<bf16> orow(p, b, hv, r16, vc0 + 4 * q);
+    // v of (token 16rt + 4q + ii, this lane's column) of the next chunk, zero
+    // past the last token (the resource ends with its row)
+    const bf16* vb = (const bf16*)p.v + (((int64_t)b * p.L + p.t0) * p.Hv + hv) * KD;
+    const int rowb = p.Hv * KD * 2, vofs = 4 * q * rowb + (vc0 + r16) * 2;
+    uint16_t v[4][4];
+    auto load_v = [&](int c) {
+      const int cc = min(c, NCb - 1), rows = min(CH, t_end - (p.t0 + cc * CH));
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(vb) + (int64_t)cc * CH * p.Hv * KD, (short)0,
+                                                        (rows - 1) * rowb + KD * 2, 0x00020000);
+#pragma unroll
+      for (int rt = 0; rt < NB; ++rt)
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) v[rt][ii] = __builtin_amdgcn_raw_buffer_load_b16(rs, vofs, (16 * rt + ii) * rowb, 0);
+    };
+    load_v(0);
+    lds_barrier();   // chunks 0 and 1, the flags
+#pragma unroll 1
+    for (int c = 0; c < NCb; ++c) {
+      const bf16* o = ops[c & 1];
+      const float* rw = row_s[c & 1];
+      const int f = __builtin_amdgcn_readfirstlane(flg[c]);
+      const float* ws = w_s[c & 1];
+      if (f & 1) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) S[m] = zero4();
+      }
+      F3 sf[4];   // S^T fragments: slab s = state rows 32s..
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const float x[8] = {S[2 * s][0], S[2 * s][1], S[2 * s][2], S[2 * s][3],
+                            S[2 * s + 1][0], S[2 * s + 1][1], S[2 * s + 1][2], S[2 * s + 1][3]};
+        sf[s] = P::f3(x);
+      }
+      // The shared operands go through three buffers of four fragments, each
+      // read two groups of products ahead of its use (the compiler's own order
+      // waits for every read: 3.4 us a chunk).
+      F1 fa[4], fb[4], fc[4];
+      auto ld = [&](F1 (&f)[4], int o0, int o1, int o2, int o3) {
+        f[0] = SS::fa(o + o0);
+        f[1] = SS::fa(o + o1);
+        f[2] = SS::fa(o + o2);
+        f[3] = SS::fa(o + o3);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto ld_k = [&](F1 (&f)[4], int rt) { ld(f, OK + fofs(rt, 0, l), OK + fofs(rt, 1, l), OK + fofs(rt, 2, l), OK + fofs(rt, 3, l)); };
+      auto ld_q = [&](F1 (&f)[4], int rt) { ld(f, OQ + fofs(rt, 0, l), OQ + fofs(rt, 1, l), OQ + fofs(rt, 2, l), OQ + fofs(rt, 3, l)); };
+      // rows 0 and 1 of a triangular operand (one slab each), or row rt >= 2 (two slabs): high, low
+      auto ld_01 = [&](F1 (&f)[4], int b0) { ld(f, b0 + tofs(0, 0, l), b0 + TM + tofs(0, 0, l), b0 + tofs(1, 0, l), b0 + TM + tofs(1, 0, l)); };
+      auto ld_rt = [&](F1 (&f)[4], int b0, int rt) { ld(f, b0 + tofs(rt, 0, l), b0 + TM + tofs(rt, 0, l), b0 + tofs(rt, 1, l), b0 + TM + tofs(rt, 1, l)); };
+      auto ld_kt = [&](F1 (&f)[4], int m) { ld(f, OKT + fofs2(m, 0, l), OKT + fofs2(m, 1, l), OKT + fofs2(m + 1, 0, l), OKT + fofs2(m + 1, 1, l)); };
+      auto done = [] { __builtin_amdgcn_sched_barrier(0); };
+
+      f32x4 R[4];
+      // R[rt] = w v - b e^Lambda (k S)
+      auto prod_k = [&](int rt, const F1 (&f)[4]) {
+        const f32x4 ww = *reinterpret_cast<const f32x4*>(&ws[16 * rt + 4 * q]);
+        const f32x4 bl = *reinterpret_cast<const f32x4*>(&rw[16 * rt + 4 * q]);
+        f32x4 a = zero4(), a2 = zero4();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) mma2<true>(a, a2, t, f[t], sf[t]);
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) R[rt][ii] = fmaf(-bl[ii], a[ii] + a2[ii], ww[ii] * __builtin_bit_cast(float, (uint32_t)v[rt][ii] << 16));
+        done();
+      };
+      auto frag = [&](const f32x4& x0, const f32x4& x1) {
+        const float x[8] = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
+        return P::f3(x);
+      };
+      F3 rf[2], vf[2], kf[2];
+      // Vn = T R, and Vn e^{Lend - Lambda}
+      f32x4 Vt[2], Kt[2];
+      auto prod_t = [&](int rt, const F1& h0, const F1& l0, const F1& h1, const F1& l1) {
+        const f32x4 eK = *reinterpret_cast<const f32x4*>(&rw[2 * CH + 16 * rt + 4 * q]);
+        f32x4 a = zero4(), a2 = zero4();
+        mma2<true>(a, a2, 0, F3{h0, l0}, rf[0]);
+        if (rt >= 2) mma2<true>(a, a2, 1, F3{h1, l1}, rf[1]);
+        Vt[rt & 1] = a + a2;
+        Kt[rt & 1] = Vt[rt & 1] * eK;
+        if (rt & 1) {
+          vf[rt >> 1] = frag(Vt[0], Vt[1]);
+          kf[rt >> 1] = frag(Kt[0], Kt[1]);
+        }
+      };
+      // S = [same doc] e^{Lend} S + k^T (Vn e^{Lend - Lambda})
+      const float dv = (f & 2) ? rw[3 * CH] : 0.f;
+      if (!(f & 2)) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) S[m] = zero4();   // (sf holds this chunk's; 0 * inf is not 0)
+      }
+      // (two rows of tiles at a time: their chains interleave)
+      auto prod_kt = [&](int m, const F1 (&x)[4]) {
+        f32x4 a = dv * S[m], b = dv * S[m + 1];
+        mma(a, x[0], kf[0].hi);
+        mma(b, x[2], kf[0].hi);
+        mma(a, x[0], kf[0].lo);
+        mma(b, x[2], kf[0].lo);
+        mma(a, x[1], kf[1].hi);
+        mma(b, x[3], kf[1].hi);
+        mma(a, x[1], kf[1].lo);
+        mma(b, x[3], kf[1].lo);
+        S[m] = a;
+        S[m + 1] = b;
+        done();
+      };
+      // O^T = e^Lambda (S^T q^T) + Vn^T M^T: lane (t, q) holds token 16rt + t,
+      // columns 4q + ii of the tile
+      f32x4 O[4];
+      auto prod_q = [&](int rt, const F1 (&f)[4]) {
+        const float eL = rw[CH + 16 * rt + r16];
+        f32x4 a = zero4(), a2 = zero4();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) mma2<true>(a, a2, t, sf[t], f[t]);
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) O[rt][ii] = (a[ii] + a2[ii]) * eL;
+        done();
+      };
+      auto prod_m = [&](int rt, const F1& h0, const F1& l0, const F1& h1, const F1& l1) {
+        f32x4 a2 = zero4();
+        mma2<true>(O[rt], a2, 0, vf[0], F3{h0, l0});
+        if (rt >= 2) mma2<true>(O[rt], a2, 1, vf[1], F3{h1, l1});
+        orow.st(O[rt] + a2, 0, 16 * rt);
+      };
+      orow.chunk(p, c);
+      ld_k(fa, 0);
+      ld_k(fb, 1);
+      ld_k(fc, 2);
+      prod_k(0, fa);
+      ld_k(fa, 3);
+      prod_k(1, fb);
+      ld_01(fb, OT);
+      rf[0] = frag(R[0], R[1]);
+      prod_k(2, fc);
+      ld_rt(fc, OT, 2);
+      prod_k(3, fa);
+      load_v(c + 1);
+      ld_rt(fa, OT, 3);
+      rf[1] = frag(R[2], R[3]);
+      prod_t(0, fb[0], fb[1], fb[0], fb[1]);
+      prod_t(1, fb[2], fb[3], fb[2], fb[3]);
+      done();
+      ld_q(fb, 0);
+      prod_t(2, fc[0], fc[1], fc[2], fc[3]);
+      done();
+      ld_kt(fc, 0);
+      prod_t(3, fa[0], fa[1], fa[2], fa[3]);
+      done();
+      ld_kt(fa, 2);
+      prod_q(0, fb);   // (fills the latency of Vn's last tile)
+      ld_kt(fb, 4);
+      prod_kt(0, fc);
+      ld_kt(fc, 6);
+      prod_kt(2, fa);
+      ld_q(fa, 1);
+      prod_kt(4, fb);
+      ld_q(fb, 2);
+      prod_kt(6, fc);
+      ld_q(fc, 3);
+      prod_q(1, fa);
+      ld_01(fa, OM);
+      prod_q(2, fb);
+      ld_rt(fb, OM, 2);
+      prod_q(3, fc);
+      ld_rt(fc, OM, 3);
+      prod_m(0, fa[0], fa[1], fa[0], fa[1]);
+      prod_m(1, fa[2], fa[3], fa[2], fa[3]);
+      prod_m(2, fb[0], fb[1], fb[2], fb[3]);
+      prod_m(3, fc[0], fc[1], fc[2], fc[3]);
+      lds_barrier();   // chunk c is read
+    }
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) p.fin[sbase + (int64_t)(16 * m + 4 * q + ii) * KD] = S[m][ii];
+  }
+}
+
+// ===========================================================================
 // host side
 // ===========================================================================
 namespace {
@@ -1279,7 +1545,7 @@ WsLayout ws_layout(const dn_prefill_args* a, int Hx, int Vp, int NCb, Form form)
   if (form == kLong) {
     L.lng = take(long_workspace(units, Vp, bf));
   } else {
-    L.rows = take(sc ? units * 3 * CH * 4 : 0);
+    L.rows = take(sc ? units * 4 * CH * 4 : 0);
     L.BeA = take(kunits * sq * es);
     L.QeAh = take(kunits * sq * es);
     L.QeAl = take(sc ? 0 : kunits * sq * ls);
@@ -1296,10 +1562,10 @@ WsLayout ws_layout(const dn_prefill_args* a, int Hx, int Vp, int NCb, Form form)
 }
 
 // Workspace budget of one call (token blocks beyond it run one after another).
-// Larger blocks mean fewer launches and longer chains per launch: at BASELINE
-// config 3 (8192 units) a 4 GiB budget measured 2.64 ms per call against
-// 2.91 ms at 160 MiB, and config 5's 8192-token streaming blocks run in one
-// launch each (4.15 ms against 5.47 ms); config 2 (147 MB) is unaffected.
+// Larger blocks mean fewer launches and longer chains per launch: chunk_gdn of 4
+// sequences of 8192 tokens (32 value heads) runs in one launch pair, and so does
+// each 8192-token block of a streamed sequence; with the 128-token form a 160 MiB
+// budget cost 10% and 32% there, and smaller budgets cost with this one too.
 constexpr size_t kAutoBudget = size_t(4096) << 20;
 
 // 128-token blocks per token block: block_tokens when given, else the most
@@ -1391,13 +1657,19 @@ Form form_of(const dn_prefill_args* a) {
 
 template <bool BF, bool SC, class TV>
 void launch_chain(const PF& p, hipStream_t st) {
-  // several column tiles per workgroup once the tiles outnumber the CUs
-  // (bf16 mode; config 3: 1024 tiles)
+  // several column tiles per workgroup once the tiles outnumber the CUs: with
+  // scalar gates at four, each wave its own (k_chain_cols)
   const int tiles = (p.Vp / 16) * p.Hx * p.B;
   int ntl = chain_tiles();
   if (ntl == 0) ntl = tiles > 2 * 256 ? 4 : (tiles > 256 ? 2 : 1);
   if (!BF) ntl = 1;
   const dim3 grid(p.Vp / (16 * ntl), p.Hx, p.B), blk(512);
+  if constexpr (SC && std::is_same<TV, bf16>::value) {
+    if (ntl == 4) {
+      hipLaunchKernelGGL(k_chain_cols, grid, blk, 0, st, p);
+      return;
+    }
+  }
   auto go = [&](auto wch) {
     constexpr bool W = decltype(wch)::value;
     if constexpr (BF) {
