@@ -172,11 +172,7 @@ __device__ __forceinline__ void op_put4(bool bf, float* arr, int i, int c, int n
     bf16* b = reinterpret_cast<bf16*>(arr) + bofs(i, c, ns);
     const float x[4] = {v.x, v.y, v.z, v.w};
     bf16x4 h, lo;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[e] = (bf16)x[e];
-      lo[e] = (bf16)(x[e] - (float)h[e]);
-    }
+    split_bf16<4>(x, h, lo);
     *reinterpret_cast<bf16x4*>(b) = h;
     *reinterpret_cast<bf16x4*>(b + 512) = lo;
   } else {
@@ -189,11 +185,7 @@ __device__ __forceinline__ void op_put8(bool bf, float* arr, int i, int c, int n
   if (bf) {
     bf16* b = reinterpret_cast<bf16*>(arr) + bofs(i, c, ns);
     bf16x8 h, lo;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      h[e] = (bf16)x[e];
-      lo[e] = (bf16)(x[e] - (float)h[e]);
-    }
+    split_bf16<8>(x, h, lo);
     *reinterpret_cast<bf16x8*>(b) = h;
     *reinterpret_cast<bf16x8*>(b + 512) = lo;
   } else {
@@ -849,22 +841,15 @@ template <int CT> struct ChainLds<true, CT> {
   bf16x4 Y[2][CT][2][64][2];
   __device__ __forceinline__ void put_s(int j, int wv, int l, const f32x4& s0, const f32x4& s1) {
     bf16x8 h, lo;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = e < 4 ? s0[e] : s1[e - 4];
-      h[e] = (bf16)x;
-      lo[e] = (bf16)(x - (float)h[e]);
-    }
+    const float x[8] = {s0[0], s0[1], s0[2], s0[3], s1[0], s1[1], s1[2], s1[3]};
+    split_bf16<8>(x, h, lo);
     S[0][j][wv][l] = h;
     S[1][j][wv][l] = lo;
   }
   __device__ __forceinline__ void put_y(int j, int wv, int l, const f32x4& y) {
     bf16x4 h, lo;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[e] = (bf16)y[e];
-      lo[e] = (bf16)(y[e] - (float)h[e]);
-    }
+    const float x[4] = {y[0], y[1], y[2], y[3]};
+    split_bf16<4>(x, h, lo);
     Y[0][j][wv >> 1][l][wv & 1] = h;
     Y[1][j][wv >> 1][l][wv & 1] = lo;
   }
@@ -1107,11 +1092,7 @@ template <int W> struct LMat<true, W> {
   __device__ __forceinline__ void put4(int r, int c, float4 v) {
     const float x[4] = {v.x, v.y, v.z, v.w};
     bf16x4 hh, ll;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      hh[e] = (bf16)x[e];
-      ll[e] = (bf16)(x[e] - (float)hh[e]);
-    }
+    split_bf16<4>(x, hh, ll);
     *reinterpret_cast<bf16x4*>(&h[r][c]) = hh;
     *reinterpret_cast<bf16x4*>(&lw[r][c]) = ll;
   }

@@ -181,27 +181,32 @@ __device__ __forceinline__ void lds_barrier() {
 // ---------------------------------------------------------------------------
 template <bool BF> struct Pol;
 
+// x = hi + lo in bf16, each rounded to nearest.  Converted in pairs: one
+// instruction rounds two values, and the high words widen again by a shift and
+// a mask of the pair, where value by value the compiler re-packs each half.
+template <int N, typename V>
+__device__ __forceinline__ void split_bf16(const float* x, V& hi, V& lo) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef bf16 b2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int e = 0; e < N; e += 2) {
+    const b2 h = __builtin_convertvector((f2{x[e], x[e + 1]}), b2);
+    const uint32_t u = __builtin_bit_cast(uint32_t, h);
+    const b2 l = __builtin_convertvector((f2{x[e] - __builtin_bit_cast(float, u << 16),
+                                             x[e + 1] - __builtin_bit_cast(float, u & 0xffff0000u)}), b2);
+    hi[e] = h[0];
+    hi[e + 1] = h[1];
+    lo[e] = l[0];
+    lo[e + 1] = l[1];
+  }
+}
 template <> struct Pol<true> {
   using F1 = Frag<true>;
   struct F3 { Frag<true> hi, lo; };
   static __device__ __forceinline__ F1 f1(const float* x) { return make_frag<true>(x); }
-  // (converted in pairs: one instruction rounds two values, and the high words
-  // widen again by a shift and a mask of the pair)
   static __device__ __forceinline__ F3 f3(const float* x) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    typedef bf16 b2 __attribute__((ext_vector_type(2)));
     F3 r;
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const b2 h = __builtin_convertvector((f2{x[e], x[e + 1]}), b2);
-      const uint32_t u = __builtin_bit_cast(uint32_t, h);
-      const b2 l = __builtin_convertvector((f2{x[e] - __builtin_bit_cast(float, u << 16),
-                                               x[e + 1] - __builtin_bit_cast(float, u & 0xffff0000u)}), b2);
-      r.hi.v[e] = h[0];
-      r.hi.v[e + 1] = h[1];
-      r.lo.v[e] = l[0];
-      r.lo.v[e + 1] = l[1];
-    }
+    split_bf16<8>(x, r.hi.v, r.lo.v);
     return r;
   }
   static __device__ __forceinline__ F1 hi(const F3& a) { return a.hi; }
@@ -263,11 +268,7 @@ template <> struct Store<true> {
   }
   static __device__ __forceinline__ void st8s(bf16* hi, bf16* lo, const float* x) {
     bf16x8 h, l;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      h[e] = (bf16)x[e];
-      l[e] = (bf16)(x[e] - (float)h[e]);
-    }
+    split_bf16<8>(x, h, l);
     *reinterpret_cast<bf16x8*>(hi) = h;
     *reinterpret_cast<bf16x8*>(lo) = l;
   }
@@ -280,11 +281,7 @@ template <> struct Store<true> {
   }
   static __device__ __forceinline__ void st4s(bf16* hi, bf16* lo, const float* x) {
     bf16x4 h, l;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      h[e] = (bf16)x[e];
-      l[e] = (bf16)(x[e] - (float)h[e]);
-    }
+    split_bf16<4>(x, h, l);
     *reinterpret_cast<bf16x4*>(hi) = h;
     *reinterpret_cast<bf16x4*>(lo) = l;
   }
