@@ -66,6 +66,8 @@ struct BW {
   int c0;                // first chunk of the block (token c0 * BC)
   const float *q, *k, *v, *g, *b, *w;
   int qk_hd, gb_hd;      // q, k (g, b) hold H / hd heads: head h reads head h / hd
+  int g_c, b_c, w_c;     // channels each gate holds per head: 128, or 1 value for all; a
+                         // gate's gradient is then the partial sums of kGateParts
   const int32_t* seg;
   const float* init;     // state entering the block's first chunk (NULL: zero)
   float* sfin;           // NULL or: the forward scan's state leaving the block
@@ -125,13 +127,46 @@ __device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(fm
 
 __device__ __forceinline__ float4 ld4g(const float* p) { return *reinterpret_cast<const float4*>(p); }
 __device__ __forceinline__ float4 zero_f4() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-// 4 consecutive elements of f32 or bf16 storage, as f32
-__device__ __forceinline__ float4 ld4_dt(const void* p, int64_t i, int dt) {
+// Four consecutive elements of f32 or bf16 storage, loaded (ld4_raw) and
+// widened where they are used (cvt4): widened inside the branch on the type,
+// every load would be waited for before the next is issued.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4 ld4_raw(const void* p, int64_t i, int dt) {
   if (dt == DT_BF16) {
-    const bf16x4 x = *reinterpret_cast<const bf16x4*>((const bf16*)p + i);
-    return make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+    const u32x2 x = *reinterpret_cast<const u32x2*>((const bf16*)p + i);
+    return u32x4{x[0], x[1], 0u, 0u};
   }
-  return ld4g((const float*)p + i);
+  return *reinterpret_cast<const u32x4*>((const float*)p + i);
+}
+__device__ __forceinline__ float u2f(uint32_t x) { return __builtin_bit_cast(float, x); }
+__device__ __forceinline__ float4 cvt4(const u32x4& x, int dt) {
+  if (dt == DT_BF16) return make_float4(u2f(x[0] << 16), u2f(x[0] & 0xffff0000u), u2f(x[1] << 16), u2f(x[1] & 0xffff0000u));
+  return make_float4(u2f(x[0]), u2f(x[1]), u2f(x[2]), u2f(x[3]));
+}
+// A gate of one value per (token, head) stays one value: it is spread over the
+// channels where it is read, and its gradient leaves the kernel that forms it
+// as sums over that kernel's own channel groups (dg: the four quarters of
+// k_bw_dqk, db: its eight 16-channel tiles, dw: whole rows of k_bw_grads).
+// Held at 128 channels, the copies of chunk_gdn's three gates and of their
+// gradients were 14 passes over a (token, head, 128) fp32 array.  4096 tokens,
+// 32 heads: preparation 93 to 39 us, the gates' last step 55 to 13; with the
+// decay factors formed once per pair (k_bw_intra, k_bw_dqk), k_bw_intra 361 to
+// 293 and k_bw_dqk 260 to 219.
+constexpr int kGateParts[3] = {4, 8, 1};
+__device__ __forceinline__ u32x4 ld_gate4(const float* g, int64_t row, int chans, int c) {
+  if (chans == 1) return u32x4{__builtin_bit_cast(uint32_t, g[row]), 0u, 0u, 0u};
+  return *reinterpret_cast<const u32x4*>(g + row * KD + c);
+}
+__device__ __forceinline__ float4 gate4_of(const u32x4& x, int chans) {
+  if (chans == 1) return make_float4(u2f(x[0]), u2f(x[0]), u2f(x[0]), u2f(x[0]));
+  return make_float4(u2f(x[0]), u2f(x[1]), u2f(x[2]), u2f(x[3]));
+}
+// sum over the N lanes (a power of two, aligned) around this one
+template <int N> __device__ __forceinline__ float lane_sum(float x) {
+#pragma unroll
+  for (int o = 1; o < N; o <<= 1) x += __shfl_xor(x, o);
+  return x;
 }
 __device__ __forceinline__ float f4at(const float4& v, int i) {
   return i == 0 ? v.x : (i == 1 ? v.y : (i == 2 ? v.z : v.w));
@@ -161,7 +196,7 @@ __device__ __forceinline__ int gofs(int i, int c, int ns) {
 // bf16 mode keeps the four scan operands split: run pair (blk, s) is 64
 // lanes x 8 high bf16 words, then 64 lanes x 8 low words, element (i, c) at
 // index e = 4 * (run) + (c & 3) of its lane (the same bytes as the fp32
-// pair).  op_put4 / op_put8 / op_get8 store and load either form.
+// pair).  op_put4 and op_put8 store either form.
 __device__ __forceinline__ int bofs(int i, int c, int ns) {
   const int cc = c & 31;
   return ((i >> 4) * ns + (c >> 5)) * 1024 + (((cc & 15) >> 2) * 16 + (i & 15)) * 8 + (cc >> 4) * 4 + (c & 3);
@@ -191,20 +226,6 @@ __device__ __forceinline__ void op_put8(bool bf, float* arr, int i, int c, int n
   } else {
     *reinterpret_cast<float4*>(arr + gofs(i, c, ns)) = make_float4(x[0], x[1], x[2], x[3]);
     *reinterpret_cast<float4*>(arr + gofs(i, c + 16, ns)) = make_float4(x[4], x[5], x[6], x[7]);
-  }
-}
-// the 8 values op_put8 stores for one lane of a run pair
-template <bool BF>
-__device__ __forceinline__ void op_get8(const float* arr, int i, int c, int ns, float* x) {
-  if constexpr (BF) {
-    const bf16* b = reinterpret_cast<const bf16*>(arr) + bofs(i, c, ns);
-    const bf16x8 h = *reinterpret_cast<const bf16x8*>(b);
-    const bf16x8 lo = *reinterpret_cast<const bf16x8*>(b + 512);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = (float)h[e] + (float)lo[e];
-  } else {
-    const float4 a = ld4g(arr + gofs(i, c, ns)), d = ld4g(arr + gofs(i, c + 16, ns));
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = d.x; x[5] = d.y; x[6] = d.z; x[7] = d.w;
   }
 }
 // PT (128 x 128) and U0T (128 x chunk) in accumulator order: a 16 x 16 tile
@@ -263,17 +284,19 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   constexpr int SIT = BC * KD / 4 / NT;
   static_assert(SIT == 4 && NT == 16 * (KD / 4) && BC == 64, "token mapping of the staging loop");
   const int nu = p.B * p.H * p.NC;
-  float4 nk[SIT], ng[SIT];
+  float4 nk[SIT];
+  u32x4 ng[SIT];
   auto stage_load = [&](int un) {
     const int c = un % p.NC, bh = un / p.NC, h = bh % p.H, bb = bh / p.H;
     const int t0 = (p.c0 + c) * BC;
 #pragma unroll
     for (int it = 0; it < SIT; ++it) {
       const int c4 = tid % (KD / 4), i = 4 * (tid / (KD / 4)) + it;
-      nk[it] = ng[it] = zero_f4();
+      nk[it] = zero_f4();
+      ng[it] = u32x4{0u, 0u, 0u, 0u};
       if (t0 + i < p.L) {
         nk[it] = ld4g(p.k + row_in(p, bb, t0 + i, h, p.qk_hd) + 4 * c4);
-        ng[it] = ld4g(p.g + row_in(p, bb, t0 + i, h, p.gb_hd) + 4 * c4);
+        ng[it] = ld_gate4(p.g, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, p.g_c, 4 * c4);
       }
     }
   };
@@ -292,19 +315,21 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   }
   // stage the log2-decay (rows past the sequence end are zero); k stays in
   // registers for Kc and beta = b k; q and b arrive during the decay scan
-  float4 kst[SIT], qst[SIT], bst[SIT];
+  float4 kst[SIT], qst[SIT];
+  u32x4 bst[SIT];
 #pragma unroll
   for (int it = 0; it < SIT; ++it) {
     // a thread holds 4 consecutive tokens x 4 channels
     const int c4 = tid % (KD / 4), i = 4 * (tid / (KD / 4)) + it;
-    const float4 gv = ng[it];
+    const float4 gv = gate4_of(ng[it], p.g_c);
     kst[it] = nk[it];
     *reinterpret_cast<float4*>(&sG[i][4 * c4]) =
         make_float4(gv.x * kLog2e, gv.y * kLog2e, gv.z * kLog2e, gv.w * kLog2e);
-    qst[it] = bst[it] = zero_f4();
+    qst[it] = zero_f4();
+    bst[it] = u32x4{0u, 0u, 0u, 0u};
     if (t0 + i < p.L) {
       qst[it] = ld4g(p.q + row_in(p, bb, t0 + i, h, p.qk_hd) + 4 * c4);
-      bst[it] = ld4g(p.b + row_in(p, bb, t0 + i, h, p.gb_hd) + 4 * c4);
+      bst[it] = ld_gate4(p.b, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, p.b_c, 4 * c4);
     }
   }
   lds_barrier();
@@ -372,7 +397,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
 #pragma unroll
   for (int it = 0; it < SIT; ++it) {
     const int c4 = tid % (KD / 4), i = 4 * (tid / (KD / 4)) + it;
-    const float4 k4 = kst[it], b4 = bst[it];
+    const float4 k4 = kst[it], b4 = gate4_of(bst[it], p.b_c);
     *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = qst[it];
     *reinterpret_cast<float4*>(&sW[i][4 * c4]) = make_float4(b4.x * k4.x, b4.y * k4.y, b4.z * k4.z, b4.w * k4.w);
   }
@@ -425,12 +450,34 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   // one task per lower-triangle tile (I, J) forms both A_IJ and M_IJ: they
   // share the column operand k_j e^{G_m - G_j} and the row factor
   // e^{G_i - G_m}
+  // (slots 4-7 hold the diagonal tiles: the two waves with a second task have
+  // none of those, which cost the most where the factors are formed apart)
   for (int tt = wv; tt < 10; tt += NWV) {
-    const int I = (tt >= 1) + (tt >= 3) + (tt >= 6);
-    const int J = tt - I * (I + 1) / 2;
+    const int I = (0xfe4e9 >> (2 * tt)) & 3, J = (0x9e410 >> (2 * tt)) & 3;
     const bool diag = J == I;
     float resA[4], resM[4];
-    if (!diag || (sSafe[2 * I] & sSafe[2 * I + 1])) {
+    if (p.g_c == 1) {
+      // one decay for every channel: plain products, scaled once per element
+      const int i = 16 * I + l16, j = 16 * J + l16;
+      const float* kj = p.k + row_in(p, bb, t0 + j < p.L ? t0 + j : 0, h, p.qk_hd);
+      f32x4 accA = zero4(), accM = zero4();
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float xa[8], xq[8], xb[8];
+        row8(&sW[i][0], s, q, xa);
+        row8(&sQ[i][0], s, q, xq);
+        row8(kj, s, q, xb);
+        const Frag<false> fbk = fr8(xb);
+        mma(accA, fr8(xa), fbk);
+        mma(accM, fr8(xq), fbk);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float f = ex2(sG[16 * I + 4 * q + e][0] - sG[j][0]);
+        resA[e] = accA[e] * f;
+        resM[e] = accM[e] * f;
+      }
+    } else if (!diag || (sSafe[2 * I] & sSafe[2 * I + 1])) {
       const int m = 16 * I;
       const int i = 16 * I + l16, j = 16 * J + l16;
       const bool vi = t0 + i < p.L, vj = t0 + j < p.L;
@@ -496,7 +543,9 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   }
   // w and v of this lane's W / U0 operands, loaded now and used after T
   static_assert(TPW == 1, "one 16-column tile per wave");
-  float wvw[2][8], wvv[2][8];
+  float wvw[2][8];
+  uint32_t wvv[2][8];   // v's bits (a bf16's widen where they are used)
+  const bool v16 = p.v_dt == DT_BF16;
 #pragma unroll
   for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -504,8 +553,9 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
       const int j = 32 * s + pi_k(q, e), r = 16 * wv + l16;
       const bool vj = t0 + j < p.L;
       const int64_t ro = row_of(p, bb, vj ? t0 + j : 0, h) + r;
-      wvw[s][e] = vj ? p.w[ro] : 0.f;
-      wvv[s][e] = vj ? ld_f(p.v, ro, p.v_dt) : 0.f;
+      wvw[s][e] = vj ? p.w[p.w_c == 1 ? ro / KD : ro] : 0.f;
+      wvv[s][e] = 0;
+      if (vj) wvv[s][e] = v16 ? (uint32_t)((const uint16_t*)p.v)[ro] : ((const uint32_t*)p.v)[ro];
     }
   lds_barrier();
 
@@ -607,7 +657,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
       for (int e = 0; e < 8; ++e) {
         const int j = 32 * s + pi_k(q, e);
         xb[e] = scar[j] ? sW[j][r] * ex2(sG[j][r]) : 0.f;
-        xu[e] = wvw[s][e] * wvv[s][e];
+        xu[e] = wvw[s][e] * u2f(v16 ? wvv[s][e] << 16 : wvv[s][e]);
       }
       const typename O::F fb = O::make(xb), fu = O::make(xu);
 #pragma unroll
@@ -656,11 +706,12 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   lds_barrier();
   // the chunk's dO (rows past the sequence end zero), loaded here for the P^T
   // phase at the end (not earlier: it would hold 16 registers through W / U0)
-  float4 dov[BC * KD / 4 / NT];
+  u32x4 dov[BC * KD / 4 / NT];
 #pragma unroll
   for (int it = 0; it < BC * KD / 4 / NT; ++it) {
     const int idx = tid + NT * it, i = idx / (KD / 4), c4 = idx % (KD / 4);
-    dov[it] = t0 + i < p.L ? ld4_dt(p.dout, row_of(p, bb, t0 + i, h) + 4 * c4, p.dout_dt) : zero_f4();
+    dov[it] = u32x4{0u, 0u, 0u, 0u};
+    if (t0 + i < p.L) dov[it] = ld4_raw(p.dout, row_of(p, bb, t0 + i, h) + 4 * c4, p.dout_dt);
   }
   // W in the scan operand order from sW: per task one lane's run pair (rows
   // of 16-row block blk, slab s)
@@ -724,7 +775,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
 #pragma unroll
     for (int it = 0; it < BC * KD / 4 / NT; ++it) {
       const int idx = tid + NT * it, i = idx / (KD / 4), c4 = idx % (KD / 4);
-      *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = dov[it];
+      *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = cvt4(dov[it], p.dout_dt);
     }
     lds_barrier();
     // P^T rows v = 16 w .. 16 w + 15, all 128 k: P[k][v] = sum_i Xf[i][k] dO[i][v]
@@ -1113,6 +1164,14 @@ __device__ __forceinline__ void nt_lds(f32x4 (&acc)[4][TPW], const LMat<BF, KD>&
 #pragma unroll
     for (int I = 0; I < 4; ++I) Op<BF>::mac(acc[I][0], X.row_frag(16 * I + l16, s, q), y[s]);
 }
+// the same with X in the scans' operand order
+template <bool BF>
+__device__ __forceinline__ void nt_op(f32x4 (&acc)[4][TPW], const float* X, const typename Op<BF>::F (&y)[4], int l) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int I = 0; I < 4; ++I) Op<BF>::mac(acc[I][0], op_frag<BF>(X, I, s, KD / 32, l), y[s]);
+}
 template <bool BF>
 __device__ __forceinline__ void split4(const float (&y)[4][8], typename Op<BF>::F (&f)[4]) {
 #pragma unroll
@@ -1125,7 +1184,8 @@ __device__ __forceinline__ void split4(const float (&y)[4][8], typename Op<BF>::
 template <bool BF>
 __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
   using O = Op<BF>;
-  __shared__ LMat<BF, KD> sdO, sX, sU, sT;   // sX: dU, then dX; sT: W, then Kc
+  __shared__ LMat<BF, KD> sdO, sX, sU;   // sX: dU, then dX
+  __shared__ __align__(16) float sT[CK];   // W, then Kc, in the scans' operand order
   __shared__ LMat<BF, BC> sMT;               // M^T, then T^T
   __shared__ int sseg[BC], scar[BC], slast[BC];
   static_assert(TPW == 1, "one 16-column tile per wave");
@@ -1145,28 +1205,36 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
   float4 u0[4];
 #pragma unroll
   for (int I = 0; I < 4; ++I) u0[I] = ld4g(p.U0T + (int64_t)u * CK + aofs(vcol, 16 * I + 4 * q, BC / 16));
+  // every staged operand is loaded before the first is stored: loaded and
+  // widened one by one they were waited for one by one (268 to 253 us at 4096
+  // tokens, 32 heads).  dO's rows past the sequence end are zero.
+  constexpr int OIT = CK / 4 / NT, MIT = CC / 4 / NT;
+  u32x4 dor[OIT], wr[OIT];
+  float4 mr[MIT];
 #pragma unroll
-  for (int it = 0; it < BC * KD / 4 / NT; ++it) {
+  for (int it = 0; it < OIT; ++it) {
     const int idx = tid + NT * it, i = idx / (KD / 4), c4 = idx % (KD / 4);
-    const float4 v = t0 + i < p.L ? ld4_dt(p.dout, row_of(p, bb, t0 + i, h) + 4 * c4, p.dout_dt) : zero_f4();
-    sdO.put4(i, 4 * c4, v);
+    dor[it] = ld4_raw(p.dout, row_of(p, bb, min(t0 + i, p.L - 1), h) + 4 * c4, p.dout_dt);
   }
-  // W (then Kc below) from the scan operand order: per task one lane's run pair
-  auto stage_op = [&](const float* arr, LMat<BF, KD>& dstT) {
-    for (int task = tid; task < BC * KD / 8; task += NT) {
-      const int ln = task & 63, pr = task >> 6, blk = pr / (KD / 32), s = pr % (KD / 32);
-      const int i = 16 * blk + (ln & 15), cc = 32 * s + 4 * (ln >> 4);
-      float x[8];
-      op_get8<BF>(arr, i, cc, KD / 32, x);
-      dstT.put4(i, cc, make_float4(x[0], x[1], x[2], x[3]));
-      dstT.put4(i, cc + 16, make_float4(x[4], x[5], x[6], x[7]));
-    }
-  };
-  stage_op(p.Wm + (int64_t)u * CK, sT);
+  const float* Wu = p.Wm + (int64_t)u * CK;
+  const float* Ku = p.Kc + (int64_t)u * CK;
 #pragma unroll
-  for (int it = 0; it < CC / 4 / NT; ++it) {
-    const int idx = tid + NT * it, i = idx / (BC / 4), c4 = idx % (BC / 4);
-    sMT.put4(i, 4 * c4, ld4g(p.MT + (int64_t)u * CC + i * BC + 4 * c4));
+  for (int it = 0; it < OIT; ++it) wr[it] = *reinterpret_cast<const u32x4*>(Wu + 4 * (tid + NT * it));
+#pragma unroll
+  for (int it = 0; it < MIT; ++it) mr[it] = ld4g(p.MT + (int64_t)u * CC + 4 * (tid + NT * it));
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int it = 0; it < OIT; ++it) {
+    const int idx = tid + NT * it, i = idx / (KD / 4), c4 = idx % (KD / 4);
+    sdO.put4(i, 4 * c4, t0 + i < p.L ? cvt4(dor[it], p.dout_dt) : zero_f4());
+  }
+  // W (then Kc below) as stored: the scans' operand order is this product's too
+#pragma unroll
+  for (int it = 0; it < OIT; ++it) *reinterpret_cast<u32x4*>(&sT[4 * (tid + NT * it)]) = wr[it];
+#pragma unroll
+  for (int it = 0; it < MIT; ++it) {
+    const int idx = tid + NT * it;
+    sMT.put4(idx / (BC / 4), 4 * (idx % (BC / 4)), mr[it]);
   }
   lds_barrier();
 
@@ -1175,34 +1243,18 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
   zero_acc(acc);
   typename O::F fA[4], fS0[4], fB[4];
   split4<BF>(yA, fA);
-  nt_lds<BF>(acc, sT, fA, q, l16);
+  nt_op<BF>(acc, sT, fA, l);
   load_yT(yB, dSC, wv, q, l16);
-  // Kc: this thread's two run-pair lanes, staged once W is done
-  static_assert(BC * KD / 8 == 2 * NT, "two run-pair lanes per thread");
-  float kcx[2][8];
-  auto kc_pos = [&](int t2, int& i, int& cc) {
-    const int task = tid + NT * t2, ln = task & 63, pr = task >> 6;
-    i = 16 * (pr / (KD / 32)) + (ln & 15);
-    cc = 32 * (pr % (KD / 32)) + 4 * (ln >> 4);
-  };
+  // Kc: loaded now, staged once W is done
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2) {
-    int i, cc;
-    kc_pos(t2, i, cc);
-    op_get8<BF>(p.Kc + (int64_t)u * CK, i, cc, KD / 32, kcx[t2]);
-  }
+  for (int it = 0; it < OIT; ++it) wr[it] = *reinterpret_cast<const u32x4*>(Ku + 4 * (tid + NT * it));
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
     for (int e = 0; e < 4; ++e) sU.put(16 * I + 4 * q + e, vcol, f4at(u0[I], e) - acc[I][0][e]);
   lds_barrier();   // U complete; every wave is done with W
 #pragma unroll
-  for (int t2 = 0; t2 < 2; ++t2) {
-    int i, cc;
-    kc_pos(t2, i, cc);
-    sT.put4(i, cc, make_float4(kcx[t2][0], kcx[t2][1], kcx[t2][2], kcx[t2][3]));
-    sT.put4(i, cc + 16, make_float4(kcx[t2][4], kcx[t2][5], kcx[t2][6], kcx[t2][7]));
-  }
+  for (int it = 0; it < OIT; ++it) *reinterpret_cast<u32x4*>(&sT[4 * (tid + NT * it)]) = wr[it];
 
   // rowsum over v of S0 * dSC for channel 16 wv + l16 (the lane's S0 and dSC
   // columns hold the same (k, v) pairs; the 4 lanes of a channel split v)
@@ -1234,14 +1286,14 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
   for (int it = 0; it < 2; ++it) ttq[it] = ld4g(p.TT + (int64_t)u * CC + 4 * (tid + NT * it));
   // w, v of the coalesced dv / dw pass: float4s tid + NT it of the chunk's
   // row-major 64 x 128 tiles
-  float4 wq[BC * KD / 4 / NT], vq[BC * KD / 4 / NT];
+  u32x4 wq[BC * KD / 4 / NT], vq[BC * KD / 4 / NT];
 #pragma unroll
   for (int it = 0; it < BC * KD / 4 / NT; ++it) {
     const int idx = tid + NT * it, i = idx / (KD / 4), c4 = idx % (KD / 4);
     const bool vi = t0 + i < p.L;
     const int64_t ro = row_of(p, bb, vi ? t0 + i : 0, h) + 4 * c4;
-    wq[it] = vi ? ld4g(p.w + ro) : zero_f4();
-    vq[it] = vi ? ld4_dt(p.v, ro, p.v_dt) : zero_f4();
+    wq[it] = ld_gate4(p.w, ro / KD, p.w_c, 4 * c4);   // (rows past the end: unused)
+    vq[it] = ld4_raw(p.v, ro, p.v_dt);
   }
   lds_barrier();   // Kc staged
 
@@ -1255,7 +1307,7 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
       if (s == 1 || I < 2) O::mac(acc[I][0], sMT.row_frag(16 * I + l16, s, q), bfr);   // M^T / T^T upper triangular
   }
   split4<BF>(yA, fA);
-  nt_lds<BF>(acc, sT, fA, q, l16);
+  nt_op<BF>(acc, sT, fA, l);
 #pragma unroll
   for (int I = 0; I < 4; ++I)
 #pragma unroll
@@ -1290,7 +1342,7 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
     if (t0 + i < p.L) {
       const int64_t ro = row_of(p, bb, t0 + i, h) + 4 * c4;
       const float4 dx = sX.get4(i, 4 * c4);
-      const float4 a = wq[it], v4 = vq[it];
+      const float4 a = gate4_of(wq[it], p.w_c), v4 = cvt4(vq[it], p.v_dt);
       const float4 dv = make_float4(dx.x * a.x, dx.y * a.y, dx.z * a.z, dx.w * a.w);
       if (p.dv_dt == DT_BF16) {
         bf16x4 hb;
@@ -1299,7 +1351,13 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
       } else {
         *reinterpret_cast<float4*>(p.dv + ro) = dv;
       }
-      *reinterpret_cast<float4*>(p.dw + ro) = make_float4(dx.x * v4.x, dx.y * v4.y, dx.z * v4.z, dx.w * v4.w);
+      const float4 dw = make_float4(dx.x * v4.x, dx.y * v4.y, dx.z * v4.z, dx.w * v4.w);
+      if (p.w_c == 1) {   // a row is one 32-lane half
+        const float sum = lane_sum<32>((dw.x + dw.y) + (dw.z + dw.w));
+        if (c4 == 0) p.dw[ro / KD] = sum;
+      } else {
+        *reinterpret_cast<float4*>(p.dw + ro) = dw;
+      }
     }
   }
 
@@ -1408,15 +1466,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
   for (int it = 0; it < BC * HC / 4 / NT; ++it) {
     const int idx = tid + NT * it, i = idx / (HC / 4), c4 = idx % (HC / 4);
-    float4 qv = zero_f4(), kv = zero_f4(), bv = zero_f4();
-    if (t0 + i < p.L) {
-      const int64_t rq = row_in(p, bb, t0 + i, h, p.qk_hd) + ch0 + 4 * c4;
-      qv = ld4g(p.q + rq); kv = ld4g(p.k + rq); bv = ld4g(p.b + row_in(p, bb, t0 + i, h, p.gb_hd) + ch0 + 4 * c4);
-    }
-    *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = qv;
-    *reinterpret_cast<float4*>(&sK[i][4 * c4]) = kv;
-    *reinterpret_cast<float4*>(&sB[i][4 * c4]) = bv;
-    *reinterpret_cast<float4*>(&sG[i][4 * c4]) = ld4g(G + i * KD + ch0 + 4 * c4);
+    // (the last row's values stand in past the sequence end, replaced by zeros)
+    const int t = min(t0 + i, p.L - 1);
+    const int64_t rq = row_in(p, bb, t, h, p.qk_hd) + ch0 + 4 * c4;
+    const float4 q4 = ld4g(p.q + rq), k4 = ld4g(p.k + rq), g4 = ld4g(G + i * KD + ch0 + 4 * c4);
+    const u32x4 b4 = ld_gate4(p.b, row_in(p, bb, t, h, p.gb_hd) / KD, p.b_c, ch0 + 4 * c4);
+    const bool in = t0 + i < p.L;
+    *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = in ? q4 : zero_f4();
+    *reinterpret_cast<float4*>(&sK[i][4 * c4]) = in ? k4 : zero_f4();
+    *reinterpret_cast<float4*>(&sB[i][4 * c4]) = in ? gate4_of(b4, p.b_c) : zero_f4();
+    *reinterpret_cast<float4*>(&sG[i][4 * c4]) = g4;
   }
 #pragma unroll
   for (int it = 0; it < CC / 4 / NT; ++it) {
@@ -1425,6 +1484,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     *reinterpret_cast<float4*>(&sdA[i][4 * c4]) = ld4g(p.dAw + (int64_t)u * CC + i * BC + 4 * c4);
   }
   lds_barrier();
+  // one decay for every channel: dM and dA take their factors e^{G_i - G_j}
+  // once, and every product below is a plain one
+  const bool sc = p.g_c == 1;
+  if (sc) {
+#pragma unroll
+    for (int it = 0; it < CC / 4 / NT; ++it) {
+      const int idx = tid + NT * it, i = idx / (BC / 4), c4 = idx % (BC / 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float f = ex2(sG[i][0] - sG[4 * c4 + e][0]);
+        sdM[i][4 * c4 + e] *= f;
+        sdA[i][4 * c4 + e] *= f;
+      }
+    }
+    lds_barrier();
+  }
 
   const float glast = sG[BC - 1][rl];
   float rdg[NB][4], rpp[NB][4];   // dG and P of this lane's rows
@@ -1447,7 +1522,41 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int m = 16 * I, m2 = 16 * I + 15;
     const float gm = sG[m][rl], gm2 = sG[m2][rl];
     // G restarts at document starts: the in-block factors need one document
-    const bool inblk = sseg[m] == sseg[m2] && __all(gm - gm2 <= 64.f);
+    const bool inblk = !sc && sseg[m] == sseg[m2] && __all(gm - gm2 <= 64.f);
+    if (sc) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float xm[8], xa[8], xk[8], ym[8], ya[8], yq[8], yb[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int j = 32 * s + pi_k(q, e);
+          const bool self = j == 16 * I + l16;
+          xm[e] = self ? 0.f : sdM[16 * I + l16][j];
+          xa[e] = sdA[16 * I + l16][j];
+          ym[e] = self ? 0.f : sdM[j][16 * I + l16];
+          ya[e] = sdA[j][16 * I + l16];
+          xk[e] = sK[j][rl];
+          yq[e] = sQ[j][rl];
+          yb[e] = sB[j][rl] * xk[e];
+        }
+        // row blocks up to I for dq and dbeta, from I for dk
+        if (2 * s == I) {
+          mma_half(oq, xm, xk, 0);
+          mma_half(ob, xa, xk, 0);
+        } else if (2 * s < I) {
+          const Frag<false> fk = fr8(xk);
+          mma(oq, fr8(xm), fk);
+          mma(ob, fr8(xa), fk);
+        }
+        if (2 * s + 1 == I) {
+          mma_half(ok_, ym, yq, 1);
+          mma_half(ok_, ya, yb, 1);
+        } else if (2 * s + 1 > I) {
+          mma(ok_, fr8(ym), fr8(yq));
+          mma(ok_, fr8(ya), fr8(yb));
+        }
+      }
+    } else
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
       float xm[8], xa[8], xk[8], ym[8], ya[8], yq[8], yb[8];
@@ -1533,7 +1642,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const int i = 16 * I + ii;
       const float gi = sG[i][rl];
       float dq = 0.f, dbeta = 0.f, dk = 0.f;
-      if (!inblk) {
+      if (!inblk && !sc) {
         // pairs inside block I, e^{G_i - G_j} per element
 #pragma unroll
         for (int jj = 0; jj < 16; ++jj) {
@@ -1548,9 +1657,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
       }
       const float eg = scar[i] ? ex2(gi) : 0.f;
-      dq += eg * rq[Ib][e] + oq[e] * ex2(gi - gm);
-      dbeta += -eg * rb[Ib][e] + ob[e] * ex2(gi - gm);
-      dk += ok_[e] * ex2(gm2 - gi);
+      const float fi = sc ? 1.f : ex2(gi - gm);
+      dq += eg * rq[Ib][e] + oq[e] * fi;
+      dbeta += -eg * rb[Ib][e] + ob[e] * fi;
+      dk += sc ? ok_[e] : ok_[e] * ex2(gm2 - gi);
       if (inblk) dk += okb[e] * __builtin_amdgcn_exp2f(gm - gi);   // <= 2^64 (the block's span)
       const float dkc = slast[i] ? ex2(glast - gi) * rk[Ib][e] : 0.f;
       const float kv = sK[i][rl], qv = sQ[i][rl], bv = sB[i][rl], dmii = sdM[i][i];
@@ -1560,7 +1670,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const int64_t ro = row_of(p, bb, t0 + i, h) + r;
         p.dq[ro] = dq + dmii * kv;
         p.dk[ro] = dk + dmii * qv + dkc + bv * dbeta;
-        p.db[ro] = kv * dbeta;
+        if (p.b_c != 1) p.db[ro] = kv * dbeta;
+      }
+      if (p.b_c == 1) {   // 16 channels of a row: one 16-lane row
+        const float sum = lane_sum<16>(kv * dbeta);
+        if (l16 == 0 && t0 + i < p.L) p.db[row_of(p, bb, t0 + i, h) / KD * kGateParts[1] + (r >> 4)] = sum;
       }
     }
   }
@@ -1616,8 +1730,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       dgv[e] += acc;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (t0 + 4 * sg + e < p.L) p.dg[row_of(p, bb, t0 + 4 * sg + e, h) + ch0 + ch] = dgv[e];
+    for (int e = 0; e < 4; ++e) {
+      const int t = t0 + 4 * sg + e;
+      if (p.g_c == 1) {   // the quarter's 32 channels: one 32-lane half
+        const float sum = lane_sum<HC>(dgv[e]);
+        if (ch == 0 && t < p.L) p.dg[row_of(p, bb, t, h) / KD * kGateParts[0] + part] = sum;
+      } else if (t < p.L) {
+        p.dg[row_of(p, bb, t, h) + ch0 + ch] = dgv[e];
+      }
+    }
   }
 }
 
@@ -1630,19 +1751,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // ---------------------------------------------------------------------------
 struct BR {
   int B, L, Hk, Hv, G;
-  const void *q, *k, *v;
-  int qk_dt, v_dt;
+  const void *q, *k;
+  int qk_dt;
   const float *g, *b, *w;
   int g_h, g_c, b_h, b_c, w_h, w_c;
   const void* seg; int seg_dt, seg_batched;
   const int32_t* init_seg; int has_init;
   float scale; int l2norm, fuse, guard;
   int32_t* canon;                                 // (B, L)
-  float *qe, *ke, *ve, *ge, *be, *we;             // prepared inputs: qe, ke (B, L, Hk, 128); ge, be
-                                                  // (B, L, Hv / gb_hd, 128); ve, we (B, L, Hv, 128)
+  float *qe, *ke, *ge, *be, *we;                  // prepared inputs: qe, ke (B, L, Hk, 128); ge, be
+                                                  // (B, L, Hv / gb_hd, channels); we (B, L, Hv, channels)
   int gb_hd;                                      // G when g and b both sit at the key heads, else 1
   int w_alias;                                    // w's prologue step is the identity: we unused
-  const float *dqe, *dke, *dge, *dbe, *dwe;       // their gradients
+  const float *dqe, *dke, *dge, *dbe, *dwe;       // their gradients (of a one-channel gate: partial sums)
   float *dq, *dk, *dg, *db, *dw;                  // raw-layout gradients (dq, dk in qk_dt)
 };
 
@@ -1748,11 +1869,10 @@ __global__ __launch_bounds__(256) void k_bw_prep(BR p) {
   const bool b16 = p.qk_dt != DT_F32;
   const int hg = gate_head(p.g_h, p.Hk, p.Hv, hv, p.G), hb = gate_head(p.b_h, p.Hk, p.Hv, hv, p.G);
   const int hw = gate_head(p.w_h, p.Hk, p.Hv, hv, p.G);
-  float gv[4], bv[4], wv[4] = {0.f, 0.f, 0.f, 0.f}, vv[4];
+  float gv[4], bv[4], wv[4] = {0.f, 0.f, 0.f, 0.f};
   gate4(p.g, (bt * p.g_h + hg) * p.g_c, p.g_c, c, gv);
   gate4(p.b, (bt * p.b_h + hb) * p.b_c, p.b_c, c, bv);
   if (!p.w_alias) gate4(p.w, (bt * p.w_h + hw) * p.w_c, p.w_c, c, wv);
-  ld4_any(p.v, (bt * p.Hv + hv) * KD + c, p.v_dt, vv);
   float qh[4], kh[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -1780,20 +1900,22 @@ __global__ __launch_bounds__(256) void k_bw_prep(BR p) {
     if (p.guard) gv[e] = fminf(gv[e], -1e-6f);
   }
   if (!valid) return;
-  const int64_t o = row * KD + c;
   // q, k (and g, b at the key heads) once per key head: the first value head
   // of the group writes them
   if (hv % p.G == 0) {
     *reinterpret_cast<float4*>(p.qe + qrow) = make_float4(qh[0], qh[1], qh[2], qh[3]);
     *reinterpret_cast<float4*>(p.ke + qrow) = make_float4(kh[0], kh[1], kh[2], kh[3]);
   }
+  auto put_gate = [&](float* g, int64_t grow, int chans, const float* x) {
+    if (chans != 1) *reinterpret_cast<float4*>(g + grow * KD + c) = make_float4(x[0], x[1], x[2], x[3]);
+    else if (c == 0) g[grow] = x[0];
+  };
   if (hv % p.gb_hd == 0) {
-    const int64_t og = (bt * (p.Hv / p.gb_hd) + hv / p.gb_hd) * KD + c;
-    *reinterpret_cast<float4*>(p.ge + og) = make_float4(gv[0], gv[1], gv[2], gv[3]);
-    *reinterpret_cast<float4*>(p.be + og) = make_float4(bv[0], bv[1], bv[2], bv[3]);
+    const int64_t grow = bt * (p.Hv / p.gb_hd) + hv / p.gb_hd;
+    put_gate(p.ge, grow, p.g_c, gv);
+    put_gate(p.be, grow, p.b_c, bv);
   }
-  if (!p.w_alias) *reinterpret_cast<float4*>(p.we + o) = make_float4(wv[0], wv[1], wv[2], wv[3]);
-  *reinterpret_cast<float4*>(p.ve + o) = make_float4(vv[0], vv[1], vv[2], vv[3]);
+  if (!p.w_alias) put_gate(p.we, row, p.w_c, wv);
 }
 
 // two (batch, token, key head) rows per wave, one per 32-lane half, four
@@ -1870,8 +1992,6 @@ __device__ __forceinline__ void post_qk_rows(const BR& p) {
 
 __global__ __launch_bounds__(256) void k_bw_post_qk(BR p) { post_qk_rows(p); }
 
-// one thread per raw gate element: the sum of the prepared gradient over the
-// value heads and channels it was broadcast to, times the prologue derivative
 // derivative of the prologue step of gate WHICH at raw value x
 template <int WHICH>
 __device__ __forceinline__ float gate_deriv(const BR& p, float x) {
@@ -1890,42 +2010,32 @@ __device__ __forceinline__ float gate_deriv(const BR& p, float x) {
   }
 }
 
+// gates of one channel: one thread per (token, head)
 template <int WHICH>   // 0 = g, 1 = b, 2 = w
 __global__ __launch_bounds__(256) void k_bw_post_gate(BR p) {
+  constexpr int NP = kGateParts[WHICH];
   const int H = WHICH == 0 ? p.g_h : (WHICH == 1 ? p.b_h : p.w_h);
-  const int C = WHICH == 0 ? p.g_c : (WHICH == 1 ? p.b_c : p.w_c);
   const float* raw = WHICH == 0 ? p.g : (WHICH == 1 ? p.b : p.w);
   const float* dpre = WHICH == 0 ? p.dge : (WHICH == 1 ? p.dbe : p.dwe);
   float* out = WHICH == 0 ? p.dg : (WHICH == 1 ? p.db : p.dw);
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t n = (int64_t)p.B * p.L * H * C;
-  if (idx >= n) return;
-  const int c = (int)(idx % C);
-  const int h = (int)((idx / C) % H);
-  const int64_t bt = idx / ((int64_t)C * H);
+  if (idx >= (int64_t)p.B * p.L * H) return;
+  const int h = (int)(idx % H);
+  const int64_t bt = idx / H;
   // value heads that read gate head h: h (H = Hv), h G .. h G + G - 1 (H = Hk), all (H = 1)
   int h0, hn;
   if (H == p.Hv) { h0 = h; hn = 1; }
   else if (H == p.Hk) { h0 = h * p.G; hn = p.G; }
   else { h0 = 0; hn = p.Hv; }
-  const float* rowp = dpre + (bt * p.Hv + h0) * KD;
+  const float* rowp = dpre + (bt * p.Hv + h0) * NP;
   float s = 0.f;
-  if (C == 1) {
-    for (int j = 0; j < hn; ++j, rowp += KD) {
-      float4 acc = zero_f4();
-#pragma unroll 8
-      for (int i4 = 0; i4 < KD / 4; ++i4) {
-        const float4 x4 = ld4g(rowp + 4 * i4);
-        acc.x += x4.x; acc.y += x4.y; acc.z += x4.z; acc.w += x4.w;
-      }
-      s += (acc.x + acc.y) + (acc.z + acc.w);
-    }
-  } else {
-    for (int j = 0; j < hn; ++j, rowp += KD) s += rowp[c];
+  for (int j = 0; j < hn; ++j, rowp += NP) {
+    float x = 0.f;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) x += rowp[i];
+    s += x;
   }
-  const float x = raw[idx];
-  const float d = gate_deriv<WHICH>(p, x);
-  out[idx] = s * d;
+  out[idx] = s * gate_deriv<WHICH>(p, raw[idx]);
 }
 
 // channel-wise gates (C = 128): one thread per 4 channels of one (token, head)
@@ -2052,7 +2162,7 @@ extern "C" size_t dn_prefill_bwd_workspace_size(const dn_backward_args* a) {
 
 // the recurrence backward with the element types of d_out and dv given
 static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt, bool bf, void* workspace,
-                    size_t workspace_bytes, void* stream, int qk_hd = 1, int gb_hd = 1) {
+                    size_t workspace_bytes, void* stream, int qk_hd = 1, int gb_hd = 1, int g_c = KD, int b_c = KD, int w_c = KD) {
   const int rc = bw_check(a);
   if (rc != DN_OK) return rc;
   const size_t need = bw_workspace_bytes(a);
@@ -2064,7 +2174,7 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
   p.bf = bf;
   p.q = (const float*)a->q; p.k = (const float*)a->k; p.v = (const float*)a->v;
   p.g = (const float*)a->g; p.b = (const float*)a->b; p.w = (const float*)a->w;
-  p.qk_hd = qk_hd; p.gb_hd = gb_hd;
+  p.qk_hd = qk_hd; p.gb_hd = gb_hd; p.g_c = g_c; p.b_c = b_c; p.w_c = w_c;
   p.seg = a->seg;
   p.dout = a->d_out; p.dout_dt = dout_dt; p.dv_dt = dv_dt; p.v_dt = v_dt;
   p.dq = (float*)a->dq; p.dk = (float*)a->dk; p.dv = (float*)a->dv;
@@ -2140,20 +2250,31 @@ extern "C" int dn_prefill_bwd(const dn_backward_args* a, void* workspace, size_t
 namespace {
 
 // Prepared inputs and their gradients: qe, ke at the key heads; ge, be at
-// Hv / gb_hd heads; ve, we and the five gradients at the value heads.
+// Hv / gb_hd heads; we and the five gradients at the value heads.  A gate of
+// one channel holds one value per row, its gradient kGateParts.
 struct RawLayout {
-  size_t canon, pre, pre_k, pre_gb, core;   // bytes (pre*: one array)
+  size_t canon, pre[10], core;   // bytes: qe, ke, ge, be, we, dqe, dke, dge, dbe, dwe
   int gb_hd;
-  size_t total() const { return canon + 7 * pre + 2 * pre_k + 2 * pre_gb + core; }
+  size_t total() const {
+    size_t t = canon + core;
+    for (size_t x : pre) t += x;
+    return t;
+  }
 };
 
 RawLayout raw_layout(const dn_prefill_args* a) {
   RawLayout r;
-  r.canon = (((size_t)a->B * a->L * sizeof(int32_t)) + 255) & ~(size_t)255;
-  r.pre = (size_t)a->B * a->L * a->Hv * KD * sizeof(float);
-  r.pre_k = (size_t)a->B * a->L * a->Hk * KD * sizeof(float);
+  auto floats = [](size_t n) { return (n * sizeof(float) + 255) & ~(size_t)255; };
+  const size_t bl = (size_t)a->B * a->L;
+  r.canon = floats(bl);
   r.gb_hd = (a->g_heads == a->Hk && a->b_heads == a->Hk) ? a->Hv / a->Hk : 1;
-  r.pre_gb = r.pre / r.gb_hd;
+  const int gc[3] = {a->g_chans, a->b_chans, a->w_chans};
+  r.pre[0] = r.pre[1] = floats(bl * a->Hk * KD);
+  r.pre[5] = r.pre[6] = floats(bl * a->Hv * KD);
+  for (int i = 0; i < 3; ++i) {
+    r.pre[2 + i] = floats(bl * (i < 2 ? a->Hv / r.gb_hd : a->Hv) * gc[i]);
+    r.pre[7 + i] = floats(bl * a->Hv * (gc[i] == 1 ? kGateParts[i] : KD));
+  }
   dn_backward_args c{};
   c.B = a->B; c.L = a->L; c.H = a->Hv;
   c.recompute_states = a->recompute_states;
@@ -2203,20 +2324,20 @@ extern "C" int dn_prefill_bwd_raw(const dn_prefill_args* a, const void* d_out, c
   char* w = (char*)workspace;
   BR r{};
   r.B = a->B; r.L = a->L; r.Hk = a->Hk; r.Hv = a->Hv; r.G = a->Hv / a->Hk;
-  r.q = a->q; r.k = a->k; r.v = a->v; r.qk_dt = a->qk_dtype; r.v_dt = a->v_dtype;
+  r.q = a->q; r.k = a->k; r.qk_dt = a->qk_dtype;
   r.g = (const float*)a->g; r.b = (const float*)a->b; r.w = (const float*)a->w;
   r.g_h = a->g_heads; r.g_c = a->g_chans; r.b_h = a->b_heads; r.b_c = a->b_chans; r.w_h = a->w_heads; r.w_c = a->w_chans;
   r.seg = a->seg; r.seg_dt = a->seg_dtype; r.seg_batched = a->seg_batched;
   r.init_seg = a->init_seg; r.has_init = a->init_state != nullptr;
   r.scale = a->scale; r.l2norm = a->qk_l2norm; r.fuse = a->fuse_prologue; r.guard = a->stability_guard;
   r.canon = (int32_t*)w; w += lay.canon;
-  float* pre[11];
-  for (int i = 0; i < 11; ++i) {
+  float* pre[10];
+  for (int i = 0; i < 10; ++i) {
     pre[i] = (float*)w;
-    w += i < 2 ? lay.pre_k : (i == 3 || i == 4) ? lay.pre_gb : lay.pre;
+    w += lay.pre[i];
   }
-  r.qe = pre[0]; r.ke = pre[1]; r.ve = pre[2]; r.ge = pre[3]; r.be = pre[4]; r.we = pre[5];
-  r.dqe = pre[6]; r.dke = pre[7]; r.dge = pre[8]; r.dbe = pre[9]; r.dwe = pre[10];
+  r.qe = pre[0]; r.ke = pre[1]; r.ge = pre[2]; r.be = pre[3]; r.we = pre[4];
+  r.dqe = pre[5]; r.dke = pre[6]; r.dge = pre[7]; r.dbe = pre[8]; r.dwe = pre[9];
   // the recurrence kernels read w in place when its prologue step is the
   // identity on a per-value-head, channel-wise layout
   r.w_alias = !a->fuse_prologue && !a->stability_guard && a->w_heads == a->Hv && a->w_chans == KD;
@@ -2232,15 +2353,16 @@ extern "C" int dn_prefill_bwd_raw(const dn_prefill_args* a, const void* d_out, c
   dn_backward_args c{};
   c.abi_version = DN_ABI_VERSION;
   c.B = a->B; c.L = a->L; c.H = a->Hv; c.K = KD; c.V = KD;
-  c.q = r.qe; c.k = r.ke; c.v = r.ve; c.g = r.ge; c.b = r.be; c.w = r.w_alias ? a->w : r.we;
+  c.q = r.qe; c.k = r.ke; c.v = a->v; c.g = r.ge; c.b = r.be; c.w = r.w_alias ? a->w : r.we;
   c.seg = r.canon; c.init_state = a->init_state; c.d_out = d_out; c.d_final = d_final;
   // without the fused prologue, w's step has derivative 1: at Hv heads and
   // channel-wise the recurrence backward writes dw in its raw layout itself
   const bool dw_direct = !a->fuse_prologue && a->w_heads == a->Hv && a->w_chans == KD;
-  c.dq = pre[6]; c.dk = pre[7]; c.dv = dv; c.dg = pre[8]; c.db = pre[9]; c.dw = dw_direct ? (float*)dw : pre[10];
+  c.dq = pre[5]; c.dk = pre[6]; c.dv = dv; c.dg = pre[7]; c.db = pre[8]; c.dw = dw_direct ? (float*)dw : pre[9];
   c.d_init = d_init;
   c.recompute_states = a->recompute_states;
-  rc = bwd_core(&c, a->v_dtype, a->v_dtype, DT_F32, a->precision == 0, w, lay.core, stream, a->Hv / a->Hk, r.gb_hd);
+  rc = bwd_core(&c, a->v_dtype, a->v_dtype, a->v_dtype, a->precision == 0, w, lay.core, stream, a->Hv / a->Hk, r.gb_hd,
+                a->g_chans, a->b_chans, a->w_chans);
   if (rc != DN_OK) return rc;
 
   const int64_t krows = (int64_t)a->B * a->L * a->Hk;
