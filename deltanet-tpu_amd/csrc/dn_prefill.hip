@@ -1642,14 +1642,15 @@ bool scalar_gates(const dn_prefill_args* a) {
 // width 72, 4096 tokens 112 / 115, 16384 638 / 536; width 104-112, 4096 tokens
 // 120-149 / 180-190, 16384 650-755 / 637-733; width 224, 16384 tokens
 // 965 / 1191; fp32 width 9-36, 2048 tokens 123 / 163, 16384 800 / 525.  With
-// scalar gates the scan's prepass is the smaller by far: width 14, 4096 tokens
-// 92 / 97, 16384 316 / 290.
+// scalar gates both prepasses are the smaller by far: width 14-28, 2048 tokens
+// 56 / 68, 4096 94 / 90, 16384 316 / 218-263; width 56, 4096 tokens 94 / 96, 16384
+// 337 / 479.
 Form form_of(const dn_prefill_args* a) {
   const bool sc = scalar_gates(a);
   const int64_t G = a->gates_at_hv ? 1 : a->Hv / a->Hk;
   const int64_t width = (int64_t)a->B * (a->gates_at_hv ? a->Hv : a->Hk) * (5 + 2 * G);
   int64_t least = INT64_MAX;   // tokens from which the long form is the faster
-  if (sc) least = width <= 28 ? 8192 : INT64_MAX;
+  if (sc) least = width <= 28 ? 3584 : INT64_MAX;
   else least = width <= 40 ? 3072 : (width <= 75 ? 8192 : (width <= 115 ? 16384 : INT64_MAX));
   if (a->nt >= least) return kLong;
   return sc ? kScalar : kScan;

@@ -61,6 +61,7 @@ def test_column_tiles(B, Hk, Hv, scalar, v_dt, fuse):
 
 # either side of the length from which few heads take the affine form
 @pytest.mark.parametrize("L,scalar,precision", [(3071, False, "bf16"), (3072, False, "bf16"), (3200, False, "fp32"),
-                                                (3073, False, "fp32"), (8191, True, "bf16"), (8193, True, "bf16")])
+                                                (3073, False, "fp32"), (3583, True, "bf16"), (3584, True, "bf16"),
+                                                (8191, True, "bf16"), (8193, True, "bf16")])
 def test_long_form_edges(L, scalar, precision):
     run(L, 1, L, 1, 2, scalar=scalar, precision=precision, init=False)
