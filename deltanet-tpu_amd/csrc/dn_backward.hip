@@ -2251,15 +2251,13 @@ namespace {
 
 // Prepared inputs and their gradients: qe, ke at the key heads; ge, be at
 // Hv / gb_hd heads; we and the five gradients at the value heads.  A gate of
-// one channel holds one value per row, its gradient kGateParts.
+// one channel holds one value per row, its gradient kGateParts.  The size asked
+// of a caller stays that of every array at 128 channels and a copy of v, which
+// these never exceed.
 struct RawLayout {
   size_t canon, pre[10], core;   // bytes: qe, ke, ge, be, we, dqe, dke, dge, dbe, dwe
+  size_t total;
   int gb_hd;
-  size_t total() const {
-    size_t t = canon + core;
-    for (size_t x : pre) t += x;
-    return t;
-  }
 };
 
 RawLayout raw_layout(const dn_prefill_args* a) {
@@ -2279,6 +2277,7 @@ RawLayout raw_layout(const dn_prefill_args* a) {
   c.B = a->B; c.L = a->L; c.H = a->Hv;
   c.recompute_states = a->recompute_states;
   r.core = bw_workspace_bytes(&c);
+  r.total = r.canon + 7 * r.pre[5] + 2 * r.pre[0] + 2 * (r.pre[5] / r.gb_hd) + r.core;
   return r;
 }
 
@@ -2308,7 +2307,7 @@ int raw_check(const dn_prefill_args* a) {
 
 extern "C" size_t dn_prefill_bwd_raw_workspace_size(const dn_prefill_args* a) {
   if (raw_check(a) != DN_OK) return 0;
-  return raw_layout(a).total();
+  return raw_layout(a).total;
 }
 
 extern "C" int dn_prefill_bwd_raw(const dn_prefill_args* a, const void* d_out, const void* d_final,
@@ -2319,7 +2318,7 @@ extern "C" int dn_prefill_bwd_raw(const dn_prefill_args* a, const void* d_out, c
   if (!d_out || !dq || !dk || !dv || !dg || !db || !dw) return set_error(DN_E_INVALID, "missing gradient pointer");
   if (d_init != nullptr && a->init_state == nullptr) return set_error(DN_E_INVALID, "d_init needs init_state");
   const RawLayout lay = raw_layout(a);
-  if (workspace == nullptr || workspace_bytes < lay.total())
+  if (workspace == nullptr || workspace_bytes < lay.total)
     return set_error(DN_E_WORKSPACE, "workspace too small");
   char* w = (char*)workspace;
   BR r{};
