@@ -1343,7 +1343,9 @@ __global__ __launch_bounds__(512) void k_chain_cols(const PF p) {
       for (int ii = 0; ii < 4; ++ii) S[m][ii] = p.has_init ? p.init[sbase + (int64_t)(16 * m + 4 * q + ii) * KD] : 0.f;
     OutRows<bf16> orow(p, b, hv, r16, vc0 + 4 * q);
     // v of (token 16rt + 4q + ii, this lane's column) of the next chunk, zero
-    // past the last token (the resource ends with its row)
+    // past the last token: the resource ends with its row, and the whole row
+    // offset is in the lane's own offset (the scalar one takes no part in the
+    // bounds check)
     const bf16* vb = (const bf16*)p.v + (((int64_t)b * p.L + p.t0) * p.Hv + hv) * KD;
     const int rowb = p.Hv * KD * 2, vofs = 4 * q * rowb + (vc0 + r16) * 2;
     uint16_t v[4][4];
@@ -1354,7 +1356,7 @@ __global__ __launch_bounds__(512) void k_chain_cols(const PF p) {
 #pragma unroll
       for (int rt = 0; rt < NB; ++rt)
 #pragma unroll
-        for (int ii = 0; ii < 4; ++ii) v[rt][ii] = __builtin_amdgcn_raw_buffer_load_b16(rs, vofs, (16 * rt + ii) * rowb, 0);
+        for (int ii = 0; ii < 4; ++ii) v[rt][ii] = __builtin_amdgcn_raw_buffer_load_b16(rs, vofs + (16 * rt + ii) * rowb, 0, 0);
     };
     load_v(0);
     lds_barrier();   // chunks 0 and 1, the flags
