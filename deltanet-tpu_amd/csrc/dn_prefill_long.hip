@@ -536,33 +536,37 @@ __global__ __launch_bounds__(512) void k_prepass_long(const PF p, const PL px) {
     float tot[8];
 #pragma unroll
     for (int a = 0; a < 8; ++a) tot[a] = X[(16 * a + 15) * XP + tid] + Y[(16 * a + 15) * XP + tid];
-    float acc = 0.f, lg[8];
+    float acc = 0.f, rl[9], span[8];
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
-      const float lsa = X[(16 * a) * XP + tid] + Y[(16 * a) * XP + tid];
-      lg[a] = acc + lsa;   // chunk-global Lambda at the first token of block a
-      Ea[a * KD + tid] = fast_exp2(lg[a]);
+      const int sa = 16 * a, ea = sa + 15;
+      const float lsa = X[sa * XP + tid] + Y[sa * XP + tid];
+      // span of the block after its first token: Lambda(sa) - Lambda(ea) >= 0
+      span[a] = (X[sa * XP + tid] - X[ea * XP + tid]) + (Y[sa * XP + tid] - Y[ea * XP + tid]);
+      // Lambda at the first token of block a relative to the chunk's first
+      // token (not a difference of chunk-global values: a large decay at the
+      // chunk's first token would cancel in it)
+      rl[a] = a == 0 ? 0.f : rl[a] + lsa;
+      rl[a + 1] = rl[a] - span[a];
+      Ea[a * KD + tid] = fast_exp2(acc + lsa);   // chunk-global Lambda at the first token of block a
+      Mid0[a * KD + tid] = fast_exp2(lsa);
       acc += tot[a];
     }
     g_dv[tid] = fast_exp2(acc);   // e^{Lambda_end}
     // chunk reference row 64: every off-diagonal A / M entry factors as
     // (row i: e^{Lambda_i - Lambda_64}) (column j: e^{Lambda_64 - Lambda_j}),
     // both within 2^{+-100} when the spans on either side of row 64 are
-    bool wide = (lg[0] - lg[4] > kDiagSafeLog2) || (lg[4] - acc > kDiagSafeLog2);
+    bool wide = (rl[0] - rl[4] > kDiagSafeLog2) || (rl[4] - rl[8] > kDiagSafeLog2);
 #pragma unroll
-    for (int a = 0; a < 8; ++a) Gt[a * KD + tid] = fast_exp2(lg[a] - lg[4]);
+    for (int a = 0; a < 8; ++a) Gt[a * KD + tid] = fast_exp2(rl[a] - rl[4]);
     acc = 0.f;
 #pragma unroll
     for (int a = 7; a >= 0; --a) { Sa[a * KD + tid] = fast_exp2(acc); acc += tot[a]; }
 #pragma unroll
     for (int a = 0; a < 8; ++a) {
       Ftab[a * KD + tid] = fast_exp2(tot[a]);
-      Mid0[a * KD + tid] = fast_exp2(X[(16 * a) * XP + tid] + Y[(16 * a) * XP + tid]);
-      // span of the block after its first token: Lambda(sa) - Lambda(ea) >= 0
-      const int sa = 16 * a, ea = sa + 15;
-      const float span = (X[sa * XP + tid] - X[ea * XP + tid]) + (Y[sa * XP + tid] - Y[ea * XP + tid]);
-      Fa[a * KD + tid] = fast_exp2(-span);
-      const bool un = __any(span > kDiagSafeLog2);
+      Fa[a * KD + tid] = fast_exp2(-span[a]);
+      const bool un = __any(span[a] > kDiagSafeLog2);
       if (l == 0) unsafe_part[w][a] = un;
       wide = wide || un;
     }
