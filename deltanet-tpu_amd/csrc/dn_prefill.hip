@@ -1222,6 +1222,10 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
       __builtin_amdgcn_sched_barrier(0);
       load_q(c + 1);
       lds_barrier();   // 2
+      // (nothing of w v moves up: with one gate per token the compiler took its
+      // wait for the gate above the loads of q: 16384 tokens of 17 heads, 634
+      // against 555 us of scan; with a gate per channel no difference)
+      if constexpr (!WCH) __builtin_amdgcn_sched_barrier(0);
       put_wv(c + 1);   // (the recurrence has read chunk c's)
       load_v(c + 2);
       lds_barrier();   // 3
