@@ -1652,24 +1652,48 @@ bool scalar_gates(const dn_prefill_args* a) {
          a->w_chans == 1 && !a->fuse_prologue;
 }
 
-// The long form where its scan, half the steps at 1.4 us against 1.3 us each,
-// outweighs its prepass, whose cost grows with the heads H and, less, with the
-// value heads G of each: `width` = H (5 + 2 G).  Measured (64-token scan / long
-// form, us): width 9-36, 2048 tokens 65 / 77, 4096 104 / 97, 16384 350 / 230;
-// width 72, 4096 tokens 112 / 115, 16384 638 / 536; width 104-112, 4096 tokens
-// 120-149 / 180-190, 16384 650-755 / 637-733; width 224, 16384 tokens
-// 965 / 1191; fp32 width 9-36, 2048 tokens 123 / 163, 16384 800 / 525.  With
-// scalar gates both prepasses are the smaller by far: width 14-28, 2048 tokens
-// 56 / 68, 4096 94 / 90, 16384 316 / 218-263; width 56, 4096 tokens 94 / 96, 16384
-// 337 / 479.
+// The long form where its scan, half the steps of 1.4 us against 1.1-1.3 us
+// each, outweighs its prepass.  That prepass runs one workgroup per CU, so it
+// costs whole rounds of 256 units (head, 128 tokens), 30 us with scalar gates
+// and 40-60 with channel-wise ones: at one round the line is a length, at more
+// rounds only long sequences of few heads are left.  Both forms measured, long
+// form's time / scan's:
+//   one round: channel gates, 1 value head per head 2560 tokens 1.00-1.04,
+//     3072 0.94-0.99; 2 value heads 3072 0.99-1.04, 4096 0.88-0.93 (8 heads
+//     1.04); 4 value heads 4096 1.06-1.13, 6144 0.92-0.97 (4 heads 1.03 at
+//     5120); fp32 2560 1.06, 3584 0.92 / 3584 1.02, 5120 0.88 / 5120 1.04,
+//     6144 0.97; scalar 4608 1.02, 6144 0.95 (6 heads 1.03 at 5120) / 6144
+//     0.95-1.01 / 8192 0.97-1.00
+//   more: channel gates 5-8 heads 6144 tokens 1.00-1.16, 8192 0.90-1.13,
+//     12288 0.93-1.07; 10-13 heads 8192 1.02-1.26, 12288 0.91-1.01 (4 value
+//     heads: 12288 1.00-1.12, 16384 0.93-0.99); 16 heads from 12288 0.98-1.06,
+//     17 and more 1.00-1.4.  fp32 6-8 heads 6144 1.01-1.28, 8192 0.91-1.09,
+//     16384 0.87-1.00; 11 heads and more 1.03-1.5.
+//   scalar gates, more: 1-2 heads 0.74-1.00 throughout; 3-4 heads in the second
+//     round 12288 0.99-1.04, 16384 0.92-0.95, 4 heads in the third 1.06 and 5 to
+//     12 heads 1.0-1.8; from 1536 units, where the scan's operands no longer fit
+//     the 256 MB cache, 3-5 heads 0.88-0.96, 6 heads 0.98-1.02, 7 and more
+//     1.00-1.2.
+// `width` = heads (5 + 2 G) weighs a head with its G value heads.
 Form form_of(const dn_prefill_args* a) {
-  const bool sc = scalar_gates(a);
+  const bool sc = scalar_gates(a), bf = a->precision == 0;
   const int64_t G = a->gates_at_hv ? 1 : a->Hv / a->Hk;
-  const int64_t width = (int64_t)a->B * (a->gates_at_hv ? a->Hv : a->Hk) * (5 + 2 * G);
-  int64_t least = INT64_MAX;   // tokens from which the long form is the faster
-  if (sc) least = width <= 28 ? 3584 : INT64_MAX;
-  else least = width <= 40 ? 3072 : (width <= 75 ? 8192 : (width <= 115 ? 16384 : INT64_MAX));
-  if (a->nt >= least) return kLong;
+  const int64_t heads = (int64_t)a->B * (a->gates_at_hv ? a->Hv : a->Hk);
+  const int64_t width = heads * (5 + 2 * G);
+  const int64_t units = heads * ((a->nt + 127) / 128), rounds = (units + 255) / 256;
+  bool lng;
+  if (sc) {
+    const bool most = rounds == 1 ? width <= 40
+                                  : (rounds == 2 && a->nt >= 16384 && width <= 28 && G <= 2) || (units >= 1536 && width <= 45);
+    lng = a->nt >= 4096 + 1024 * G && (width <= 14 || most);
+  } else if (rounds == 1) {
+    lng = width <= (G <= 2 ? 70 : 40) && a->nt >= 2048 + (bf ? 768 : 1024) * G;
+  } else if (width <= 56 && G <= 2) {
+    lng = a->nt >= 8192;
+  } else {
+    lng = width <= (bf ? 112 : 75) && a->nt >= (bf && G <= 2 ? 12288 : 16384);
+  }
+  if (lng) return kLong;
   return sc ? kScalar : kScan;
 }
 

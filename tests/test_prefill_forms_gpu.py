@@ -59,9 +59,13 @@ def test_column_tiles(B, Hk, Hv, scalar, v_dt, fuse):
     run(7 * B + Hv, B, 77, Hk, Hv, scalar=scalar, precision="bf16", v_dt=v_dt, fuse=fuse)
 
 
-# either side of the length from which few heads take the affine form
+# either side of the lengths from which few heads take the affine form (3584
+# tokens here, 4096 in fp32, 5120 with scalar gates), and its chunks' edges
 @pytest.mark.parametrize("L,scalar,precision", [(3071, False, "bf16"), (3072, False, "bf16"), (3200, False, "fp32"),
                                                 (3073, False, "fp32"), (3583, True, "bf16"), (3584, True, "bf16"),
-                                                (8191, True, "bf16"), (8193, True, "bf16")])
+                                                (8191, True, "bf16"), (8193, True, "bf16"), (3583, False, "bf16"),
+                                                (3584, False, "bf16"), (3585, False, "bf16"), (4095, False, "fp32"),
+                                                (4096, False, "fp32"), (4097, False, "fp32"), (5119, True, "bf16"),
+                                                (5120, True, "bf16")])
 def test_long_form_edges(L, scalar, precision):
     run(L, 1, L, 1, 2, scalar=scalar, precision=precision, init=False)

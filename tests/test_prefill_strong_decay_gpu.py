@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 # of 2e6; float32 prefill is within 1e-6 of the oracle otherwise, 4e-6 the bound
 # of both.  A decay that took 2e6 in one float32 word would be off by 2^-3.
 @pytest.mark.parametrize("scalar", [True, False])
-@pytest.mark.parametrize("L,chunk", [(200, 64), (3200, 128)])
+@pytest.mark.parametrize("L,chunk", [(200, 64), (4200, 128)])
 def test_large_decay_at_chunk_starts(scalar, L, chunk):
     rng = np.random.default_rng(L)
     rn = rng.standard_normal

@@ -43,8 +43,8 @@ def run(B, L, Hk, Hv, scalar, v_dt, precision, behind):
     (2, 16, 32, True, torch.bfloat16, "bf16", 2),
     (1, 2, 4, False, torch.bfloat16, "bf16", 2),
     (1, 2, 4, False, torch.float32, "fp32", 2),
-    (1, 1, 2, False, torch.bfloat16, "bf16", 50),
-    (1, 1, 2, True, torch.bfloat16, "bf16", 58),
+    (1, 1, 2, False, torch.bfloat16, "bf16", 56),
+    (1, 1, 2, True, torch.bfloat16, "bf16", 96),
 ])
 def test_memory_behind_the_inputs(tail, B, Hk, Hv, scalar, v_dt, precision, chunks):
     L = 64 * chunks + tail
