@@ -44,9 +44,10 @@ struct PF {
 
 // The 128-token affine form (dn_prefill_long.hip): its workspace for `units`
 // (batch, exec head, 128-token chunk) units of value width Vp, and one token
-// block over it (p's flags, dvec and 128-token NCb set).
+// block over it (p's flags, dvec and 128-token NCb set), one decay and one b per
+// token as plain products if `scalar_phases`.
 size_t long_workspace(size_t units, int Vp, bool bf);
-hipError_t long_prefill(const PF& p, char* ws, hipStream_t st, bool bf, int qk_dt, bool v_bf16);
+hipError_t long_prefill(const PF& p, char* ws, hipStream_t st, bool bf, int qk_dt, bool v_bf16, bool scalar_phases);
 
 // Records the message for dn_last_error() and returns `code`.
 int set_error(int code, const char* msg);

@@ -1640,15 +1640,18 @@ int chain_tiles() {
 }
 
 int g_prepass_scalar = -1;   // -1: unread; 0: general path forced (DN_PREPASS_SCALAR=0, measurements)
-
-// One decay, one b and one w per (token, head) with bf16 q / k in precision
-// "bf16" (the Gated DeltaNet form) runs the scalar-gate kernels.
-bool scalar_gates(const dn_prefill_args* a) {
+bool prepass_scalar() {
   if (g_prepass_scalar < 0) {
     const char* e = getenv("DN_PREPASS_SCALAR");
     g_prepass_scalar = (e && atoi(e) == 0) ? 0 : 1;
   }
-  return g_prepass_scalar == 1 && a->precision == 0 && a->qk_dtype == DN_BF16 && a->g_chans == 1 && a->b_chans == 1 &&
+  return g_prepass_scalar == 1;
+}
+
+// One decay, one b and one w per (token, head) with bf16 q / k in precision
+// "bf16" (the Gated DeltaNet form) runs the scalar-gate kernels.
+bool scalar_gates(const dn_prefill_args* a) {
+  return prepass_scalar() && a->precision == 0 && a->qk_dtype == DN_BF16 && a->g_chans == 1 && a->b_chans == 1 &&
          a->w_chans == 1 && !a->fuse_prologue;
 }
 
@@ -1819,7 +1822,7 @@ int prefill_run(const dn_prefill_args* a, char* ws, size_t workspace_bytes, int 
     p.init = first ? a->init_state : carry;
     p.fin = carry;
     const bool v_bf16 = a->v_dtype == DN_BF16;
-    const hipError_t e = form == kLong ? long_prefill(p, ws + Lw.lng, st, bf, a->qk_dtype, v_bf16)
+    const hipError_t e = form == kLong ? long_prefill(p, ws + Lw.lng, st, bf, a->qk_dtype, v_bf16, prepass_scalar())
                                        : dispatch(p, st, bf, a->qk_dtype, v_bf16, form == kScalar);
     if (e != hipSuccess) return set_error(DN_E_LAUNCH, hipGetErrorString(e));
   }

@@ -1499,12 +1499,12 @@ __global__ __launch_bounds__(512) void k_chain_long(const PF p, const PL px) {
 }
 
 template <bool BF, class TIn, class TV>
-hipError_t launch_long(const PF& p, const PL& px, hipStream_t st) {
+hipError_t launch_long(const PF& p, const PL& px, hipStream_t st, bool scalar_phases) {
   prof_mark(0, st, false);
   const dim3 grid(p.B * p.Hx * p.NCb), blk(512);
   bool sc = false;   // one decay and one b per token: phases 1-3 are plain products
   if constexpr (BF && std::is_same<TIn, bf16>::value) {
-    sc = p.g_c == 1 && p.b_c == 1 && !p.fuse;
+    sc = scalar_phases && p.g_c == 1 && p.b_c == 1 && !p.fuse;
     if (sc) hipLaunchKernelGGL((k_prepass_long<true, bf16, TV, true>), grid, blk, 0, st, p, px);
   }
   if (!sc) hipLaunchKernelGGL((k_prepass_long<BF, TIn, TV, false>), grid, blk, 0, st, p, px);
@@ -1518,15 +1518,16 @@ hipError_t launch_long(const PF& p, const PL& px, hipStream_t st) {
 }
 
 template <bool BF, class TIn>
-hipError_t dispatch_v(const PF& p, const PL& px, hipStream_t st, bool v_bf16) {
-  return v_bf16 ? launch_long<BF, TIn, bf16>(p, px, st) : launch_long<BF, TIn, float>(p, px, st);
+hipError_t dispatch_v(const PF& p, const PL& px, hipStream_t st, bool v_bf16, bool scalar_phases) {
+  return v_bf16 ? launch_long<BF, TIn, bf16>(p, px, st, scalar_phases)
+                : launch_long<BF, TIn, float>(p, px, st, scalar_phases);
 }
 
 template <bool BF>
-hipError_t dispatch_qk(const PF& p, const PL& px, hipStream_t st, int qk_dt, bool v_bf16) {
-  if (qk_dt == DN_BF16) return dispatch_v<BF, bf16>(p, px, st, v_bf16);
-  if (qk_dt == DN_F16) return dispatch_v<BF, f16>(p, px, st, v_bf16);
-  return dispatch_v<BF, float>(p, px, st, v_bf16);
+hipError_t dispatch_qk(const PF& p, const PL& px, hipStream_t st, int qk_dt, bool v_bf16, bool scalar_phases) {
+  if (qk_dt == DN_BF16) return dispatch_v<BF, bf16>(p, px, st, v_bf16, scalar_phases);
+  if (qk_dt == DN_F16) return dispatch_v<BF, f16>(p, px, st, v_bf16, scalar_phases);
+  return dispatch_v<BF, float>(p, px, st, v_bf16, scalar_phases);
 }
 
 // The workspace arrays from `ws` on (nullptr: only their size), for `units`
@@ -1565,10 +1566,11 @@ size_t long_workspace(size_t units, int Vp, bool bf) {
   return n;
 }
 
-hipError_t long_prefill(const PF& p, char* ws, hipStream_t st, bool bf, int qk_dt, bool v_bf16) {
+hipError_t long_prefill(const PF& p, char* ws, hipStream_t st, bool bf, int qk_dt, bool v_bf16, bool scalar_phases) {
   size_t n = 0;
   const PL px = long_layout(ws, (size_t)p.B * p.Hx * p.NCb, p.Vp, bf, &n);
-  return bf ? dispatch_qk<true>(p, px, st, qk_dt, v_bf16) : dispatch_qk<false>(p, px, st, qk_dt, v_bf16);
+  return bf ? dispatch_qk<true>(p, px, st, qk_dt, v_bf16, scalar_phases)
+            : dispatch_qk<false>(p, px, st, qk_dt, v_bf16, scalar_phases);
 }
 
 }  // namespace dn
