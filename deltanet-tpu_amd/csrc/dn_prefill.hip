@@ -1718,8 +1718,9 @@ void launch_chain(const PF& p, hipStream_t st) {
   auto go = [&](auto wch) {
     constexpr bool W = decltype(wch)::value;
     if constexpr (BF) {
-      if (ntl == 4) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 4>), grid, blk, 0, st, p);
-      else if (ntl == 2) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 2>), grid, blk, 0, st, p);
+      if constexpr (!(SC && std::is_same<TV, bf16>::value))
+        if (ntl == 4) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 4>), grid, blk, 0, st, p);
+      if (ntl == 2) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 2>), grid, blk, 0, st, p);
     }
     if (ntl == 1) hipLaunchKernelGGL((k_chain<BF, SC, W, TV, 1>), grid, blk, 0, st, p);
   };
