@@ -416,7 +416,11 @@ def _decode_gate(t, B, Hk, Hv, last, name):
 _STATE_DT = {torch.float32: _lib.DN_F32, torch.bfloat16: _lib.DN_BF16}
 _EMPTY = torch.empty
 _SCALE = 1.0 / math.sqrt(128)
-_raw_stream = torch._C._cuda_getCurrentRawStream
+try:   # (a torch built without GPU support lacks it; the package imports there too)
+    from torch._C import _cuda_getCurrentRawStream as _raw_stream
+except ImportError:
+    def _raw_stream(dev):
+        return torch.cuda.current_stream(dev).cuda_stream
 
 
 def _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, steps):

@@ -4,6 +4,9 @@ the GPU bit-identical results over the forms it takes and no call taken that
 the general path reads differently."""
 
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -19,6 +22,24 @@ def test_packed_block_has_the_struct_layout():
         setattr(a, name, v)
         vals.append(v)
     assert _lib.DECODE_PACK(*vals) == bytes(a)
+
+
+def test_imports_without_gpu_support():
+    code = """
+import torch
+for name in [n for n in dir(torch._C) if n.startswith("_cuda_")]:
+    delattr(torch._C, name)
+import deltanet_tpu_amd
+try:
+    deltanet_tpu_amd.gdn2_decode_step(*[torch.zeros(1, 2, 128)] * 6, torch.zeros(1, 2, 128, 128))
+except RuntimeError as e:
+    assert "runs only on a ROCm GPU" in str(e), e
+else:
+    raise SystemExit("no error")
+"""
+    r = subprocess.run([sys.executable, "-c", code], env={**os.environ, "PYTHONPATH": os.path.dirname(os.path.dirname(_lib.__file__))},
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
 
 
 def operands(B, L, Hk, Hv, rank, gates, qdt, sdt, dev="cuda:0"):
