@@ -118,8 +118,8 @@ def packed_decode():
     the argument block as packed bytes."""
     global _packed
     if _packed is None:
-        load_library()
-        lib = ctypes.CDLL(LIB_PATH)   # the same library; function objects of its own
+        lib = load_library()
+        lib = ctypes.CDLL(lib._name, handle=lib._handle)   # the library loaded already; function objects of its own
         one, many = lib.dn_decode_step, lib.dn_decode_steps
         one.argtypes, one.restype = [ctypes.c_char_p, _c_ptr], ctypes.c_int
         many.argtypes, many.restype = [ctypes.c_char_p, _c_i32, _c_ptr], ctypes.c_int

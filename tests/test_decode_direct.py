@@ -5,6 +5,7 @@ the general path reads differently."""
 
 import ctypes
 import os
+import shutil
 import subprocess
 import sys
 
@@ -22,6 +23,19 @@ def test_packed_block_has_the_struct_layout():
         setattr(a, name, v)
         vals.append(v)
     assert _lib.DECODE_PACK(*vals) == bytes(a)
+
+
+def test_packed_entries_are_the_loaded_library(tmp_path, monkeypatch):
+    # a library rebuilt under a running process stays the one that was loaded
+    # (its error text and its caches are its own)
+    lib = _lib.load_library()
+    other = tmp_path / _lib.LIB_NAME
+    shutil.copy(_lib.LIB_PATH, other)
+    monkeypatch.setattr(_lib, "LIB_PATH", str(other))
+    monkeypatch.setattr(_lib, "_packed", None)
+    address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+    one, many = _lib.packed_decode()
+    assert address(one) == address(lib.dn_decode_step) and address(many) == address(lib.dn_decode_steps)
 
 
 def test_imports_without_gpu_support():
