@@ -423,7 +423,7 @@ except ImportError:
         return torch.cuda.current_stream(dev).cuda_stream
 
 
-def _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, steps):
+def _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, steps, tau=1000.0):
     """The decode call for operands the kernels read as they are: plain
     contiguous tensors of kernel types on one GPU, gates at the key or value
     heads.  None for anything else (including whatever is to be refused): the
@@ -499,6 +499,8 @@ def _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype
         scale = _SCALE
     elif type(scale) is not float:
         return None
+    if type(tau) is not float:
+        float(tau)   # (unused without the guard, refused like in the general path)
     if out_state is None:
         out_state = _EMPTY(ss, dtype=state_dtype or torch.float32, device=q.device)
     elif (type(out_state) is not T or out_state.shape != ss or _STATE_DT.get(out_state.dtype) != sd_out
@@ -535,7 +537,7 @@ def gdn2_decode_step(
     itself for an in-place update when the dtypes match.
     """
     if not stability_guard:
-        r = _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, False)
+        r = _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, False, stability_tau)
         if r is not None:
             return r
     if stability_guard and isinstance(stability_tau, (int, float)) and not stability_tau > 0:
@@ -686,7 +688,7 @@ def gdn2_decode_steps(
     those with the guard) round it after every token as chained calls do.
     """
     if not stability_guard:
-        r = _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, True)
+        r = _decode_direct(q, k, v, g, b, w, state, reset, scale, qk_l2norm, state_dtype, out_state, True, stability_tau)
         if r is not None:
             return r
     if stability_guard and isinstance(stability_tau, (int, float)) and not stability_tau > 0:

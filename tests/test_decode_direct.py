@@ -132,3 +132,12 @@ def test_what_the_direct_path_leaves(monkeypatch):
     assert direct(base, reset=torch.tensor([True])) is None and direct(base, reset=True) is None
     assert direct(base, state_dtype="bf16") is None
     assert direct(base, out_state=torch.empty_like(st, dtype=torch.bfloat16)) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tau", [None, "large", [1000.0]])
+def test_a_tau_that_is_no_number_is_refused(tau):
+    for T, fn in ((1, gdn2_decode_step), (3, gdn2_decode_steps)):
+        args = operands(2, T, 2, 4, 4, ("channel",) * 3, torch.bfloat16, torch.float32)
+        with pytest.raises((TypeError, ValueError)):
+            fn(*args, stability_tau=tau)
