@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import torch
 
-from .gdn2 import chunk_gdn2, gdn2_decode_step
+from .gdn2 import _decode_step_general, chunk_gdn2, gdn2_decode_step
 
 __all__ = [
     "chunk_gdn", "gdn_decode_step",
@@ -112,18 +112,19 @@ def kda_decode_step(q, k, v, g, beta, state, *, reset=None, scale=None, qk_l2nor
                             qk_l2norm=qk_l2norm, state_dtype=state_dtype)
 
 
+# (a gate of one head takes the general path of gdn2_decode_step: gla and delta go there at once)
 def _const_decode_gate(ref, value):
     return torch.full((ref.shape[0], 1), value, dtype=torch.float32, device=ref.device)
 
 
 def gla_decode_step(q, k, v, g, state, *, reset=None, scale=None, qk_l2norm=False, state_dtype=None):
     """GLA decode step (b = 0, w = 1); variants.py:364-389."""
-    return gdn2_decode_step(q, k, v, g, _const_decode_gate(q, 0.0), _const_decode_gate(q, 1.0), state,
-                            reset=reset, scale=scale, qk_l2norm=qk_l2norm, state_dtype=state_dtype)
+    return _decode_step_general(q, k, v, g, _const_decode_gate(q, 0.0), _const_decode_gate(q, 1.0), state,
+                                reset=reset, scale=scale, qk_l2norm=qk_l2norm, state_dtype=state_dtype)
 
 
 def delta_rule_decode_step(q, k, v, beta, state, *, reset=None, scale=None, qk_l2norm=False, state_dtype=None):
     """DeltaNet decode step (g = 0); variants.py:392-417."""
     beta = _validate_decode_beta(beta)
-    return gdn2_decode_step(q, k, v, _const_decode_gate(q, 0.0), beta, beta, state, reset=reset,
-                            scale=scale, qk_l2norm=qk_l2norm, state_dtype=state_dtype)
+    return _decode_step_general(q, k, v, _const_decode_gate(q, 0.0), beta, beta, state, reset=reset,
+                                scale=scale, qk_l2norm=qk_l2norm, state_dtype=state_dtype)

@@ -12,7 +12,8 @@ import sys
 import pytest
 import torch
 
-from deltanet_tpu_amd import _lib, gdn2, gdn2_decode_step, gdn2_decode_steps
+from deltanet_tpu_amd import (_lib, delta_rule_decode_step, gdn2, gdn2_decode_step, gdn2_decode_steps,
+                              gla_decode_step)
 
 
 def test_packed_block_has_the_struct_layout():
@@ -36,6 +37,17 @@ def test_packed_entries_are_the_loaded_library(tmp_path, monkeypatch):
     address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
     one, many = _lib.packed_decode()
     assert address(one) == address(lib.dn_decode_step) and address(many) == address(lib.dn_decode_steps)
+
+
+def test_variants_with_constant_gates_go_to_the_general_path(monkeypatch):
+    # gla and delta pass gates of one head, which the direct path never takes
+    tried = []
+    monkeypatch.setattr(gdn2, "_decode_direct", lambda *a: tried.append(a))
+    z = torch.zeros(1, 2, 128)
+    for step, args in ((gla_decode_step, (z, z, z, z)), (delta_rule_decode_step, (z, z, z, torch.zeros(1, 2)))):
+        with pytest.raises(RuntimeError, match="runs only on a ROCm GPU"):
+            step(*args, torch.zeros(1, 2, 128, 128))
+    assert not tried
 
 
 def test_imports_without_gpu_support():
