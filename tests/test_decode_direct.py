@@ -84,6 +84,21 @@ def operands(B, L, Hk, Hv, rank, gates, qdt, sdt, dev="cuda:0"):
     return q, k, v, *out, (0.1 * rn(B, Hv, 128, 128)).to(sdt)
 
 
+def tried(monkeypatch, fn, args, kw):
+    """The call's results, and whether the direct path took it."""
+    direct, seen = gdn2._decode_direct, []
+
+    def record(*a):
+        seen.append(direct(*a))
+        return seen[-1]
+
+    with monkeypatch.context() as m:
+        m.setattr(gdn2, "_decode_direct", record)
+        got = fn(*args, **kw)
+    assert len(seen) == 1
+    return got, seen[0] is not None
+
+
 FORMS = [("channel",) * 3, ("scalar",) * 3, ("one", "flat", "value"), ("flat channel", "value", "channel"),
          ("broadcast", "channel", "broadcast")]
 
@@ -102,7 +117,8 @@ def test_step_direct_equals_general(gates, rank, Hk, Hv, monkeypatch):
         args = operands(B, 1, Hk, Hv, rank, gates, qdt, sdt)
         reset = torch.tensor([True, False, True], device="cuda:0")
         kw = dict(reset=reset, qk_l2norm=True, state_dtype=torch.bfloat16 if out_dt else None)
-        got = gdn2_decode_step(*args, **kw)
+        got, taken = tried(monkeypatch, gdn2_decode_step, args, kw)
+        assert taken == (Hk > 1 and "broadcast" not in gates)   # gates of one head are left
         with monkeypatch.context() as m:
             m.setattr(gdn2, "_decode_direct", lambda *a: None)
             want = gdn2_decode_step(*args, **kw)
@@ -119,7 +135,8 @@ def test_steps_direct_equals_general(T, gates, monkeypatch):
         args = operands(2, T, 2, 4, 4, gates, qdt, sdt)
         for reset in (None, torch.rand(2, T, device="cuda:0") < 0.3, torch.tensor([True, False], device="cuda:0")):
             kw = dict(reset=reset, scale=0.1, state_dtype=sdt)
-            got = gdn2_decode_steps(*args, **kw)
+            got, taken = tried(monkeypatch, gdn2_decode_steps, args, kw)
+            assert taken == (reset is None or reset.dim() == 2)   # a reset per row is left
             with monkeypatch.context() as m:
                 m.setattr(gdn2, "_decode_direct", lambda *a: None)
                 want = gdn2_decode_steps(*args, **kw)
