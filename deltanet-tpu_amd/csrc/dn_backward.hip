@@ -151,8 +151,8 @@ __device__ __forceinline__ float4 cvt4(const u32x4& x, int dt) {
 // Held at 128 channels, the copies of chunk_gdn's three gates and of their
 // gradients were 14 passes over a (token, head, 128) fp32 array.  4096 tokens,
 // 32 heads: preparation 93 to 39 us, the gates' last step 55 to 13; with the
-// decay factors formed once per pair (k_bw_intra, k_bw_dqk), k_bw_intra 361 to
-// 293 and k_bw_dqk 260 to 219.
+// decay factors formed once per pair (k_bw_intra, k_bw_dqk), k_bw_intra 366 to
+// 262 and k_bw_dqk 262 to 214.
 constexpr int kGateParts[3] = {4, 8, 1};
 __device__ __forceinline__ u32x4 ld_gate4(const float* g, int64_t row, int chans, int c) {
   if (chans == 1) return u32x4{__builtin_bit_cast(uint32_t, g[row]), 0u, 0u, 0u};
@@ -262,9 +262,15 @@ template <> struct Op<true> {
 // ---------------------------------------------------------------------------
 // k_bw_intra
 // ---------------------------------------------------------------------------
-template <bool BF>
+// SC: one decay per (token, head).  A template argument, since the kernel is at
+// its 256 VGPRs: with both forms behind a branch it spilled 19 of them (float32
+// 5), one decay per channel alone spills 11 (1), one per token none.  4096
+// tokens, 32 heads, one per token 297 us behind the branch, 262 apart; 2 x 2048
+// tokens, 16 heads, one per channel 161 and 156, float32 2048 x 24 122 and 117.
+template <bool BF, bool SC>
 __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   using O = Op<BF>;
+  constexpr int GC = SC ? 1 : KD;   // channels of the decay
   __shared__ float sG[BC][KP];
   __shared__ float sA[BC][CP];   // A, then T
   __shared__ float sM[BC][CP];
@@ -296,7 +302,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
       ng[it] = u32x4{0u, 0u, 0u, 0u};
       if (t0 + i < p.L) {
         nk[it] = ld4g(p.k + row_in(p, bb, t0 + i, h, p.qk_hd) + 4 * c4);
-        ng[it] = ld_gate4(p.g, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, p.g_c, 4 * c4);
+        ng[it] = ld_gate4(p.g, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, GC, 4 * c4);
       }
     }
   };
@@ -321,7 +327,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   for (int it = 0; it < SIT; ++it) {
     // a thread holds 4 consecutive tokens x 4 channels
     const int c4 = tid % (KD / 4), i = 4 * (tid / (KD / 4)) + it;
-    const float4 gv = gate4_of(ng[it], p.g_c);
+    const float4 gv = gate4_of(ng[it], GC);
     kst[it] = nk[it];
     *reinterpret_cast<float4*>(&sG[i][4 * c4]) =
         make_float4(gv.x * kLog2e, gv.y * kLog2e, gv.z * kLog2e, gv.w * kLog2e);
@@ -456,7 +462,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
     const int I = (0xfe4e9 >> (2 * tt)) & 3, J = (0x9e410 >> (2 * tt)) & 3;
     const bool diag = J == I;
     float resA[4], resM[4];
-    if (p.g_c == 1) {
+    if constexpr (SC) {
       // one decay for every channel: plain products, scaled once per element
       const int i = 16 * I + l16, j = 16 * J + l16;
       const float* kj = p.k + row_in(p, bb, t0 + j < p.L ? t0 + j : 0, h, p.qk_hd);
@@ -1409,6 +1415,9 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
 // span allows, else use e^{G_i-G_j} per element.
 // Wave w owns the 16 channels 16 (w % 2) .. and the 16-row block w / 2;
 // lanes hold rows 4q..4q+3 of it.  About 73 KB of LDS: two workgroups per CU.
+// SC: one decay per (token, head), whose products need no factors (99 VGPRs,
+// 109 with one per channel; 4096 tokens, 32 heads 224 us behind a branch, 213
+// apart).
 // ---------------------------------------------------------------------------
 constexpr int HC = KD / 4;      // channels per k_bw_dqk workgroup
 constexpr int NQ = KD / HC;     // k_bw_dqk workgroups per unit
@@ -1426,6 +1435,7 @@ __device__ __forceinline__ void mma_half(f32x4& acc, const float* a, const float
   }
 }
 
+template <bool SC>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_bw_dqk(BW p) {
   __shared__ float sQ[BC][HP], sK[BC][HP], sB[BC][HP], sG[BC][HP];
   __shared__ float sdM[BC][CP], sdA[BC][CP];
@@ -1484,10 +1494,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     *reinterpret_cast<float4*>(&sdA[i][4 * c4]) = ld4g(p.dAw + (int64_t)u * CC + i * BC + 4 * c4);
   }
   lds_barrier();
-  // one decay for every channel: dM and dA take their factors e^{G_i - G_j}
-  // once, and every product below is a plain one
-  const bool sc = p.g_c == 1;
-  if (sc) {
+  if constexpr (SC) {
+    // dM and dA take their factors e^{G_i - G_j} once, and every product below
+    // is a plain one
 #pragma unroll
     for (int it = 0; it < CC / 4 / NT; ++it) {
       const int idx = tid + NT * it, i = idx / (BC / 4), c4 = idx % (BC / 4);
@@ -1522,8 +1531,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int m = 16 * I, m2 = 16 * I + 15;
     const float gm = sG[m][rl], gm2 = sG[m2][rl];
     // G restarts at document starts: the in-block factors need one document
-    const bool inblk = !sc && sseg[m] == sseg[m2] && __all(gm - gm2 <= 64.f);
-    if (sc) {
+    const bool inblk = !SC && sseg[m] == sseg[m2] && __all(gm - gm2 <= 64.f);
+    if constexpr (SC) {
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
         float xm[8], xa[8], xk[8], ym[8], ya[8], yq[8], yb[8];
@@ -1642,7 +1651,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       const int i = 16 * I + ii;
       const float gi = sG[i][rl];
       float dq = 0.f, dbeta = 0.f, dk = 0.f;
-      if (!inblk && !sc) {
+      if (!inblk && !SC) {
         // pairs inside block I, e^{G_i - G_j} per element
 #pragma unroll
         for (int jj = 0; jj < 16; ++jj) {
@@ -1657,10 +1666,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         }
       }
       const float eg = scar[i] ? ex2(gi) : 0.f;
-      const float fi = sc ? 1.f : ex2(gi - gm);
+      const float fi = SC ? 1.f : ex2(gi - gm);
       dq += eg * rq[Ib][e] + oq[e] * fi;
       dbeta += -eg * rb[Ib][e] + ob[e] * fi;
-      dk += sc ? ok_[e] : ok_[e] * ex2(gm2 - gi);
+      dk += SC ? ok_[e] : ok_[e] * ex2(gm2 - gi);
       if (inblk) dk += okb[e] * __builtin_amdgcn_exp2f(gm - gi);   // <= 2^64 (the block's span)
       const float dkc = slast[i] ? ex2(glast - gi) * rk[Ib][e] : 0.f;
       const float kv = sK[i][rl], qv = sQ[i][rl], bv = sB[i][rl], dmii = sdM[i][i];
@@ -1732,7 +1741,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int t = t0 + 4 * sg + e;
-      if (p.g_c == 1) {   // the quarter's 32 channels: one 32-lane half
+      if constexpr (SC) {   // the quarter's 32 channels: one 32-lane half
         const float sum = lane_sum<HC>(dgv[e]);
         if (ch == 0 && t < p.L) p.dg[row_of(p, bb, t, h) / KD * kGateParts[0] + part] = sum;
       } else if (t < p.L) {
@@ -2199,7 +2208,15 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
   if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       ncu <= 0)
     ncu = 256;
-  auto intra_grid = [&](unsigned n) { return dim3(std::min(n, (unsigned)ncu)); };
+  // one decay per (token, head), or one per channel
+  const bool sc = p.g_c == 1;
+  auto launch_intra = [&](unsigned n) {
+    const dim3 grid(std::min(n, (unsigned)ncu)), blk(NT);
+    if (p.bf && sc) hipLaunchKernelGGL((k_bw_intra<true, true>), grid, blk, 0, st, p);
+    else if (p.bf) hipLaunchKernelGGL((k_bw_intra<true, false>), grid, blk, 0, st, p);
+    else if (sc) hipLaunchKernelGGL((k_bw_intra<false, true>), grid, blk, 0, st, p);
+    else hipLaunchKernelGGL((k_bw_intra<false, false>), grid, blk, 0, st, p);
+  };
   const int chains = a->B * a->H * chains_per_head(p.bf);
   auto chain_grid = [](int nb) { return dim3((unsigned)(8 * ((nb + 7) / 8))); };
   auto block = [&](int j) {
@@ -2214,8 +2231,7 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
     p.init = j == 0 ? (const float*)a->init_state : boundary(j);
     p.sfin = boundary(j + 1);
     p.dfin = nullptr; p.dinit = nullptr;
-    if (p.bf) hipLaunchKernelGGL(k_bw_intra<true>, intra_grid(n), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(k_bw_intra<false>, intra_grid(n), dim3(NT), 0, st, p);
+    launch_intra(n);
     if (p.bf) hipLaunchKernelGGL(k_bw_chains<true>, chain_grid(chains), dim3(256), 0, st, p, chains, chains);
     else hipLaunchKernelGGL(k_bw_chains<false>, chain_grid(chains), dim3(256), 0, st, p, chains, chains);
   }
@@ -2229,13 +2245,13 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
     p.sfin = nullptr;
     p.dfin = j == nblk - 1 ? (const float*)a->d_final : dcarry;
     p.dinit = j == 0 ? (float*)a->d_init : dcarry;
-    if (p.bf) hipLaunchKernelGGL(k_bw_intra<true>, intra_grid(n), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(k_bw_intra<false>, intra_grid(n), dim3(NT), 0, st, p);
+    launch_intra(n);
     if (p.bf) hipLaunchKernelGGL(k_bw_chains<true>, chain_grid(2 * chains), dim3(256), 0, st, p, chains, 2 * chains);
     else hipLaunchKernelGGL(k_bw_chains<false>, chain_grid(2 * chains), dim3(256), 0, st, p, chains, 2 * chains);
     if (p.bf) hipLaunchKernelGGL(k_bw_grads<true>, dim3(n), dim3(NT), 0, st, p);
     else hipLaunchKernelGGL(k_bw_grads<false>, dim3(n), dim3(NT), 0, st, p);
-    hipLaunchKernelGGL(k_bw_dqk, dim3((unsigned)(NQ * n)), dim3(NT), 0, st, p);
+    if (sc) hipLaunchKernelGGL(k_bw_dqk<true>, dim3((unsigned)(NQ * n)), dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL(k_bw_dqk<false>, dim3((unsigned)(NQ * n)), dim3(NT), 0, st, p);
   }
   prof_mark(4, st, true);
   const hipError_t e = hipGetLastError();
