@@ -455,7 +455,7 @@ def rocprof_summary(kt_dir, f_dir, w_dir):
 
 CFG_CMD = ("cd /tmp && export TMPDIR=/tmp && cd $GRAFT_REPO_ROOT && rocprofv3 --kernel-trace --output-format csv "
            "-d gpurun_out/ktc -o run -- python3 bench.py --no-cpu-baseline --steps 2 --warmup 1 --decode-steps 0 "
-           "--train-steps 0 --config-steps 4 --no-kernel-trace")
+           "--train-steps 0 --config-steps 12 --no-kernel-trace")
 CFG_PMC_CMD = ("cd /tmp && export TMPDIR=/tmp && cd $GRAFT_REPO_ROOT && rocprofv3 --pmc {ctr} --output-format csv "
                "-d gpurun_out/{d} -o run -- python3 bench.py --no-cpu-baseline --steps 1 --warmup 1 --decode-steps 0 "
                "--train-steps 0 --config-steps 2 --no-kernel-trace --copy-calibration")
@@ -520,12 +520,12 @@ def rocprof_configs_summary(kt_dir, f_dir=None, w_dir=None):
               "the config-2 calls of the same run are the 12-head grids.  Algorithmic bytes: inputs read once and "
               "outputs written once (config 5: per 8192-token block).", ""]
     if ctr:
-        lines += ["| kernel | grid (workgroups) | dispatches | avg us | total us | fetch MB | write MB | "
-                  "algorithmic MB | traffic / algorithmic |", "|---|---|---|---|---|---|---|---|---|"]
+        lines += ["| kernel | grid (workgroups) | dispatches | avg us | min us | total us | fetch MB | write MB | "
+                  "algorithmic MB | traffic / algorithmic |", "|---|---|---|---|---|---|---|---|---|---|"]
     else:
-        lines += ["| kernel | grid (workgroups) | dispatches | avg us | total us |", "|---|---|---|---|---|"]
+        lines += ["| kernel | grid (workgroups) | dispatches | avg us | min us | total us |", "|---|---|---|---|---|---|"]
     for (k, grid), v in sorted(rows.items(), key=lambda kv: -sum(kv[1])):
-        line = f"| {k} | {grid[0]} x {grid[1]} x {grid[2]} | {len(v)} | {sum(v) / len(v):.1f} | {sum(v):.0f} |"
+        line = f"| {k} | {grid[0]} x {grid[1]} x {grid[2]} | {len(v)} | {sum(v) / len(v):.1f} | {min(v):.1f} | {sum(v):.0f} |"
         if ctr:
             nwg = grid[0] * grid[1] * grid[2]
             fb = ctr["FETCH_SIZE"][0].get((k, nwg), float("nan"))

@@ -681,8 +681,9 @@ __global__ __launch_bounds__(256, 2) void k_prepass(const PF p) {
 //   * be, qe and ke are row scalars times k, q and k: the scan takes the
 //     normalised rows once per key head (k, q and k^T fragments, single bf16
 //     words, exact) and the row scalars per execution head.
-// Bound by memory: 4 x 8192 tokens, 32 heads 326 us for 1.67 GB (5.1 TB/s), against
-// 1510 us for the 128-token form's phases, which write operands per head.
+// Bound by memory: 4 x 8192 tokens, 32 heads 382 us for 1.67 GB (4.4 TB/s; 338 to
+// 416 us within a dozen calls in a row), against 1510 us for the 128-token
+// form's phases, which write operands per head.
 // ===========================================================================
 template <class TIn>
 __global__ __launch_bounds__(256, 3) void k_prepass_sc(const PF p) {
@@ -886,8 +887,8 @@ template <class TV> struct OutRows {
 // LDS fragments are read in bursts ahead of the products that use them.
 // The role is a scalar (wave-uniform) branch.
 // Bound by the step's six dependent products beside 110 KB of loads per CU (64
-// bytes a clock): 1.65 us a chunk with 192 workgroups, 1.0 with every load taken
-// out.  2048 tokens, 24 value heads 53 us, against 26 for the 128-token form's
+// bytes a clock): 1.5 us a chunk with 192 workgroups, 1.0 with every load taken
+// out.  2048 tokens, 24 value heads 48 us, against 26 for the 128-token form's
 // scan, whose prepass costs 32 more.
 // ===========================================================================
 
@@ -1271,9 +1272,10 @@ __global__ __launch_bounds__(512) void k_chain(const PF p) {
 // chunk, fragment-native, 1 KB per instruction and no registers) from the
 // workspace into the other half of a double buffer, one chunk ahead.
 // Bound by the LDS reads of those operands (84 KB per wave and chunk) beside
-// 132 MFMAs per wave.  chunk_gdn, 4 x 8192 tokens, 32 value heads, bf16: 434 us
-// with the rows split, 400 us here (3.1 us a chunk against 1 us of MFMA issue);
-// with every read waited for in turn, the compiler's order, 435 us.
+// 132 MFMAs per wave.  chunk_gdn, 4 x 8192 tokens, 32 value heads, bf16, timed in
+// turn: 434 us with the rows split, 400 us here (3.1 us a chunk against 1 us of
+// MFMA issue); with every read waited for in turn, the compiler's order, 435 us.
+// (Under the profiler, a dozen calls in a row: 419 to 534 us.)
 // ===========================================================================
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // 64 lanes x 16 bytes from src (each lane's own address) to 1 KB of LDS at dst

@@ -1311,7 +1311,7 @@ __device__ __forceinline__ void value_cols(const PF& p, const PL& px, int b, int
 //     chunk as O^T = S^T X^T + (M U)^T from the same fragments, beside the
 //     recurrence on the other wave slot of each SIMD.
 // A chunk step is short next to the latency of its operand loads, so each
-// role keeps several chunks of operands in flight in VGPRs (ChainSets: the
+// role keeps several chunks of operands in flight in VGPRs (RS and OS: the
 // number of operand sets; a chunk's loads are issued that many steps minus
 // one ahead).  Two waves per SIMD leave each wave 256 VGPRs for them.
 // The role is a scalar (wave-uniform) branch, and both roles execute exactly
