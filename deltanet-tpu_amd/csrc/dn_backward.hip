@@ -151,8 +151,8 @@ __device__ __forceinline__ float4 cvt4(const u32x4& x, int dt) {
 // Held at 128 channels, the copies of chunk_gdn's three gates and of their
 // gradients were 14 passes over a (token, head, 128) fp32 array.  4096 tokens,
 // 32 heads: preparation 93 to 39 us, the gates' last step 55 to 13; with the
-// decay factors formed once per pair (k_bw_intra, k_bw_dqk), k_bw_intra 366 to
-// 262 and k_bw_dqk 262 to 214.
+// decay factors formed once per pair (k_bw_intra, k_bw_dqk), k_bw_intra 365 to
+// 236 and k_bw_dqk 261 to 203.
 constexpr int kGateParts[3] = {4, 8, 1};
 __device__ __forceinline__ u32x4 ld_gate4(const float* g, int64_t row, int chans, int c) {
   if (chans == 1) return u32x4{__builtin_bit_cast(uint32_t, g[row]), 0u, 0u, 0u};
@@ -262,15 +262,19 @@ template <> struct Op<true> {
 // ---------------------------------------------------------------------------
 // k_bw_intra
 // ---------------------------------------------------------------------------
-// SC: one decay per (token, head).  A template argument, since the kernel is at
-// its 256 VGPRs: with both forms behind a branch it spilled 19 of them (float32
-// 5), one decay per channel alone spills 11 (1), one per token none.  4096
-// tokens, 32 heads, one per token 297 us behind the branch, 262 apart; 2 x 2048
-// tokens, 16 heads, one per channel 161 and 156, float32 2048 x 24 122 and 117.
-template <bool BF, bool SC>
+// SC: one decay per (token, head).  BWC: the channels of b and w where both hold
+// as many, else 0.  Template arguments, since the kernel is at its 256 VGPRs:
+// with every form behind branches it spilled 19 of them (float32 5), apart it
+// spills 9-11 (1), with one decay per token none.  Behind branches / SC alone
+// apart / both: 4096 tokens, 32 heads, one value per gate 297 / 257 / 236 us;
+// KDA 2 x 2048 tokens, 16 heads 161 / 152 / 143; a value per channel 2048 x 24
+// heads 130 / 128 / 127, float32 122 / 114 / 109 (109 before gates of one value
+// had a form of their own).
+template <bool BF, bool SC, int BWC>
 __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
   using O = Op<BF>;
-  constexpr int GC = SC ? 1 : KD;   // channels of the decay
+  constexpr int GC = SC ? 1 : KD;   // channels of the decay, of b and of w
+  const int b_c = BWC ? BWC : p.b_c, w_c = BWC ? BWC : p.w_c;
   __shared__ float sG[BC][KP];
   __shared__ float sA[BC][CP];   // A, then T
   __shared__ float sM[BC][CP];
@@ -335,7 +339,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
     bst[it] = u32x4{0u, 0u, 0u, 0u};
     if (t0 + i < p.L) {
       qst[it] = ld4g(p.q + row_in(p, bb, t0 + i, h, p.qk_hd) + 4 * c4);
-      bst[it] = ld_gate4(p.b, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, p.b_c, 4 * c4);
+      bst[it] = ld_gate4(p.b, row_in(p, bb, t0 + i, h, p.gb_hd) / KD, b_c, 4 * c4);
     }
   }
   lds_barrier();
@@ -403,7 +407,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
 #pragma unroll
   for (int it = 0; it < SIT; ++it) {
     const int c4 = tid % (KD / 4), i = 4 * (tid / (KD / 4)) + it;
-    const float4 k4 = kst[it], b4 = gate4_of(bst[it], p.b_c);
+    const float4 k4 = kst[it], b4 = gate4_of(bst[it], b_c);
     *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = qst[it];
     *reinterpret_cast<float4*>(&sW[i][4 * c4]) = make_float4(b4.x * k4.x, b4.y * k4.y, b4.z * k4.z, b4.w * k4.w);
   }
@@ -559,7 +563,7 @@ __global__ __launch_bounds__(NT) void k_bw_intra(BW p) {
       const int j = 32 * s + pi_k(q, e), r = 16 * wv + l16;
       const bool vj = t0 + j < p.L;
       const int64_t ro = row_of(p, bb, vj ? t0 + j : 0, h) + r;
-      wvw[s][e] = vj ? p.w[p.w_c == 1 ? ro / KD : ro] : 0.f;
+      wvw[s][e] = vj ? p.w[w_c == 1 ? ro / KD : ro] : 0.f;
       wvv[s][e] = 0;
       if (vj) wvv[s][e] = v16 ? (uint32_t)((const uint16_t*)p.v)[ro] : ((const uint32_t*)p.v)[ro];
     }
@@ -1415,9 +1419,9 @@ __global__ __launch_bounds__(NT) void k_bw_grads(BW p) {
 // span allows, else use e^{G_i-G_j} per element.
 // Wave w owns the 16 channels 16 (w % 2) .. and the 16-row block w / 2;
 // lanes hold rows 4q..4q+3 of it.  About 73 KB of LDS: two workgroups per CU.
-// SC: one decay per (token, head), whose products need no factors (99 VGPRs,
-// 109 with one per channel; 4096 tokens, 32 heads 224 us behind a branch, 213
-// apart).
+// SC: one decay per (token, head), whose products need no factors; B1: one b.
+// Template arguments: behind branches on both 4096 tokens, 32 heads took 224 us,
+// apart 203; KDA 2 x 2048 tokens, 16 heads 126 and 116.
 // ---------------------------------------------------------------------------
 constexpr int HC = KD / 4;      // channels per k_bw_dqk workgroup
 constexpr int NQ = KD / HC;     // k_bw_dqk workgroups per unit
@@ -1435,7 +1439,7 @@ __device__ __forceinline__ void mma_half(f32x4& acc, const float* a, const float
   }
 }
 
-template <bool SC>
+template <bool SC, bool B1>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_bw_dqk(BW p) {
   __shared__ float sQ[BC][HP], sK[BC][HP], sB[BC][HP], sG[BC][HP];
   __shared__ float sdM[BC][CP], sdA[BC][CP];
@@ -1480,11 +1484,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     const int t = min(t0 + i, p.L - 1);
     const int64_t rq = row_in(p, bb, t, h, p.qk_hd) + ch0 + 4 * c4;
     const float4 q4 = ld4g(p.q + rq), k4 = ld4g(p.k + rq), g4 = ld4g(G + i * KD + ch0 + 4 * c4);
-    const u32x4 b4 = ld_gate4(p.b, row_in(p, bb, t, h, p.gb_hd) / KD, p.b_c, ch0 + 4 * c4);
+    const u32x4 b4 = ld_gate4(p.b, row_in(p, bb, t, h, p.gb_hd) / KD, B1 ? 1 : KD, ch0 + 4 * c4);
     const bool in = t0 + i < p.L;
     *reinterpret_cast<float4*>(&sQ[i][4 * c4]) = in ? q4 : zero_f4();
     *reinterpret_cast<float4*>(&sK[i][4 * c4]) = in ? k4 : zero_f4();
-    *reinterpret_cast<float4*>(&sB[i][4 * c4]) = in ? gate4_of(b4, p.b_c) : zero_f4();
+    *reinterpret_cast<float4*>(&sB[i][4 * c4]) = in ? gate4_of(b4, B1 ? 1 : KD) : zero_f4();
     *reinterpret_cast<float4*>(&sG[i][4 * c4]) = g4;
   }
 #pragma unroll
@@ -1679,9 +1683,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
         const int64_t ro = row_of(p, bb, t0 + i, h) + r;
         p.dq[ro] = dq + dmii * kv;
         p.dk[ro] = dk + dmii * qv + dkc + bv * dbeta;
-        if (p.b_c != 1) p.db[ro] = kv * dbeta;
+        if constexpr (!B1) p.db[ro] = kv * dbeta;
       }
-      if (p.b_c == 1) {   // 16 channels of a row: one 16-lane row
+      if constexpr (B1) {   // 16 channels of a row: one 16-lane row
         const float sum = lane_sum<16>(kv * dbeta);
         if (l16 == 0 && t0 + i < p.L) p.db[row_of(p, bb, t0 + i, h) / KD * kGateParts[1] + (r >> 4)] = sum;
       }
@@ -2212,10 +2216,17 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
   const bool sc = p.g_c == 1;
   auto launch_intra = [&](unsigned n) {
     const dim3 grid(std::min(n, (unsigned)ncu)), blk(NT);
-    if (p.bf && sc) hipLaunchKernelGGL((k_bw_intra<true, true>), grid, blk, 0, st, p);
-    else if (p.bf) hipLaunchKernelGGL((k_bw_intra<true, false>), grid, blk, 0, st, p);
-    else if (sc) hipLaunchKernelGGL((k_bw_intra<false, true>), grid, blk, 0, st, p);
-    else hipLaunchKernelGGL((k_bw_intra<false, false>), grid, blk, 0, st, p);
+    const int bwc = p.b_c == p.w_c ? p.b_c : 0;
+    auto go = [&](auto bf) {
+      constexpr bool BF = decltype(bf)::value;
+      if (sc && bwc == 1) hipLaunchKernelGGL((k_bw_intra<BF, true, 1>), grid, blk, 0, st, p);
+      else if (sc) hipLaunchKernelGGL((k_bw_intra<BF, true, 0>), grid, blk, 0, st, p);
+      else if (bwc == KD) hipLaunchKernelGGL((k_bw_intra<BF, false, KD>), grid, blk, 0, st, p);
+      else if (bwc == 1) hipLaunchKernelGGL((k_bw_intra<BF, false, 1>), grid, blk, 0, st, p);
+      else hipLaunchKernelGGL((k_bw_intra<BF, false, 0>), grid, blk, 0, st, p);
+    };
+    if (p.bf) go(std::true_type{});
+    else go(std::false_type{});
   };
   const int chains = a->B * a->H * chains_per_head(p.bf);
   auto chain_grid = [](int nb) { return dim3((unsigned)(8 * ((nb + 7) / 8))); };
@@ -2250,8 +2261,12 @@ static int bwd_core(const dn_backward_args* a, int dout_dt, int dv_dt, int v_dt,
     else hipLaunchKernelGGL(k_bw_chains<false>, chain_grid(2 * chains), dim3(256), 0, st, p, chains, 2 * chains);
     if (p.bf) hipLaunchKernelGGL(k_bw_grads<true>, dim3(n), dim3(NT), 0, st, p);
     else hipLaunchKernelGGL(k_bw_grads<false>, dim3(n), dim3(NT), 0, st, p);
-    if (sc) hipLaunchKernelGGL(k_bw_dqk<true>, dim3((unsigned)(NQ * n)), dim3(NT), 0, st, p);
-    else hipLaunchKernelGGL(k_bw_dqk<false>, dim3((unsigned)(NQ * n)), dim3(NT), 0, st, p);
+    const dim3 dqk_grid((unsigned)(NQ * n));
+    const bool b1 = p.b_c == 1;
+    if (sc && b1) hipLaunchKernelGGL((k_bw_dqk<true, true>), dqk_grid, dim3(NT), 0, st, p);
+    else if (sc) hipLaunchKernelGGL((k_bw_dqk<true, false>), dqk_grid, dim3(NT), 0, st, p);
+    else if (b1) hipLaunchKernelGGL((k_bw_dqk<false, true>), dqk_grid, dim3(NT), 0, st, p);
+    else hipLaunchKernelGGL((k_bw_dqk<false, false>), dqk_grid, dim3(NT), 0, st, p);
   }
   prof_mark(4, st, true);
   const hipError_t e = hipGetLastError();
