@@ -65,3 +65,10 @@ def test_scalar_gates(L, decay, precision, v_dt):
                                                   ((2, 4, 2), False, True)])
 def test_mixed_gates(chans, heads, fuse, recompute):
     compare(130, 2, 4, heads, chans, precision="fp32", v_dt=torch.float32, decay=0.3, docs=2, fuse=fuse, recompute=recompute)
+
+
+# the kernels of each mix with split-bf16 products (one decay or one per channel;
+# b and w of one channel, of 128, or mixed)
+@pytest.mark.parametrize("chans", [c for c in itertools.product((1, 128), repeat=3) if c != (128, 128, 128)])
+def test_mixed_gates_bf16(chans):
+    compare(130, 2, 4, (2, 2, 4), chans, precision="bf16", v_dt=torch.bfloat16, decay=0.3, docs=2)
